@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/native_hip.h"
+#include "early_gemm.h"
 #include "kernels.h"
 
 static_assert(LNH_NOALLOC_WORKSPACE_BYTES == nh::STATIC_SCRATCH_BYTES, "header and device array disagree");
@@ -68,6 +69,8 @@ struct lnh_exec {
     void *d_ws = nullptr;                     // kernel workspace (multi-token products), grow-only
     std::vector<void *> ws_retired;           // earlier, smaller workspaces: captured graphs may still point at them
     size_t ws_cap = 0;
+    std::unique_ptr<nh::HostPool> pool;       // large host copies and comparisons, made by the first of them
+    size_t begun = 0;                         // floats of the result nh::gemm_end will fetch
     std::string err;
 };
 
@@ -138,11 +141,11 @@ int ensure_scratch(lnh_exec *e, size_t in_floats, size_t out_floats) {
     return LNH_ERR_OOM;
 }
 
-// Pinned host staging for calls whose activations are small (a decode step's vectors, a few tokens).
-// A copy from or to pageable memory makes the runtime stage and synchronise on its own, tens of
-// microseconds per call; from pinned memory a small kernel moves the data at PCIe latency.  False = no
-// pinned memory to be had: the caller takes the plain copies.
-constexpr size_t PINNED_MAX_FLOATS = (size_t)1 << 20;  // 4 MB each way
+// Pinned host staging.  A copy from or to pageable memory makes the runtime stage and synchronise on its own, tens of
+// microseconds per call and 10 GB/s; from pinned memory a small kernel moves the data at PCIe latency, and for large
+// results the worker threads take the staging copy (one thread alone: 96 tokens x 14336 rows spent 1 ms in it).
+// False = no pinned memory to be had: the caller takes the plain copies.
+constexpr size_t PINNED_MAX_FLOATS = (size_t)1 << 24;  // 64 MB each way
 bool ensure_pinned(lnh_exec *e, size_t in_floats, size_t out_floats) {
     auto grow = [&](float *&buf, size_t &cap, size_t want) {
         if (want <= cap) return true;
@@ -343,18 +346,52 @@ int check_gemm(lnh_exec *e, const lnh_matrix *m, size_t tokens, bool have_lens, 
     return LNH_OK;
 }
 
-// H2D x, kernel(s), blocking D2H y (native-cuda/src/gpu.rs:301-303, 332-334).
+// Whether a kernel of this device can read or write the caller's buffer in place: pinned memory, whole aligned 16-byte
+// vectors.  Asked for buffers where a staging copy costs more than the question.
+constexpr size_t IN_PLACE_MIN_FLOATS = 16384;
+float *in_place(const float *p, size_t floats) {
+    if (floats < IN_PLACE_MIN_FLOATS || floats % 4 != 0 || misaligned(p)) return nullptr;
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();  // an ordinary pointer
+        return nullptr;
+    }
+    return at.type == hipMemoryTypeHost && !misaligned(at.devicePointer) ? static_cast<float *>(at.devicePointer) : nullptr;
+}
+
+void copy_floats(lnh_exec *e, float *dst, const float *src, size_t n) {
+    if (n < 131072) {
+        std::memcpy(dst, src, n * sizeof(float));
+        return;
+    }
+    nh::host_pool(e).run_ranges(n, 32768, [&](size_t begin, size_t end) { std::memcpy(dst + begin, src + begin, (end - begin) * sizeof(float)); });
+}
+
+// A product of host buffers between the enqueueing of its work and the arrival of its result.
+struct HostCall {
+    bool staged = false;  // y comes through the executor's pinned staging
+    size_t y_total = 0;
+};
+
+// H2D x, kernel(s), D2H y enqueued on the executor's stream (native-cuda/src/gpu.rs:301-303, 332-334).
 // shared_x: every group reads the same x (tokens[0] rows of it), copied to the device once.
-int run_host(lnh_exec *e, size_t n_groups, const lnh_matrix *const *mats, const size_t *tokens, const float *x,
-             size_t x_total, float *y, size_t y_total, bool shared_x = false) {
+// y: where a result too large for the staging buffers is copied directly; null if such a call is to be refused
+// (LNH_ERR_UNSUPPORTED, nothing enqueued).
+int begin_host(lnh_exec *e, size_t n_groups, const lnh_matrix *const *mats, const size_t *tokens, const float *x,
+               size_t x_total, float *y, size_t y_total, bool shared_x, HostCall *call) {
     hipError_t h = hipSetDevice(e->ctx->device);
     if (h != hipSuccess) return hip_fail(e, h, "hipSetDevice");
     int rc = ensure_scratch(e, x_total, y_total);
     if (rc != LNH_OK) return rc;
-    const bool pinned = x_total <= PINNED_MAX_FLOATS && y_total <= PINNED_MAX_FLOATS && ensure_pinned(e, x_total, y_total);
+    float *const x_there = in_place(x, x_total), *const y_there = y ? in_place(y, y_total) : nullptr;
+    const bool pinned = x_total <= PINNED_MAX_FLOATS && y_total <= PINNED_MAX_FLOATS &&
+                        ensure_pinned(e, x_there ? 0 : x_total, y_there ? 0 : y_total);
+    if (!pinned && !y) return LNH_ERR_UNSUPPORTED;
+    call->staged = pinned && !y_there;
+    call->y_total = y_total;
     if (pinned) {
-        std::memcpy(e->h_in, x, x_total * sizeof(float));
-        h = nh::launch_copy_small(e->stream, e->d_in, e->h_in, ((x_total + 3) & ~(size_t)3) * sizeof(float));
+        if (!x_there) copy_floats(e, e->h_in, x, x_total);
+        h = nh::launch_copy_small(e->stream, e->d_in, x_there ? x_there : e->h_in, ((x_total + 3) & ~(size_t)3) * sizeof(float));
     } else {
         h = hipMemcpyAsync(e->d_in, x, x_total * sizeof(float), hipMemcpyHostToDevice, e->stream);
     }
@@ -369,19 +406,30 @@ int run_host(lnh_exec *e, size_t n_groups, const lnh_matrix *const *mats, const 
         yo += tokens[g] * mats[g]->view.rows;
     }
     rc = launch_products(e, e->stream, n_groups, mats, tokens, xs.data(), ys.data());
-    if (rc != LNH_OK) {
-        (void)hipStreamSynchronize(e->stream);
-        return rc;
+    if (rc == LNH_OK) {
+        if (pinned)
+            h = nh::launch_copy_small(e->stream, y_there ? y_there : e->h_out, e->d_out, ((y_total + 3) & ~(size_t)3) * sizeof(float));
+        else
+            h = hipMemcpyAsync(y, e->d_out, y_total * sizeof(float), hipMemcpyDeviceToHost, e->stream);
+        if (h != hipSuccess) rc = hip_fail(e, h, "HIP output copy");
     }
-    if (pinned)
-        h = nh::launch_copy_small(e->stream, e->h_out, e->d_out, ((y_total + 3) & ~(size_t)3) * sizeof(float));
-    else
-        h = hipMemcpyAsync(y, e->d_out, y_total * sizeof(float), hipMemcpyDeviceToHost, e->stream);
-    hipError_t hs = hipStreamSynchronize(e->stream);
-    if (h == hipSuccess) h = hs;
+    if (rc != LNH_OK) (void)hipStreamSynchronize(e->stream);
+    return rc;
+}
+
+// Waits for the work of `call`; a staged y is written only after everything succeeded.  y null: the result is dropped.
+int end_host(lnh_exec *e, const HostCall &call, float *y) {
+    const hipError_t h = hipStreamSynchronize(e->stream);
     if (h != hipSuccess) return hip_fail(e, h, "HIP output copy");
-    if (pinned) std::memcpy(y, e->h_out, y_total * sizeof(float));  // y is written only after everything succeeded
+    if (call.staged && y) copy_floats(e, y, e->h_out, call.y_total);
     return LNH_OK;
+}
+
+int run_host(lnh_exec *e, size_t n_groups, const lnh_matrix *const *mats, const size_t *tokens, const float *x,
+             size_t x_total, float *y, size_t y_total, bool shared_x = false) {
+    HostCall call;
+    const int rc = begin_host(e, n_groups, mats, tokens, x, x_total, y, y_total, shared_x, &call);
+    return rc == LNH_OK ? end_host(e, call, y) : rc;
 }
 
 }  // namespace
@@ -547,6 +595,40 @@ int lnh_gemm(lnh_exec *e, const lnh_matrix *m, size_t tokens, const float *x, si
     if (!x || !y) return fail(e, LNH_ERR_INVALID, "buffer pointer is null");
     return run_host(e, 1, &m, &tokens, x, inputs, y, outputs);
 }
+
+}  // extern "C"
+
+namespace nh {
+
+HostPool &host_pool(lnh_exec *e) {
+    if (!e->pool) e->pool = std::make_unique<HostPool>();
+    return *e->pool;
+}
+
+bool gemm_begin(lnh_exec *e, const lnh_matrix *m, size_t tokens, const float *x, size_t x_len, size_t y_len) {
+    size_t inputs, outputs;
+    if (check_gemm(e, m, tokens, true, x_len, y_len, &inputs, &outputs) != LNH_OK || !x) return false;
+    if (nh::product_reads_tiled(m->view.type, (uint32_t)tokens)) {
+        std::lock_guard<std::mutex> lock(m->lazy);
+        if (!m->tiled.p0) return false;
+    }
+    HostCall call;
+    if (begin_host(e, 1, &m, &tokens, x, inputs, nullptr, outputs, false, &call) != LNH_OK) return false;
+    e->begun = call.y_total;
+    return true;
+}
+
+int gemm_end(lnh_exec *e, float *y) {
+    HostCall call;
+    call.staged = true;
+    call.y_total = e->begun;
+    e->begun = 0;
+    return end_host(e, call, y);
+}
+
+}  // namespace nh
+
+extern "C" {
 
 int lnh_gemv_once(lnh_exec *e, const float *weights, size_t weights_len, const float *x, size_t x_len, float *y,
                   size_t y_len) {
