@@ -15,9 +15,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
-#include <condition_variable>
-#include <functional>
-#include <mutex>
+#include <new>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -34,6 +32,7 @@
 #include "../../include/native_hip.h"
 #include "../../include/native_hip_llama.h"
 #include "gguf.h"
+#include "host_pool.h"
 
 namespace {
 
@@ -258,70 +257,122 @@ void router_weights(const float *probs, const uint32_t *order, size_t k, bool no
     for (size_t j = 0; j < k; j++) w[j] /= wsum;
 }
 
-// ------------------------------------------------------------------ worker threads for the attention heads
+// ------------------------------------------------------------------ attention of one query head on the host
 
-// The reference attends head after head on one thread.  Heads are independent, so they are
-// spread over a few threads here; the arithmetic of each head is untouched.
-class HeadPool {
+typedef float v4f __attribute__((ext_vector_type(4)));
+inline v4f load4(const float *p) {
+    v4f v;
+    std::memcpy(&v, p, sizeof v);
+    return v;
+}
+
+// (cos, sin) of every rotated pair at `pos`: rope()'s own values, formed once for all heads of a token.
+void rope_factors(size_t len, size_t pos, size_t n_rot, float base, std::vector<float> *cs) {
+    const size_t n = n_rot < len ? n_rot : len;
+    cs->clear();
+    if (n < 2) return;
+    const float n_rot_f = n_rot <= 65535 ? (float)n_rot : 2.f;
+    float theta = pos <= 65535 ? (float)pos : 65535.f;
+    const float theta_scale = std::pow(base, -2.0f / n_rot_f);
+    for (size_t i = 0; i + 1 < n; i += 2) {
+        cs->push_back(std::cos(theta));
+        cs->push_back(std::sin(theta));
+        theta *= theta_scale;
+    }
+}
+void rope_apply(float *v, const std::vector<float> &cs) {
+    for (size_t i = 0; i < cs.size(); i += 2) {
+        const float x = v[i], y = v[i + 1];
+        v[i] = x * cs[i] - y * cs[i + 1];
+        v[i + 1] = x * cs[i + 1] + y * cs[i];
+    }
+}
+
+// dot[j] = q . rows[j] for N rows, each summed over the dimensions in order from zero as attend_query does it
+// (langtax/src/decode.rs:11126-11197).  One such sum is a chain of additions, four processor cycles each; N of them
+// side by side, four to a vector (4 x 4 blocks of the rows turned by shuffles), keep the adders busy instead.
+template <int N> inline void dot_rows(const float *q, const float *const *rows, size_t hd, float *dot) {
+    static_assert(N % 4 == 0, "whole vectors of rows");
+    v4f sum[N / 4];
+    for (int g = 0; g < N / 4; g++) sum[g] = v4f{0.f, 0.f, 0.f, 0.f};
+    size_t i = 0;
+    for (; i + 4 <= hd; i += 4) {
+        const v4f qv = load4(q + i);
+#pragma unroll
+        for (int g = 0; g < N / 4; g++) {
+            const v4f a = load4(rows[4 * g] + i), b = load4(rows[4 * g + 1] + i), c = load4(rows[4 * g + 2] + i), d = load4(rows[4 * g + 3] + i);
+            const v4f ab_lo = __builtin_shufflevector(a, b, 0, 4, 1, 5), ab_hi = __builtin_shufflevector(a, b, 2, 6, 3, 7);
+            const v4f cd_lo = __builtin_shufflevector(c, d, 0, 4, 1, 5), cd_hi = __builtin_shufflevector(c, d, 2, 6, 3, 7);
+            const v4f k0 = __builtin_shufflevector(ab_lo, cd_lo, 0, 1, 4, 5), k1 = __builtin_shufflevector(ab_lo, cd_lo, 2, 3, 6, 7);
+            const v4f k2 = __builtin_shufflevector(ab_hi, cd_hi, 0, 1, 4, 5), k3 = __builtin_shufflevector(ab_hi, cd_hi, 2, 3, 6, 7);
+            sum[g] += qv.xxxx * k0;
+            sum[g] += qv.yyyy * k1;
+            sum[g] += qv.zzzz * k2;
+            sum[g] += qv.wwww * k3;
+        }
+    }
+    for (; i < hd; i++)
+        for (int g = 0; g < N / 4; g++) sum[g] += v4f{q[i], q[i], q[i], q[i]} * v4f{rows[4 * g][i], rows[4 * g + 1][i], rows[4 * g + 2][i], rows[4 * g + 3][i]};
+    for (int g = 0; g < N / 4; g++) std::memcpy(dot + 4 * g, &sum[g], sizeof sum[g]);
+}
+
+// dst[i] = sum over u of score[u] * rows[u][i], added in the order of u; a strip of 32 dimensions stays in registers.
+void weighted_rows(const float *score, const float *const *rows, size_t n, size_t hd, float *dst) {
+    size_t i = 0;
+    for (; i + 32 <= hd; i += 32) {
+        v4f acc[8];
+        for (int k = 0; k < 8; k++) acc[k] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (size_t u = 0; u < n; u++) {
+            const v4f w = {score[u], score[u], score[u], score[u]};
+            const float *v = rows[u] + i;
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc[k] += w * load4(v + 4 * k);
+        }
+        std::memcpy(dst + i, acc, sizeof acc);
+    }
+    for (; i < hd; i++) {
+        float o = 0.f;
+        for (size_t u = 0; u < n; u++) o += score[u] * rows[u][i];
+        dst[i] = o;
+    }
+}
+
+// A session's activation buffer: grow-only, its contents are not kept when it grows.  Pinned where products run on the
+// GPU, so that they read and write it in place instead of through a staging copy.
+class HostBuf {
   public:
-    explicit HeadPool(size_t workers) {
-        for (size_t i = 0; i < workers; i++) threads_.emplace_back([this] { loop(); });
-    }
-    ~HeadPool() {
-        {
-            std::lock_guard<std::mutex> g(mu_);
-            stop_ = true;
+    HostBuf() = default;
+    HostBuf(const HostBuf &) = delete;
+    HostBuf &operator=(const HostBuf &) = delete;
+    ~HostBuf() { drop(); }
+    float *data() { return p_; }
+    float &operator[](size_t i) { return p_[i]; }
+    void resize(size_t n, bool pinned) {
+        if (n <= cap_ && (pinned_ || !pinned)) return;
+        drop();
+        void *p = nullptr;
+        if (pinned && hipHostMalloc(&p, n * sizeof(float), hipHostMallocDefault) == hipSuccess) {
+            pinned_ = true;
+        } else {
+            if (pinned) (void)hipGetLastError();
+            p = std::malloc(n * sizeof(float));
+            if (!p) throw std::bad_alloc();
         }
-        wake_.notify_all();
-        for (auto &t : threads_) t.join();
-    }
-    // Calls fn(i) for every i < n, on the workers and on the calling thread; returns when all are done.
-    void run(size_t n, const std::function<void(size_t)> &fn) {
-        if (threads_.empty() || n < 2) {
-            for (size_t i = 0; i < n; i++) fn(i);
-            return;
-        }
-        {
-            std::lock_guard<std::mutex> g(mu_);
-            fn_ = &fn;
-            n_ = n;
-            next_.store(0);
-            busy_ = threads_.size();
-            epoch_++;
-        }
-        wake_.notify_all();
-        drain();
-        std::unique_lock<std::mutex> g(mu_);
-        done_.wait(g, [this] { return busy_ == 0; });
-        fn_ = nullptr;
+        p_ = static_cast<float *>(p);
+        cap_ = n;
     }
 
   private:
-    void drain() {
-        for (size_t i = next_.fetch_add(1); i < n_; i = next_.fetch_add(1)) (*fn_)(i);
+    void drop() {
+        if (pinned_) (void)hipHostFree(p_);
+        else std::free(p_);
+        p_ = nullptr;
+        cap_ = 0;
+        pinned_ = false;
     }
-    void loop() {
-        uint64_t seen = 0;
-        for (;;) {
-            {
-                std::unique_lock<std::mutex> g(mu_);
-                wake_.wait(g, [&] { return stop_ || epoch_ != seen; });
-                if (stop_) return;
-                seen = epoch_;
-            }
-            drain();
-            std::lock_guard<std::mutex> g(mu_);
-            if (--busy_ == 0) done_.notify_one();
-        }
-    }
-    std::vector<std::thread> threads_;
-    std::mutex mu_;
-    std::condition_variable wake_, done_;
-    const std::function<void(size_t)> *fn_ = nullptr;
-    size_t n_ = 0, busy_ = 0;
-    std::atomic<size_t> next_{0};
-    uint64_t epoch_ = 0;
-    bool stop_ = false;
+    float *p_ = nullptr;
+    size_t cap_ = 0;
+    bool pinned_ = false;
 };
 
 // ------------------------------------------------------------------ model
@@ -415,11 +466,11 @@ struct lnm_session {
     std::vector<float> cache_k, cache_v;
     // q, k, v share one buffer (matrix after matrix), and so do gate and up: products of one
     // input can then be fetched by a single call
-    std::vector<float> x, residual, qkv, attn, attn_proj, gate_up, ffn_out, xn;
+    HostBuf x, xn, qkv, attn, proj, gate_up, logits;  // x: the residual stream, xn: its norm, proj: the o or the feed-forward output
     MoeScratch moe;
     double products_s = 0.0, attention_s = 0.0;  // wall time spent in weight products / in attend + RoPE
     uint64_t n_products = 0;
-    std::unique_ptr<HeadPool> pool;
+    std::unique_ptr<nh::HostPool> pool;
 };
 
 namespace {
@@ -960,90 +1011,108 @@ int forward(lnm_session *s, const uint32_t *tokens, size_t n, float *logits) {
     const size_t d = hp.n_embd, hd = hp.head_dim, qw = (size_t)hp.n_head * hd, kvw = (size_t)hp.n_head_kv * hd;
     const size_t gqa = hp.n_head / hp.n_head_kv;
     if (ensure_blocks(s, s->past + n) != 0) return 1;
-    if (!s->pool) {
-        const unsigned hw = std::thread::hardware_concurrency();
-        const size_t threads = hw < 2 ? 1 : (hw > 16 ? 16 : hw);
-        s->pool.reset(new HeadPool(threads - 1));
-    }
-    s->x.resize(n * d);
-    const size_t emb_row = m->token_embd.nbytes / m->token_embd.n_rows;
-    for (size_t t = 0; t < n; t++) {
+    if (!s->pool) s->pool.reset(new nh::HostPool());
+    nh::HostPool &pool = *s->pool;
+    for (size_t t = 0; t < n; t++)
         if (tokens[t] >= hp.n_vocab) return fail("token id out of range");
-        if (!dequant_row(m->token_embd.type, d, m->token_embd.bytes + (size_t)tokens[t] * emb_row, &s->x[t * d]))
-            return fail("cannot dequantize token_embd.weight");
-    }
-    s->qkv.resize(n * (qw + 2 * kvw));
-    s->gate_up.resize(2 * n * hp.n_ff);
+    const bool pin = m->route == LNM_PRODUCTS_RESIDENT;
+    s->x.resize(n * d, pin);
+    s->xn.resize(n * d, pin);
+    s->qkv.resize(n * (qw + 2 * kvw), pin);
+    s->gate_up.resize(2 * n * hp.n_ff, pin);
+    s->attn.resize(n * qw, pin);
+    s->proj.resize(n * d, pin);
+    s->logits.resize(hp.n_vocab, pin);
+    const size_t emb_row = m->token_embd.nbytes / m->token_embd.n_rows;
+    std::atomic<bool> decoded{true};
+    pool.run(n, [&](size_t t) {
+        if (!dequant_row(m->token_embd.type, d, m->token_embd.bytes + (size_t)tokens[t] * emb_row, &s->x[t * d])) decoded = false;
+    });
+    if (!decoded) return fail("cannot dequantize token_embd.weight");
     float *const q = s->qkv.data(), *const k = q + n * qw, *const v = k + n * kvw;
     float *const gate = s->gate_up.data(), *const up = gate + n * hp.n_ff;
-    s->attn.resize(n * qw);
-    s->attn_proj.resize(n * d);
-    s->ffn_out.resize(n * d);
     const float hd_f = hd <= 65535 ? (float)hd : 1.f;
     const float root = std::sqrt(hd_f);
     const float score_scale = root > 0.f ? 1.f / root : 0.f;
+    std::vector<std::vector<float>> factors(n);  // RoPE of every position of the batch, for all layers and heads
+    pool.run(n, [&](size_t t) { rope_factors(hd, s->past + t, hp.n_rot, hp.rope_base, &factors[t]); });
+    // xn = rmsnorm(x) * w; with `add` first x += proj, the residual addition before it
+    auto norm_rows = [&](const float *w, bool add) {
+        pool.run(n, [&](size_t t) {
+            float *row = &s->x[t * d], *out = &s->xn[t * d];
+            const float *proj = &s->proj[t * d];
+            if (add)
+                for (size_t i = 0; i < d; i++) row[i] = proj[i] + row[i];
+            std::memcpy(out, row, d * sizeof(float));
+            rmsnorm(out, w, d, hp.rms_eps);
+        });
+    };
 
     for (size_t li = 0; li < hp.n_layer; li++) {
         Layer &l = m->layers[li];
-        s->residual = s->x;
-        for (size_t t = 0; t < n; t++) rmsnorm(&s->x[t * d], l.attn_norm.data(), d, hp.rms_eps);
-        if (products_shared(s, {&l.wq, &l.wk, &l.wv}, n, s->x.data(), q)) return 1;
+        norm_rows(l.attn_norm.data(), li > 0);
+        if (products_shared(s, {&l.wq, &l.wk, &l.wv}, n, s->xn.data(), q)) return 1;
         const auto t_att = wall_clock::now();
-        for (size_t t = 0; t < n; t++) {  // rotate and store K, store V
+        // rotate and store K, store V (every token before any attends: they attend to each other)
+        auto store = [&](size_t t) {
             const size_t p = s->past + t;
             float *kt = k + t * kvw;
             for (size_t h = 0; h < hp.n_head_kv; h++) {
-                rope(kt + h * hd, hd, p, hp.n_rot, hp.rope_base);
+                rope_apply(kt + h * hd, factors[t]);
                 std::memcpy(&s->cache_k[kv_offset(s, li, h, p)], kt + h * hd, hd * sizeof(float));
                 std::memcpy(&s->cache_v[kv_offset(s, li, h, p)], v + t * kvw + h * hd, hd * sizeof(float));
             }
+        };
+        if (n < 8) {
+            for (size_t t = 0; t < n; t++) store(t);
+        } else {
+            pool.run(n, store);
         }
         // decode.rs:11126-11197, one (token, query head) pair per work item
-        const std::function<void(size_t)> attend = [&](size_t item) {
+        pool.run(n * hp.n_head, [&](size_t item) {
             static thread_local std::vector<float> scores;
+            static thread_local std::vector<const float *> k_rows, v_rows;
             const size_t t = item / hp.n_head, hq = item % hp.n_head;
-            const size_t p = s->past + t, seq = p + 1;
-            scores.resize(seq);
+            const size_t p = s->past + t, seq = p + 1, padded = (seq + 15) & ~(size_t)15;
+            scores.resize(padded);
+            k_rows.resize(padded);
+            v_rows.resize(seq);
             float *qv = q + t * qw + hq * hd;
-            rope(qv, hd, p, hp.n_rot, hp.rope_base);
+            rope_apply(qv, factors[t]);
             const size_t hkv = hq / gqa;
             for (size_t u = 0; u < seq; u++) {
-                const float *kv = &s->cache_k[kv_offset(s, li, hkv, u)];
-                float dot = 0.f;
-                for (size_t i = 0; i < hd; i++) dot += qv[i] * kv[i];
-                scores[u] = dot * score_scale;
+                const size_t at = kv_offset(s, li, hkv, u);
+                k_rows[u] = &s->cache_k[at];
+                v_rows[u] = &s->cache_v[at];
             }
+            for (size_t u = seq; u < padded; u++) k_rows[u] = k_rows[0];  // computed and dropped
+            for (size_t u = 0; u < seq; u += 16) dot_rows<16>(qv, &k_rows[u], hd, &scores[u]);
+            for (size_t u = 0; u < seq; u++) scores[u] = scores[u] * score_scale;
             softmax(scores.data(), seq);
-            float *dst = &s->attn[t * qw + hq * hd];
-            for (size_t i = 0; i < hd; i++) dst[i] = 0.f;
-            for (size_t u = 0; u < seq; u++) {
-                const float *vv = &s->cache_v[kv_offset(s, li, hkv, u)];
-                const float st = scores[u];
-                for (size_t i = 0; i < hd; i++) dst[i] += st * vv[i];
-            }
-        };
-        s->pool->run(n * hp.n_head, attend);
+            weighted_rows(scores.data(), v_rows.data(), seq, hd, &s->attn[t * qw + hq * hd]);
+        });
         s->attention_s += since(t_att);
-        if (product(s, l.wo, n, s->attn.data(), s->attn_proj.data())) return 1;
-        for (size_t i = 0; i < n * d; i++) s->x[i] = s->attn_proj[i] + s->residual[i];
-        s->residual = s->x;
-        for (size_t t = 0; t < n; t++) rmsnorm(&s->x[t * d], l.ffn_norm.data(), d, hp.rms_eps);
+        if (product(s, l.wo, n, s->attn.data(), s->proj.data())) return 1;
+        norm_rows(l.ffn_norm.data(), true);
         if (l.moe) {
-            if (moe_ffn(m, l, n, s->x.data(), s->ffn_out.data(), &s->moe, s)) return 1;
+            if (moe_ffn(m, l, n, s->xn.data(), s->proj.data(), &s->moe, s)) return 1;
         } else {
-            if (products_shared(s, {&l.gate, &l.up}, n, s->x.data(), gate)) return 1;
-            for (size_t i = 0; i < n * hp.n_ff; i++) {  // SiLU(gate) * up, decode.rs:11826-11830 and 2981-2984
-                const float g = gate[i];
-                gate[i] = g / (1.f + std::exp(-g));
-                gate[i] *= up[i];
-            }
-            if (product(s, l.down, n, gate, s->ffn_out.data())) return 1;
+            if (products_shared(s, {&l.gate, &l.up}, n, s->xn.data(), gate)) return 1;
+            pool.run_ranges(n * hp.n_ff, 1024, [&](size_t begin, size_t end) {  // SiLU(gate) * up, decode.rs:11826-11830 and 2981-2984
+                for (size_t i = begin; i < end; i++) {
+                    const float g = gate[i];
+                    gate[i] = g / (1.f + std::exp(-g));
+                    gate[i] *= up[i];
+                }
+            });
+            if (product(s, l.down, n, gate, s->proj.data())) return 1;
         }
-        for (size_t i = 0; i < n * d; i++) s->x[i] = s->ffn_out[i] + s->residual[i];
     }
-    s->xn.assign(s->x.begin() + (n - 1) * d, s->x.begin() + n * d);
-    rmsnorm(s->xn.data(), m->output_norm.data(), d, hp.rms_eps);
-    if (product(s, m->output, 1, s->xn.data(), logits)) return 1;
+    float *const last = &s->x[(n - 1) * d], *const last_n = &s->xn[(n - 1) * d];
+    for (size_t i = 0; i < d; i++) last_n[i] = last[i] = s->proj[(n - 1) * d + i] + last[i];
+    rmsnorm(last_n, m->output_norm.data(), d, hp.rms_eps);
+    if (product(s, m->output, 1, last_n, s->logits.data())) return 1;
+    std::memcpy(logits, s->logits.data(), hp.n_vocab * sizeof(float));
     s->past += n;
     return 0;
 }
