@@ -24,6 +24,7 @@ namespace nh {
 #include "repack.inc"
 #include "gemv_kernels.inc"
 #include "gemm_kernels.inc"
+#include "plain_gemm.inc"
 
 // ------------------------------------------------------------------ launchers
 
@@ -662,7 +663,7 @@ static hipError_t launch_mm(hipStream_t stream, MmPlan &p, void *ws, size_t ws_b
     }
 }
 
-// F32 / F16 weights, two or more tokens: gemm_fmfma_kernel (+ fg_reduce_kernel when columns are shared).
+// F32 / F16 weights, up to 32 tokens: gemm_fmfma_kernel (+ fg_reduce_kernel when columns are shared).
 struct FgPlan {
     FgJob job;
     int tt;
@@ -670,8 +671,8 @@ struct FgPlan {
     size_t part_bytes;
 };
 static void fg_plan(const MatView &m, uint32_t tokens, FgPlan &p) {
-    p.tt = tokens > 32 ? 2 : tokens > 16 ? 1 : 0;   // 0: a 16-token tile
-    const uint32_t tile_tok = p.tt == 0 ? 16u : 32u * (uint32_t)p.tt;
+    p.tt = tokens > 16 ? 1 : 0;   // 0: a 16-token tile
+    const uint32_t tile_tok = p.tt == 0 ? 16u : 32u;
     const uint32_t tok_tiles = (tokens + tile_tok - 1) / tile_tok, row_tiles = (m.rows + FG_ROWS - 1) / FG_ROWS;
     const uint32_t tiles = tok_tiles * row_tiles, n_steps = (m.cols + FG_K - 1) / FG_K;
     // about two workgroups per CU (16-token tiles measured at 1 / 2 / 3 / 4 per CU: F16 4096x14336, 8 tokens, 51 / 40 / 40 / 44 us)
@@ -715,13 +716,101 @@ static hipError_t launch_fg(hipStream_t stream, const MatView &m, uint32_t token
     p.job.part = static_cast<float *>(ws);
     hipError_t e;
     if (m.type == T_F16)
-        e = p.tt == 2 ? launch_fg_main<T_F16, 2>(stream, p) : p.tt == 1 ? launch_fg_main<T_F16, 1>(stream, p) : launch_fg_main<T_F16, 0>(stream, p);
+        e = p.tt == 1 ? launch_fg_main<T_F16, 1>(stream, p) : launch_fg_main<T_F16, 0>(stream, p);
     else
-        e = p.tt == 2 ? launch_fg_main<T_F32, 2>(stream, p) : p.tt == 1 ? launch_fg_main<T_F32, 1>(stream, p) : launch_fg_main<T_F32, 0>(stream, p);
+        e = p.tt == 1 ? launch_fg_main<T_F32, 1>(stream, p) : launch_fg_main<T_F32, 0>(stream, p);
     if (e != hipSuccess || p.job.ksplit < 2) return e;
     const size_t total = (size_t)tokens * m.rows, vec = (total + 3) / 4, blocks = (vec + 255) / 256;
     hipLaunchKernelGGL(fg_reduce_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, stream, p.job.part, y, total,
                        p.job.ksplit);
+    return hipGetLastError();
+}
+
+// F32 / F16 weights, more tokens: pg_split_kernel, gemm_plain_kernel (+ fg_reduce_kernel).
+struct PgPlan {
+    PgJob job;
+    uint32_t tok, wgs;
+    size_t x_bytes, part_bytes;
+};
+// Whether a product of F32 / F16 weights takes gemm_plain_kernel.  Up to 16 tokens the launch that cuts the activations
+// costs more than the faster matrix instruction gives (F16 4096x14336, 8 tokens: 40 us on the f32 instruction, 44 here);
+// up to 32 only the two parts of F16 weights are worth it, for matrices large enough to hide that launch (52 -> 46 us;
+// 1000x2048 13.3 -> 14.1; F32 56 -> 61).
+static bool pg_takes(const MatView &m, uint32_t tokens) {
+    return tokens > 32 || (tokens > 16 && m.type == T_F16 && (size_t)m.rows * m.cols >= ((size_t)1 << 23));
+}
+// Token tile and column shares, priced together: a step of a workgroup that shares its CU with another and of one that
+// has it alone (us, F16, measured on 4096x14336 with 512 tokens: the wider tile reads and cuts its weights for more
+// tokens), two steps for a workgroup's start and end, and what the launch that sums the shares costs (3 TB/s + 3.5 us).
+// Wide tiles win where there is work for the whole chip (512 tokens: 444 / 334 / 312 us with tiles of 32 / 64 / 128),
+// narrow ones where rows and tokens are few (300x1000, 128 tokens: 14.4 / 15.9 / 21.3 us).
+static void pg_plan(const MatView &m, uint32_t tokens, PgPlan &p) {
+    static constexpr uint32_t tile[3] = {32, 64, 128};
+    static constexpr double shared_us[3] = {0.47, 0.69, 1.25}, alone_us[3] = {0.55, 0.8, 1.39};
+    const uint32_t row_tiles = (m.rows + PG_ROWS - 1) / PG_ROWS, n_steps = (m.cols + PG_K - 1) / PG_K;
+    uint32_t ks_max = n_steps / 8;  // a share is at least 256 columns
+    ks_max = ks_max > 32 ? 32 : ks_max < 1 ? 1 : ks_max;
+    double best = 0.0;
+    uint32_t tok = 0, ks = 1;
+    for (int k = 0; k < 3; k++) {
+        if (k > 0 && tokens <= tile[k - 1]) break;
+        const uint32_t tiles = (tokens + tile[k] - 1) / tile[k] * row_tiles;
+        for (uint32_t s = 1; s <= ks_max; s++) {
+            const uint64_t wgs = (uint64_t)tiles * s, per_cu = (wgs + (uint32_t)g_cu_count - 1) / (uint32_t)g_cu_count;
+            double cost = ((double)((n_steps + s - 1) / s) + 2.0) * (per_cu == 1 ? alone_us[k] : (double)per_cu * shared_us[k]);
+            if (s > 1) cost += (double)s * tokens * m.rows * sizeof(float) / 3.0e6 + 3.5;
+            if (tok == 0 || cost < best) {
+                best = cost;
+                tok = tile[k];
+                ks = s;
+            }
+        }
+    }
+    p.tok = tok;
+    p.job = PgJob{};
+    p.job.m = m;
+    p.job.tokens = tokens;
+    p.job.tok_tiles = (tokens + tok - 1) / tok;
+    p.job.ksplit = ks;
+    p.job.mpad = p.job.tok_tiles * tok;
+    p.job.n_steps = n_steps;
+    p.wgs = p.job.tok_tiles * row_tiles * ks;
+    p.x_bytes = up256((size_t)n_steps * 12 * p.job.mpad * sizeof(uint4));
+    p.part_bytes = ks > 1 ? up256((size_t)ks * tokens * m.rows * sizeof(float)) : 0;
+}
+
+template <uint32_t T, int TOK>
+static hipError_t launch_pg_main(hipStream_t stream, const PgPlan &p) {
+    constexpr size_t lds = 2 * PgTraits<T, TOK>::STAGE;
+    auto kern = gemm_plain_kernel<T, TOK>;
+    static bool configured = false;
+    if (lds > 48 * 1024 && !configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        configured = true;
+    }
+    hipLaunchKernelGGL(kern, dim3(p.wgs), dim3(256), lds, stream, p.job);
+    return hipGetLastError();
+}
+
+static hipError_t launch_pg(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *y, void *ws, size_t ws_bytes) {
+    PgPlan p;
+    pg_plan(m, tokens, p);
+    if (p.x_bytes + p.part_bytes > ws_bytes) return hipErrorInvalidValue;
+    p.job.x = x;
+    p.job.y = y;
+    p.job.xb = static_cast<uint4 *>(ws);
+    p.job.part = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + p.x_bytes);
+    hipLaunchKernelGGL(pg_split_kernel, dim3((p.job.mpad + PG_XS_TOK - 1) / PG_XS_TOK, (p.job.n_steps * PG_K + PG_XS_COLS - 1) / PG_XS_COLS),
+                       dim3(256), 0, stream, p.job);
+    hipError_t e;
+    if (m.type == T_F16)
+        e = p.tok == 128 ? launch_pg_main<T_F16, 128>(stream, p) : p.tok == 64 ? launch_pg_main<T_F16, 64>(stream, p) : launch_pg_main<T_F16, 32>(stream, p);
+    else
+        e = p.tok == 128 ? launch_pg_main<T_F32, 128>(stream, p) : p.tok == 64 ? launch_pg_main<T_F32, 64>(stream, p) : launch_pg_main<T_F32, 32>(stream, p);
+    if (e != hipSuccess || p.job.ksplit < 2) return e;
+    const size_t total = (size_t)tokens * m.rows, vec = (total + 3) / 4, blocks = (vec + 255) / 256;
+    hipLaunchKernelGGL(fg_reduce_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, stream, p.job.part, y, total, p.job.ksplit);
     return hipGetLastError();
 }
 
@@ -790,9 +879,17 @@ size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_
         const uint32_t run = mm_run(mats, tokens, n, g);
         if (run == 0) {
             if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
-                FgPlan p;
-                fg_plan(mats[g], tokens[g], p);
-                need = p.part_bytes > need ? p.part_bytes : need;
+                size_t bytes;
+                if (pg_takes(mats[g], tokens[g])) {
+                    PgPlan p;
+                    pg_plan(mats[g], tokens[g], p);
+                    bytes = p.x_bytes + p.part_bytes;
+                } else {
+                    FgPlan p;
+                    fg_plan(mats[g], tokens[g], p);
+                    bytes = p.part_bytes;
+                }
+                need = bytes > need ? bytes : need;
             }
             g++;
             continue;
@@ -822,7 +919,8 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
                 for (uint32_t t = 0; t < tokens[g] && e == hipSuccess; t++)
                     e = launch_plain(stream, mats[g], 1, xs[g] + (size_t)t * mats[g].cols, ys[g] + (size_t)t * mats[g].rows);
             } else if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
-                e = launch_fg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes);
+                e = pg_takes(mats[g], tokens[g]) ? launch_pg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes)
+                                                : launch_fg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes);
             } else {
                 e = launch_plain(stream, mats[g], tokens[g], xs[g], ys[g]);
             }

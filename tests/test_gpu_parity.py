@@ -390,6 +390,30 @@ def test_plain_dtypes_on_the_matrix_cores_every_tile_and_share_shape(pkg, gpu, t
         m.close()
 
 
+@pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,tokens", [(4100, 333, 300), (8200, 330, 257), (4097, 1032, 65), (2050, 8, 33), (4224, 8192, 20),
+                                              (3000, 2050, 129), (128, 520, 64), (1, 32, 400), (9000, 64, 513)])
+def test_plain_dtypes_cut_into_bf16_parts(pkg, gpu, ty, rows, cols, tokens):
+    """F16 / F32 weights with more than 32 tokens (F16 from 17 in large matrices): products of exact bf16 parts on tiles of
+    32, 64 and 128 tokens, column counts off the step of 32 and off 16-byte rows, activations over many binades, some
+    zero.  A sample of rows on both sides of the 128-row tiles, with the bound of a sequential f32 sum."""
+    rng = np.random.default_rng(rows + tokens)
+    w = K.random_packed(ty, rows, cols, rng)
+    x = (rng.normal(0, 1, (tokens, cols)) * 2.0 ** rng.integers(-30, 12, (tokens, cols))).astype(np.float32)
+    x[rng.random((tokens, cols)) < 0.1] = 0
+    m = gpu.upload_packed(ty, rows, cols, w)
+    y = np.full(tokens * rows, np.nan, np.float32)
+    gpu.gemm_resident(m, tokens, x.ravel(), y)
+    m.close()
+    y = y.reshape(tokens, rows)
+    assert np.isfinite(y).all()
+    sample = sorted({r for r in (0, 31, 32, 63, 64, 127, 128, 129, rows // 2, rows - 129, rows - 2, rows - 1) if 0 <= r < rows})
+    rb = K.row_bytes(ty, cols)
+    ws = np.concatenate([w[r * rb:(r + 1) * rb] for r in sample])
+    exact, mag = O.gemm_f64_mag(ty, cols, tokens, ws, x.ravel(), len(sample))
+    assert np.all(np.abs(y[:, sample] - exact.reshape(tokens, -1)) <= K.single_kernel_bound(cols, mag.reshape(tokens, -1)))
+
+
 @pytest.mark.parametrize("ty", O.ALL_TYPES, ids=lambda t: O.TYPE_NAMES[t])
 def test_random_gemv_and_gemm_within_bounds(pkg, gpu, ty):
     """Signed scales, every code value, int8 -128, token counts across the kernel switch points."""
@@ -878,6 +902,28 @@ def test_edge_sample_collision_does_not_alias(pkg):
     check(yb, K.Q8_0, cols, 1, rows, b, x)
     assert not np.array_equal(ya, yb)
     assert pkg.cache_stats()["entries"] == 2
+
+
+@pytest.mark.parametrize("rows,at", [(1, 40), (690, 0), (694, 32 * 4), (695, -35), (3000, 98304 - 1), (3000, 98304)])
+def test_large_weights_differing_in_one_byte_do_not_alias(pkg, rows, at):
+    """Weights on both sides of the size from which worker threads compare them (Q8_0 rows of 272 bytes), one byte
+    apart beyond the edge sample: at a piece's first or last byte, or right behind and before the samples.  The product
+    begun for the resident matrix is dropped when the bytes turn out to differ."""
+    rng = np.random.default_rng(rows)
+    cols = 256
+    a = K.random_packed(K.Q8_0, rows, cols, rng)
+    b = a.copy()
+    place = at % a.size if at else a.size // 2
+    place += place % 34 in (0, 1) and 2   # a code, not a block's scale
+    b[place] ^= 0x55
+    x = rng.normal(0, 1, cols).astype(np.float32)
+    pkg.reset()
+    for w in (a, b, a, b):
+        y = np.zeros(rows, np.float32)
+        pkg.gemv(K.Q8_0, cols, w, x, y)
+        check(y, K.Q8_0, cols, 1, rows, w, x)
+    stats = pkg.cache_stats()
+    assert (stats["entries"], stats["hits"], stats["misses"]) == (2, 2, 2)
 
 
 # ------------------------------------------------------------------ device-resident buffers

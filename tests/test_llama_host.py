@@ -279,6 +279,25 @@ def test_forward_matches_an_independent_float64_restatement(llama, tiny_path):
     assert int(np.argmax(want[-1])) == llama.argmax(got)
 
 
+@pytest.mark.parametrize("n_embd,n_head,n_head_kv", [(96, 16, 4), (160, 4, 2), (288, 8, 8)])
+def test_attention_of_head_sizes_off_the_vector_strips(llama, tmp_path, n_embd, n_head, n_head_kv):
+    """Head sizes 6, 40 and 36 (neither whole vectors of 4 nor strips of 32 dimensions) at 1 to 35 positions (sums of
+    sixteen positions at a time), against the float64 restatement with the tolerance of the test above."""
+    path = str(tmp_path / "m.gguf")
+    llama.write_synthetic_llama(path, n_layer=1, n_embd=n_embd, n_head=n_head, n_head_kv=n_head_kv, n_ff=64, n_vocab=96,
+                                block_type=8, embd_type=8, output_type=8, seed=n_embd)
+    blob = np.fromfile(path, dtype=np.uint8)
+    m = llama.Llama(blob=blob, products=llama.CALLBACK, matmul=oracle_matmul)
+    tokens = [(7 * i * i + 3 * i) % 96 for i in range(35)]
+    want = numpy_forward(blob, llama.gguf_tensors(blob), m.hparams, tokens)
+    scale = np.abs(want).max()
+    s = m.session(kv_block=5)
+    done = 0
+    for upto in (1, 15, 16, 17, 32, 35):
+        assert np.abs(s.forward(tokens[done:upto]) - want[upto - 1]).max() <= 2e-4 * scale, upto
+        done = upto
+
+
 def test_paged_kv_is_independent_of_block_size_and_placement(llama, tiny_path):
     """langtax/src/kv_page.rs:410-438: only addressing changes, so logits are bit-identical."""
     m = llama.Llama(path=tiny_path, products=llama.CALLBACK, matmul=oracle_matmul)

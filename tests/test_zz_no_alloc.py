@@ -95,6 +95,29 @@ def test_noalloc_plain_dtypes_with_shared_columns(gpu, hip, ty):
         m2.close()
 
 
+@pytest.mark.parametrize("tokens", [801, 1700])
+def test_noalloc_plain_dtype_whose_cut_activations_exceed_the_workspace(gpu, hip, tokens):
+    """The three bf16 parts of 801 x 14336 activations alone are 74 MB: the call goes out in pieces.  Against the
+    allocating call, whose sums may be shared differently: twice the bound of either."""
+    rng = np.random.default_rng(tokens)
+    rows, cols = 40, 14336
+    w = K.random_packed(K.F16, rows, cols, rng)
+    m = gpu.upload_packed(K.F16, rows, cols, w)
+    x = rng.normal(0, 1, tokens * cols).astype(np.float32)
+    xd, yd = hip.DeviceBuffer.from_numpy(x), hip.DeviceBuffer(tokens * rows * 4)
+    gpu.gemm_device(m, tokens, xd.ptr, yd.ptr)
+    gpu.synchronize()
+    ref = yd.to_numpy(np.float32)
+    yd.fill_byte(0xff)
+    hip.device_synchronize()
+    gpu.gemm_device_noalloc(m, tokens, xd.ptr, yd.ptr)
+    gpu.synchronize()
+    got = yd.to_numpy(np.float32)
+    mag = K.abs_product(K.F16, rows, cols, w, x).ravel()
+    assert np.all(np.abs(got.astype(np.float64) - ref) <= 2 * K.single_kernel_bound(cols, mag))
+    m.close(); xd.free(); yd.free()
+
+
 @pytest.mark.parametrize("ty,tokens", [(K.Q4_K, 24), (K.Q5_1, 7), (K.Q8_0, 70), (K.F16, 5)])
 def test_noalloc_recorded_into_a_graph_and_replayed(gpu, hip, ty, tokens):
     """What the entry point is for: a call recorded while the stream is being captured (nothing may be allocated
