@@ -73,7 +73,7 @@ int lnm_session_new(lnm_model *model, size_t kv_block, const uint32_t *block_ids
  * (langtax/src/native_gpu.rs:124-213); the arithmetic of the small kernels is the host code's, element for
  * element, except for the order of the sums inside RMSNorm and the softmax denominator.
  * `max_positions` sizes the cache (rounded up to whole blocks).  A batch of n >= 3 tokens runs its first n - 1
- * tokens through the multi-token products in chunks of up to 128 (only their K and V are kept) and the last one
+ * tokens through the multi-token products in chunks of up to 512 (only their K and V are kept) and the last one
  * as a step; the environment variable LLAMA_HIP_DECODE_STEP_PREFILL makes every token a step. */
 int lnm_session_new_device(lnm_model *model, size_t kv_block, const uint32_t *block_ids, size_t n_block_ids,
                            size_t max_positions, lnm_session **out);
@@ -87,7 +87,7 @@ int lnm_session_new_device_batch(lnm_model *model, size_t kv_block, size_t n_seq
                                  lnm_session **out);
 /* Greedy decode of all sequences from scratch: `prompts` holds the prompts one after the other, prompt_lens[b]
  * tokens for sequence b (at least 1); out[b * n_new + i] is token i of sequence b.  Prompts run one sequence
- * after the other (all tokens but the last in chunks of up to 128, K and V only), then n_new steps of all
+ * after the other (all tokens but the last, in chunks of up to 512 that several prompts may share, K and V only), then n_new steps of all
  * sequences together, step 0 taking every prompt's last token. */
 int lnm_batch_generate_greedy(lnm_session *session, const uint32_t *prompts, const size_t *prompt_lens, size_t n_new,
                               uint32_t *out, double *prefill_seconds, double *decode_seconds);
