@@ -590,9 +590,9 @@ static hipError_t launch_mm16_main(hipStream_t stream, const MmBatch &b) {
     if constexpr (T == T_Q4_0 && !FB) {
         if (g_nibble_i4) return launch_mm16_main<T, INLINE, true, NORM, NT>(stream, b);
     }
-    constexpr size_t lds = Mm16Traits<T, NT>::LDS_BYTES;  // two pipeline stages, the scale exchange
+    constexpr size_t lds = Mm16Traits<T, NT>::LDS_BYTES;  // per group of wavefronts two pipeline stages and the exchange slots
     static_assert(lds <= 48 * 1024, "within the default dynamic LDS limit");
-    hipLaunchKernelGGL((gemm_mfma16_kernel<T, FB, INLINE, NORM, NT>), dim3(b.total_wgs), dim3(256), lds, stream, b);
+    hipLaunchKernelGGL((gemm_mfma16_kernel<T, FB, INLINE, NORM, NT>), dim3(b.total_wgs), dim3(Mm16Traits<T, NT>::THREADS), lds, stream, b);
     return hipGetLastError();
 }
 
