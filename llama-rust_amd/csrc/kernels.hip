@@ -559,16 +559,30 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
 // INLINE (TT = 1): the jobs' x are plain f32 rows and the kernel cuts them itself.
 template <uint32_t T, int TT, int VQ, bool INLINE = false, bool FB = false, bool NORM = false>
 static hipError_t launch_mm_main(hipStream_t stream, const MmBatch &b) {
-    // FB: the device's shortcut from nibbles to bf16 codes is usable (probed at start-up): the packed
-    // fp8 convert for Q4_K, the signed 4-bit convert for Q4_0
-    if constexpr (T == T_Q4_K && !FB) {
-        if (b.nibble_bf16) return launch_mm_main<T, TT, VQ, INLINE, true, NORM>(stream, b);
-    }
+    // FB: the device's shortcut from nibbles to codes is usable (probed at start-up): the signed 4-bit convert for Q4_0
     if constexpr (T == T_Q4_0 && !FB) {
         if (g_nibble_i4) return launch_mm_main<T, TT, VQ, INLINE, true, NORM>(stream, b);
     }
     constexpr size_t lds = 2 * MmStage<T, TT>::BYTES;  // two pipeline stages
     auto kern = gemm_mfma_kernel<T, TT, VQ, FB, INLINE, NORM>;
+    static bool configured = false;
+    if (lds > 48 * 1024 && !configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)lds);
+        if (e != hipSuccess) return e;
+        configured = true;
+    }
+    hipLaunchKernelGGL(kern, dim3(b.total_wgs), dim3(256), lds, stream, b);
+    return hipGetLastError();
+}
+
+// Q4_K, more than 32 tokens
+template <bool FB> static hipError_t launch_mm_q4k64(hipStream_t stream, const MmBatch &b) {
+    if constexpr (!FB) {
+        if (b.nibble_bf16) return launch_mm_q4k64<true>(stream, b);
+    }
+    constexpr size_t lds = 2 * MmQ4k64::BYTES;  // two pipeline stages
+    auto kern = gemm_q4k64_kernel<FB>;
     static bool configured = false;
     if (lds > 48 * 1024 && !configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -638,14 +652,18 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
             return hipGetLastError();
         }
     }
-    if (p.tt == 2) {  // 64-token tiles: the activations are cut once, by a launch of their own
+    if (p.tt == 2)  // 64-token tiles: the activations are cut once, by a launch of their own
         hipLaunchKernelGGL(mm_xsplit_kernel<T>, dim3((b.mpad + XS_TOK - 1) / XS_TOK, (p.n_groups + XS_GRP - 1) / XS_GRP),
                            dim3(256), 0, stream, b, p.n_groups);
-        e = launch_mm_main<T, 2, 4>(stream, b);
-    } else if (p.max_tok <= 8) e = launch_mm_main<T, 1, 1, true>(stream, b);
-    else if (p.max_tok <= 16) e = launch_mm_main<T, 1, 2, true>(stream, b);
-    else if (p.max_tok <= 24) e = launch_mm_main<T, 1, 3, true>(stream, b);
-    else e = launch_mm_main<T, 1, 4, true>(stream, b);
+    if constexpr (T == T_Q4_K) {
+        e = launch_mm_q4k64<false>(stream, b);
+    } else {
+        if (p.tt == 2) e = launch_mm_main<T, 2, 4>(stream, b);
+        else if (p.max_tok <= 8) e = launch_mm_main<T, 1, 1, true>(stream, b);
+        else if (p.max_tok <= 16) e = launch_mm_main<T, 1, 2, true>(stream, b);
+        else if (p.max_tok <= 24) e = launch_mm_main<T, 1, 3, true>(stream, b);
+        else e = launch_mm_main<T, 1, 4, true>(stream, b);
+    }
     if (e != hipSuccess) return e;
     if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
     return hipGetLastError();
@@ -1105,28 +1123,32 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
             if (p.tile16x2)
                 return x_plain ? launch_mm16_main<T, true, false, false, 2>(stream, b) : launch_mm16_main<T, false, false, false, 2>(stream, b);
         }
-        if (norm) {
-            if constexpr (T == T_Q6_K) {  // the other dtypes take 16-token tiles up to 16 tokens
-                if (p.max_tok <= 8) return launch_mm_main<T, 1, 1, true, false, true>(stream, b);
-                if (p.max_tok <= 16) return launch_mm_main<T, 1, 2, true, false, true>(stream, b);
-            }
-            if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true, false, true>(stream, b);
-            return launch_mm_main<T, 1, 4, true, false, true>(stream, b);
-        }
         if (cut_first)
             hipLaunchKernelGGL(mm_xsplit_kernel<T>, dim3((b.mpad + XS_TOK - 1) / XS_TOK, (p.n_groups + XS_GRP - 1) / XS_GRP),
                                dim3(256), 0, stream, b, p.n_groups);
-        if (p.tt == 2) return launch_mm_main<T, 2, 4>(stream, b);
-        if (x_plain) {  // 32-token tiles cut plain activations themselves
-            if (p.max_tok <= 8) return launch_mm_main<T, 1, 1, true>(stream, b);
-            if (p.max_tok <= 16) return launch_mm_main<T, 1, 2, true>(stream, b);
-            if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true>(stream, b);
-            return launch_mm_main<T, 1, 4, true>(stream, b);
+        if constexpr (T == T_Q4_K) {  // up to 32 tokens: above
+            return launch_mm_q4k64<false>(stream, b);
+        } else {
+            if (norm) {
+                if constexpr (T == T_Q6_K) {  // the other dtypes take 16-token tiles up to 16 tokens
+                    if (p.max_tok <= 8) return launch_mm_main<T, 1, 1, true, false, true>(stream, b);
+                    if (p.max_tok <= 16) return launch_mm_main<T, 1, 2, true, false, true>(stream, b);
+                }
+                if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true, false, true>(stream, b);
+                return launch_mm_main<T, 1, 4, true, false, true>(stream, b);
+            }
+            if (p.tt == 2) return launch_mm_main<T, 2, 4>(stream, b);
+            if (x_plain) {  // 32-token tiles cut plain activations themselves
+                if (p.max_tok <= 8) return launch_mm_main<T, 1, 1, true>(stream, b);
+                if (p.max_tok <= 16) return launch_mm_main<T, 1, 2, true>(stream, b);
+                if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true>(stream, b);
+                return launch_mm_main<T, 1, 4, true>(stream, b);
+            }
+            if (p.max_tok <= 8) return launch_mm_main<T, 1, 1>(stream, b);
+            if (p.max_tok <= 16) return launch_mm_main<T, 1, 2>(stream, b);
+            if (p.max_tok <= 24) return launch_mm_main<T, 1, 3>(stream, b);
+            return launch_mm_main<T, 1, 4>(stream, b);
         }
-        if (p.max_tok <= 8) return launch_mm_main<T, 1, 1>(stream, b);
-        if (p.max_tok <= 16) return launch_mm_main<T, 1, 2>(stream, b);
-        if (p.max_tok <= 24) return launch_mm_main<T, 1, 3>(stream, b);
-        return launch_mm_main<T, 1, 4>(stream, b);
     });
     if (e != hipSuccess) return e;
     if (!fused) {

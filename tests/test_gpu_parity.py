@@ -435,6 +435,22 @@ def test_random_gemv_and_gemm_within_bounds(pkg, gpu, ty):
         m.close()
 
 
+@pytest.mark.parametrize("rows,cols,tokens", [(1, 256, 33), (255, 512, 64), (256, 768, 65), (257, 4352, 97), (600, 14336, 128),
+                                              (4099, 1280, 129)])
+def test_q4_k_products_of_more_than_32_tokens(gpu, rows, cols, tokens):
+    """The Q4_K kernel for more than 32 tokens walks pairs of steps and adds the offsets on the matrix cores: rows around
+    its 256-row tile, tokens around its 64-token tile, column counts that give one share of four pairs, shares of
+    unequal length and many shares."""
+    rng = np.random.default_rng(rows + cols + tokens)
+    w = K.random_packed(K.Q4_K, rows, cols, rng)
+    m = gpu.upload_packed(K.Q4_K, rows, cols, w)
+    x = rng.normal(0, 1, tokens * cols).astype(np.float32)
+    y = np.full(tokens * rows, np.nan, np.float32)
+    gpu.gemm_resident(m, tokens, x, y)
+    check(y, K.Q4_K, cols, tokens, rows, w, x)
+    m.close()
+
+
 @pytest.mark.parametrize("ty", [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K, K.Q6_K], ids=lambda t: O.TYPE_NAMES[t])
 def test_multi_token_products_of_random_shapes(pkg, gpu, ty):
     """Seeded sweep over what decides the launch of a multi-token product: rows around the 256-row tile, column
