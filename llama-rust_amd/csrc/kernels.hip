@@ -596,18 +596,28 @@ template <bool FB> static hipError_t launch_mm_q4k64(hipStream_t stream, const M
 
 // INLINE: the jobs' x are plain f32 rows and the kernel cuts them itself (no mm_xsplit launch before it).
 // NT: 16-token tiles per workgroup (2: the plan's 32-token tiles).
-template <uint32_t T, bool INLINE = false, bool FB = false, bool NORM = false, int NT = 1>
-static hipError_t launch_mm16_main(hipStream_t stream, const MmBatch &b) {
+// LO: how many matrix instructions a K-slice takes (the kernel's), by the most tokens of a job.
+template <uint32_t T, bool INLINE, bool FB, bool NORM, int NT, int LO>
+static hipError_t launch_mm16_lo(hipStream_t stream, const MmBatch &b) {
     if constexpr (T == T_Q4_K && !FB) {
-        if (b.nibble_bf16) return launch_mm16_main<T, INLINE, true, NORM, NT>(stream, b);
+        if (b.nibble_bf16) return launch_mm16_lo<T, INLINE, true, NORM, NT, LO>(stream, b);
     }
     if constexpr (T == T_Q4_0 && !FB) {
-        if (g_nibble_i4) return launch_mm16_main<T, INLINE, true, NORM, NT>(stream, b);
+        if (g_nibble_i4) return launch_mm16_lo<T, INLINE, true, NORM, NT, LO>(stream, b);
     }
-    constexpr size_t lds = Mm16Traits<T, NT>::LDS_BYTES;  // per group of wavefronts two pipeline stages and the exchange slots
+    using Tr = Mm16Traits<T, NT, LO>;
+    constexpr size_t lds = Tr::LDS_BYTES;  // per group of wavefronts two pipeline stages and the exchange slots
     static_assert(lds <= 48 * 1024, "within the default dynamic LDS limit");
-    hipLaunchKernelGGL((gemm_mfma16_kernel<T, FB, INLINE, NORM, NT>), dim3(b.total_wgs), dim3(Mm16Traits<T, NT>::THREADS), lds, stream, b);
+    hipLaunchKernelGGL((gemm_mfma16_kernel<T, FB, INLINE, NORM, NT, LO>), dim3(b.total_wgs), dim3(Tr::THREADS), lds, stream, b);
     return hipGetLastError();
+}
+template <uint32_t T, bool INLINE = false, bool NORM = false, int NT = 1>
+static hipError_t launch_mm16_main(hipStream_t stream, const MmBatch &b, uint32_t max_tok) {
+    if constexpr (NT == 1) {
+        if (max_tok <= 5) return launch_mm16_lo<T, INLINE, false, NORM, 1, 1>(stream, b);
+        if (max_tok <= 8) return launch_mm16_lo<T, INLINE, false, NORM, 1, 2>(stream, b);
+    }
+    return launch_mm16_lo<T, INLINE, false, NORM, NT, 3>(stream, b);
 }
 
 // Workgroups per job of the share reduction: one float4 per thread (one float for small jobs, as the kernel
@@ -638,7 +648,7 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
     hipError_t e;
     if constexpr (T != T_Q6_K) {
         if (p.tile16) {  // the 16-token kernel cuts the activations itself
-            e = launch_mm16_main<T, true>(stream, b);
+            e = launch_mm16_main<T, true>(stream, b, p.max_tok);
             if (e != hipSuccess) return e;
             if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
             return hipGetLastError();
@@ -646,7 +656,7 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
     }
     if constexpr (T == T_Q4_K) {
         if (p.tile16x2) {
-            e = launch_mm16_main<T, true, false, false, 2>(stream, b);
+            e = launch_mm16_main<T, true, false, 2>(stream, b, p.max_tok);
             if (e != hipSuccess) return e;
             if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
             return hipGetLastError();
@@ -1115,13 +1125,13 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     hipError_t e = mm_by_type(tiled[0].type, [&](auto t) {
         constexpr uint32_t T = decltype(t)::value;
         if constexpr (T != T_Q6_K) {
-            if (p.tile16 && norm) return launch_mm16_main<T, true, false, true>(stream, b);
-            if (p.tile16) return x_plain ? launch_mm16_main<T, true>(stream, b) : launch_mm16_main<T>(stream, b);
+            if (p.tile16 && norm) return launch_mm16_main<T, true, true>(stream, b, p.max_tok);
+            if (p.tile16) return x_plain ? launch_mm16_main<T, true>(stream, b, p.max_tok) : launch_mm16_main<T>(stream, b, p.max_tok);
         }
         if constexpr (T == T_Q4_K) {
-            if (p.tile16x2 && norm) return launch_mm16_main<T, true, false, true, 2>(stream, b);
+            if (p.tile16x2 && norm) return launch_mm16_main<T, true, true, 2>(stream, b, p.max_tok);
             if (p.tile16x2)
-                return x_plain ? launch_mm16_main<T, true, false, false, 2>(stream, b) : launch_mm16_main<T, false, false, false, 2>(stream, b);
+                return x_plain ? launch_mm16_main<T, true, false, 2>(stream, b, p.max_tok) : launch_mm16_main<T, false, false, 2>(stream, b, p.max_tok);
         }
         if (cut_first)
             hipLaunchKernelGGL(mm_xsplit_kernel<T>, dim3((b.mpad + XS_TOK - 1) / XS_TOK, (p.n_groups + XS_GRP - 1) / XS_GRP),

@@ -451,6 +451,23 @@ def test_q4_k_products_of_more_than_32_tokens(gpu, rows, cols, tokens):
     m.close()
 
 
+@pytest.mark.parametrize("ty", [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K], ids=lambda t: O.TYPE_NAMES[t])
+def test_products_whose_activation_parts_share_an_instruction(gpu, ty):
+    """Up to 5 and up to 8 tokens the activations' parts take rows of the matrix instructions that tokens leave empty:
+    every token count from 3 to 9, one iteration of columns, an odd number, and several shares."""
+    rng = np.random.default_rng(77 + ty)
+    unit = K.QK[ty]
+    for rows, cols in ((65, 256), (257, unit * (3 if unit == 256 else 35)), (300, 8192)):
+        w = K.random_packed(ty, rows, cols, rng)
+        m = gpu.upload_packed(ty, rows, cols, w)
+        for tokens in range(3, 10):
+            x = rng.normal(0, 1, tokens * cols).astype(np.float32)
+            y = np.full(tokens * rows, np.nan, np.float32)
+            gpu.gemm_resident(m, tokens, x, y)
+            check(y, ty, cols, tokens, rows, w, x)
+        m.close()
+
+
 @pytest.mark.parametrize("ty", [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K, K.Q6_K], ids=lambda t: O.TYPE_NAMES[t])
 def test_multi_token_products_of_random_shapes(pkg, gpu, ty):
     """Seeded sweep over what decides the launch of a multi-token product: rows around the 256-row tile, column
