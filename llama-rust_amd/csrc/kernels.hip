@@ -466,6 +466,9 @@ struct MmPlan {
     size_t xb_bytes, sx_bytes, part_bytes;
 };
 
+// Most tokens of a job that the 16-token kernel takes (Q6_K fills its rows with 8).
+static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
+
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Jobs share dtype and column count; every job has at least MM_MIN_TOKENS tokens.
@@ -476,7 +479,7 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     for (uint32_t j = 0; j < n; j++) max_tok = tokens[j] > max_tok ? tokens[j] : max_tok;
     p.tt = max_tok > 32 ? 2 : 1;
     p.max_tok = max_tok;
-    p.tile16 = max_tok <= 16 && mats[0].type != T_Q6_K;
+    p.tile16 = max_tok <= mm_tile16_max(mats[0].type);
     // measured on 4096x14336 / 14336x4096 at 17, 24 and 32 tokens: Q4_K 26.4 / 27.7 / 30.4 -> 25.9 / 27.4 / 28.5 us, a
     // routed layer 394 -> 380 us, 32 sequences decoded together +3 %; Q4_0, Q5_0, Q5_1 and Q8_0 lose 1-2.5 us to the
     // 32-token tile, which skips the matrix-core work of empty token quarters
@@ -576,6 +579,13 @@ static hipError_t launch_mm_main(hipStream_t stream, const MmBatch &b) {
     return hipGetLastError();
 }
 
+// 9 to 16 tokens: only Q6_K gets here, the other dtypes take 16-token tiles
+template <uint32_t T, bool INLINE = false, bool NORM = false>
+static hipError_t launch_mm_main_q6k_16(hipStream_t stream, const MmBatch &b) {
+    if constexpr (T == T_Q6_K) return launch_mm_main<T, 1, 2, INLINE, false, NORM>(stream, b);
+    else return hipErrorInvalidValue;
+}
+
 // Q4_K, more than 32 tokens
 template <bool FB> static hipError_t launch_mm_q4k64(hipStream_t stream, const MmBatch &b) {
     if constexpr (!FB) {
@@ -613,7 +623,7 @@ static hipError_t launch_mm16_lo(hipStream_t stream, const MmBatch &b) {
 }
 template <uint32_t T, bool INLINE = false, bool NORM = false, int NT = 1>
 static hipError_t launch_mm16_main(hipStream_t stream, const MmBatch &b, uint32_t max_tok) {
-    if constexpr (NT == 1) {
+    if constexpr (NT == 1 && T != T_Q6_K) {
         if (max_tok <= 5) return launch_mm16_lo<T, INLINE, false, NORM, 1, 1>(stream, b);
         if (max_tok <= 8) return launch_mm16_lo<T, INLINE, false, NORM, 1, 2>(stream, b);
     }
@@ -646,13 +656,11 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
             part += up256((size_t)b.job[j].ksplit * b.job[j].tokens * b.job[j].m.rows * sizeof(float));
         }
     hipError_t e;
-    if constexpr (T != T_Q6_K) {
-        if (p.tile16) {  // the 16-token kernel cuts the activations itself
-            e = launch_mm16_main<T, true>(stream, b, p.max_tok);
-            if (e != hipSuccess) return e;
-            if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
-            return hipGetLastError();
-        }
+    if (p.tile16) {  // the 16-token kernel cuts the activations itself
+        e = launch_mm16_main<T, true>(stream, b, p.max_tok);
+        if (e != hipSuccess) return e;
+        if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
+        return hipGetLastError();
     }
     if constexpr (T == T_Q4_K) {
         if (p.tile16x2) {
@@ -669,8 +677,7 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
         e = launch_mm_q4k64<false>(stream, b);
     } else {
         if (p.tt == 2) e = launch_mm_main<T, 2, 4>(stream, b);
-        else if (p.max_tok <= 8) e = launch_mm_main<T, 1, 1, true>(stream, b);
-        else if (p.max_tok <= 16) e = launch_mm_main<T, 1, 2, true>(stream, b);
+        else if (T == T_Q6_K && p.max_tok <= 16) e = launch_mm_main_q6k_16<T, true>(stream, b);
         else if (p.max_tok <= 24) e = launch_mm_main<T, 1, 3, true>(stream, b);
         else e = launch_mm_main<T, 1, 4, true>(stream, b);
     }
@@ -893,7 +900,7 @@ static void mm_classes(const MatView *mats, const uint32_t *tokens, const float 
                        MmClass (&cls)[2]) {
     cls[0].n = cls[1].n = 0;
     for (uint32_t j = 0; j < run; j++) {
-        MmClass &c = cls[tokens[j] <= 16 && mats[j].type != T_Q6_K ? 0 : 1];
+        MmClass &c = cls[tokens[j] <= mm_tile16_max(mats[j].type) ? 0 : 1];
         c.mats[c.n] = mats[j];
         c.tokens[c.n] = tokens[j];
         c.xs[c.n] = xs ? xs[j] : nullptr;
@@ -973,7 +980,7 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
 
 // ---- activations that stay in the split form between products
 
-static uint32_t act_mpad(uint32_t type, uint32_t tokens) { return tokens + (tokens <= 16 && type != T_Q6_K ? 16u : 64u); }
+static uint32_t act_mpad(uint32_t type, uint32_t tokens) { return tokens + (tokens <= mm_tile16_max(type) ? 16u : 64u); }
 
 size_t act_bytes(uint32_t type, uint32_t cols, uint32_t max_tokens) {
     if (!mm_type(type) || cols % 32 != 0 || max_tokens == 0) return 0;
@@ -1124,10 +1131,8 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     }
     hipError_t e = mm_by_type(tiled[0].type, [&](auto t) {
         constexpr uint32_t T = decltype(t)::value;
-        if constexpr (T != T_Q6_K) {
-            if (p.tile16 && norm) return launch_mm16_main<T, true, true>(stream, b, p.max_tok);
-            if (p.tile16) return x_plain ? launch_mm16_main<T, true>(stream, b, p.max_tok) : launch_mm16_main<T>(stream, b, p.max_tok);
-        }
+        if (p.tile16 && norm) return launch_mm16_main<T, true, true>(stream, b, p.max_tok);
+        if (p.tile16) return x_plain ? launch_mm16_main<T, true>(stream, b, p.max_tok) : launch_mm16_main<T>(stream, b, p.max_tok);
         if constexpr (T == T_Q4_K) {
             if (p.tile16x2 && norm) return launch_mm16_main<T, true, true, 2>(stream, b, p.max_tok);
             if (p.tile16x2)
@@ -1140,22 +1145,17 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
             return launch_mm_q4k64<false>(stream, b);
         } else {
             if (norm) {
-                if constexpr (T == T_Q6_K) {  // the other dtypes take 16-token tiles up to 16 tokens
-                    if (p.max_tok <= 8) return launch_mm_main<T, 1, 1, true, false, true>(stream, b);
-                    if (p.max_tok <= 16) return launch_mm_main<T, 1, 2, true, false, true>(stream, b);
-                }
+                if (T == T_Q6_K && p.max_tok <= 16) return launch_mm_main_q6k_16<T, true, true>(stream, b);
                 if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true, false, true>(stream, b);
                 return launch_mm_main<T, 1, 4, true, false, true>(stream, b);
             }
             if (p.tt == 2) return launch_mm_main<T, 2, 4>(stream, b);
             if (x_plain) {  // 32-token tiles cut plain activations themselves
-                if (p.max_tok <= 8) return launch_mm_main<T, 1, 1, true>(stream, b);
-                if (p.max_tok <= 16) return launch_mm_main<T, 1, 2, true>(stream, b);
+                if (T == T_Q6_K && p.max_tok <= 16) return launch_mm_main_q6k_16<T, true>(stream, b);
                 if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true>(stream, b);
                 return launch_mm_main<T, 1, 4, true>(stream, b);
             }
-            if (p.max_tok <= 8) return launch_mm_main<T, 1, 1>(stream, b);
-            if (p.max_tok <= 16) return launch_mm_main<T, 1, 2>(stream, b);
+            if (T == T_Q6_K && p.max_tok <= 16) return launch_mm_main_q6k_16<T>(stream, b);
             if (p.max_tok <= 24) return launch_mm_main<T, 1, 3>(stream, b);
             return launch_mm_main<T, 1, 4>(stream, b);
         }

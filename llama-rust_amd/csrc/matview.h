@@ -164,7 +164,7 @@ inline PlaneSpec plane_spec(uint32_t t, size_t rows, size_t cols) {
 //   Q5_0 : codes 16 B x nb   | qh 4 B x nb | d 2 B x nb
 //   Q5_1 : codes 16 B x nb   | qh 4 B x nb | (d, m) 4 B x nb
 //   Q4_K : codes 16 B x 8 nb | header 16 B x nb (its scales regrouped: q4k_tiled_header, repack.inc)
-//   Q6_K : ql 16 B x 8 nb    | qh 16 B x 4 nb | sc 8 B x 2 nb | d 2 B x nb
+//   Q6_K : ql 16 B x 8 nb    | qh 16 B x 4 nb (every second bit flipped) | sc 8 B x 2 nb | d 2 B x nb
 // (code units in the order of the GGUF block).  F32/F16 have no such copy.
 constexpr uint32_t TILE_ROWS = 256;
 

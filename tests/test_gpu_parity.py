@@ -451,10 +451,10 @@ def test_q4_k_products_of_more_than_32_tokens(gpu, rows, cols, tokens):
     m.close()
 
 
-@pytest.mark.parametrize("ty", [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K], ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("ty", [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K, K.Q6_K], ids=lambda t: O.TYPE_NAMES[t])
 def test_products_whose_activation_parts_share_an_instruction(gpu, ty):
-    """Up to 5 and up to 8 tokens the activations' parts take rows of the matrix instructions that tokens leave empty:
-    every token count from 3 to 9, one iteration of columns, an odd number, and several shares."""
+    """Up to 5 and up to 8 tokens the activations' parts (Q6_K: their halves, a scale each) take rows of the matrix
+    instructions that tokens leave empty: every token count from 3 to 9, one iteration of columns, an odd number, and several shares."""
     rng = np.random.default_rng(77 + ty)
     unit = K.QK[ty]
     for rows, cols in ((65, 256), (257, unit * (3 if unit == 256 else 35)), (300, 8192)):
