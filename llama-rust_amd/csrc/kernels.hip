@@ -591,16 +591,7 @@ template <bool FB> static hipError_t launch_mm_q4k64(hipStream_t stream, const M
     if constexpr (!FB) {
         if (b.nibble_bf16) return launch_mm_q4k64<true>(stream, b);
     }
-    constexpr size_t lds = 2 * MmQ4k64::BYTES;  // two pipeline stages
-    auto kern = gemm_q4k64_kernel<FB>;
-    static bool configured = false;
-    if (lds > 48 * 1024 && !configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)lds);
-        if (e != hipSuccess) return e;
-        configured = true;
-    }
-    hipLaunchKernelGGL(kern, dim3(b.total_wgs), dim3(256), lds, stream, b);
+    hipLaunchKernelGGL(gemm_q4k64_kernel<FB>, dim3(b.total_wgs), dim3(256), 0, stream, b);
     return hipGetLastError();
 }
 
