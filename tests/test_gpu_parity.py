@@ -414,6 +414,61 @@ def test_plain_dtypes_cut_into_bf16_parts(pkg, gpu, ty, rows, cols, tokens):
     assert np.all(np.abs(y[:, sample] - exact.reshape(tokens, -1)) <= K.single_kernel_bound(cols, mag.reshape(tokens, -1)))
 
 
+def product_by_ieee_rules(w, x):
+    """x w^T as f32 arithmetic in any order defines it where operands are infinite or NaN, the float64 product elsewhere;
+    and the sum of the absolute finite terms."""
+    w, x = w.astype(np.float64), x.astype(np.float64)
+    fw, fx = np.where(np.isfinite(w), w, 0), np.where(np.isfinite(x), x, 0)
+    out, mag = fx @ fw.T, np.abs(fx) @ np.abs(fw).T
+
+    def pairs(a, b):   # whether any column has a in x beside b in w
+        return a.astype(np.float32) @ b.T.astype(np.float32) > 0
+
+    up, down = np.zeros(out.shape, bool), np.zeros(out.shape, bool)
+    for sx in (1, -1):
+        for sw in (1, -1):
+            hit = pairs(x == sx * np.inf, sw * w > 0) | pairs(sx * x > 0, w == sw * np.inf)
+            up, down = (up | hit, down) if sx == sw else (up, down | hit)
+    nan = pairs(np.isnan(x), np.ones(w.shape)) | pairs(np.ones(x.shape), np.isnan(w))
+    nan |= pairs(np.isinf(x), w == 0) | pairs(x == 0, np.isinf(w)) | (up & down)
+    out[up], out[down], out[nan] = np.inf, -np.inf, np.nan
+    return out, mag
+
+
+@pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,tokens", [(200, 1001, 33), (129, 4099, 64), (257, 2048, 128), (4096, 2056, 20), (40, 264, 300),
+                                              (300, 520, 4), (300, 520, 1)])
+def test_plain_dtypes_multiply_infinities_and_nan_like_f32(gpu, ty, rows, cols, tokens):
+    """An infinity times a number is an infinity, times zero a NaN, whatever the number of tokens and however the operands
+    are cut: infinite and NaN activations and weights in single tokens and rows, in the last column too, beside weights
+    of few significand bits (whose later parts are zero), zero weights and zero activations."""
+    rng = np.random.default_rng(rows + cols + tokens)
+    w = rng.normal(0, 1, (rows, cols)).astype(np.float32)
+    w[:, ::2] = (w[:, ::2].view(np.uint32) & 0xffff0000).view(np.float32)   # as converted from bf16
+    w[rng.random(w.shape) < 1e-3] = 0
+    w = w.astype(np.float16).astype(np.float32) if ty == K.F16 else w
+    x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    x[rng.random(x.shape) < 1e-3] = 0
+    w[3, cols - 1], w[rows - 1, 5], w[17, 33], w[36, 8] = np.inf, -np.inf, np.nan, np.inf
+    if tokens > 1:
+        x[0, 7], x[3, cols - 1], x[2, 40], x[2, 41] = np.inf, -np.inf, np.inf, -np.inf
+        x[1, cols - 1] = 0
+    if tokens > 4:
+        x[tokens - 2, 100] = np.nan
+    packed = (w.astype(np.float16) if ty == K.F16 else w).view(np.uint8).reshape(-1)
+    m = gpu.upload_packed(ty, rows, cols, np.ascontiguousarray(packed))
+    y = np.zeros(tokens * rows, np.float32)
+    gpu.gemm_resident(m, tokens, np.ascontiguousarray(x).ravel(), y)
+    m.close()
+    y = y.reshape(tokens, rows)
+    want, mag = product_by_ieee_rules(w, x)
+    finite = np.isfinite(want)
+    assert finite.any() and np.isinf(want).any() and np.isnan(want).any()
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    assert np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
+    assert np.all(np.abs(y[finite] - want[finite]) <= K.single_kernel_bound(cols, mag[finite]))
+
+
 @pytest.mark.parametrize("ty", O.ALL_TYPES, ids=lambda t: O.TYPE_NAMES[t])
 def test_random_gemv_and_gemm_within_bounds(pkg, gpu, ty):
     """Signed scales, every code value, int8 -128, token counts across the kernel switch points."""
