@@ -155,8 +155,10 @@ int lnh_gemm_grouped_device(lnh_exec *exec, size_t n_groups, const lnh_matrix *c
  * kernels, same results as lnh_gemm_device, but the workspace of the multi-token kernels is a fixed
  * array inside the library's device code (LNH_NOALLOC_WORKSPACE_BYTES per GPU, held from lnh_create on
  * that GPU until the process ends) instead of the executor's grow-on-demand allocation: the call
- * never allocates or frees.  A product that needs more fails with LNH_ERR_INVALID
- * (the message states the need) before anything is launched; so does a product of three or more tokens by a
+ * never allocates or frees.  A product by a quantized matrix that needs more fails with LNH_ERR_INVALID
+ * (the message states the need) before anything is launched; one by an F32 / F16 matrix goes out in pieces of
+ * fewer tokens instead, with the same sums (rows of some 270000 columns and more take another kernel, whose sums
+ * are taken in another order).  Refused likewise is a product of three or more tokens by a
  * quantized matrix whose multi-token layout has not been made yet (lnh_matrix_prepare, or any earlier such product
  * through an allocating entry point, makes it).  Every call on one GPU, from any executor, uses the
  * same array and nothing in it outlives a call: calls that may overlap on one GPU (different streams,

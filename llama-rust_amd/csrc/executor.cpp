@@ -714,15 +714,7 @@ int lnh_gemm_device_noalloc(lnh_exec *e, const lnh_matrix *m, size_t tokens, con
     void *ws = nh::static_scratch(e->ctx->device);
     if (!ws) return fail(e, LNH_ERR_DEVICE, "static workspace of this device was not initialised");
     const uint32_t tok32 = (uint32_t)tokens;
-    size_t need = nh::gemm_workspace_bytes(&m->view, &tok32, 1);
-    // F32 / F16 weights cut their activations into the workspace, all tokens at once; such a product goes out in as many
-    // pieces as it takes for their activations to fit, down to the sizes that cut nothing
-    uint32_t piece = tok32;
-    if (m->view.type == nh::T_F32 || m->view.type == nh::T_F16)
-        while (need > nh::STATIC_SCRATCH_BYTES && piece > 16) {
-            piece = (piece + 1) / 2;
-            need = nh::gemm_workspace_bytes(&m->view, &piece, 1);
-        }
+    const size_t need = nh::gemm_workspace_bytes(&m->view, &tok32, 1, true);
     if (need > nh::STATIC_SCRATCH_BYTES)
         return fail(e, LNH_ERR_INVALID,
                     "product needs " + std::to_string(need) + " bytes of workspace, the allocation-free entry point holds " +
@@ -736,13 +728,7 @@ int lnh_gemm_device_noalloc(lnh_exec *e, const lnh_matrix *m, size_t tokens, con
                         "the matrix has no multi-token copy yet and this entry point does not allocate: call lnh_matrix_prepare first");
         tiled = m->tiled;
     }
-    hipError_t h = hipSuccess;
-    for (uint32_t t = 0; t < tok32 && h == hipSuccess; t += piece) {
-        const uint32_t n = tok32 - t < piece ? tok32 - t : piece;
-        const float *x = dx + (size_t)t * m->view.cols;
-        float *y = dy + (size_t)t * m->view.rows;
-        h = nh::launch_gemm_groups(s, &m->view, &tiled, &n, &x, &y, 1, ws, nh::STATIC_SCRATCH_BYTES);
-    }
+    const hipError_t h = nh::launch_gemm_groups(s, &m->view, &tiled, &tok32, &dx, &dy, 1, ws, nh::STATIC_SCRATCH_BYTES);
     if (h != hipSuccess) return hip_fail(e, h, "HIP kernel launch");
     return LNH_OK;
 }

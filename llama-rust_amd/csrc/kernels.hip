@@ -758,6 +758,23 @@ struct PgPlan {
     uint32_t tok, wgs;
     size_t x_bytes, part_bytes;
 };
+// Sizes of a product of `tokens` tokens on tiles of `tok`, columns shared `ks` ways.
+static void pg_fit(const MatView &m, uint32_t tokens, uint32_t tok, uint32_t ks, PgPlan &p) {
+    const uint32_t row_tiles = (m.rows + PG_ROWS - 1) / PG_ROWS, n_steps = (m.cols + PG_K - 1) / PG_K;
+    p.tok = tok;
+    p.job = PgJob{};
+    p.job.m = m;
+    p.job.tokens = tokens;
+    p.job.tok_tiles = (tokens + tok - 1) / tok;
+    p.job.ksplit = ks;
+    // an odd number of 128-byte lines: a workgroup reads twelve planes of a step at the same slots, and planes a power of two
+    // apart meet on few of the memory's channels (F16 512 tokens 307 -> 301 us, F32 447 -> 437)
+    p.job.mpad = p.job.tok_tiles * tok + 8;
+    p.job.n_steps = n_steps;
+    p.wgs = p.job.tok_tiles * row_tiles * ks;
+    p.x_bytes = up256((size_t)n_steps * 12 * p.job.mpad * sizeof(uint4));
+    p.part_bytes = ks > 1 ? up256((size_t)ks * tokens * m.rows * sizeof(float)) : 0;
+}
 // Whether a product of F32 / F16 weights takes gemm_plain_kernel.  Up to 16 tokens the launch that cuts the activations
 // costs more than the faster matrix instruction gives (F16 4096x14336, 8 tokens: 40 us on the f32 instruction, 44 here);
 // up to 32 only the two parts of F16 weights are worth it, for matrices large enough to hide that launch (52 -> 46 us;
@@ -792,19 +809,25 @@ static void pg_plan(const MatView &m, uint32_t tokens, PgPlan &p) {
             }
         }
     }
-    p.tok = tok;
-    p.job = PgJob{};
-    p.job.m = m;
-    p.job.tokens = tokens;
-    p.job.tok_tiles = (tokens + tok - 1) / tok;
-    p.job.ksplit = ks;
-    // an odd number of 128-byte lines: a workgroup reads twelve planes of a step at the same slots, and planes a power of two
-    // apart meet on few of the memory's channels (F16 512 tokens 307 -> 301 us, F32 447 -> 437)
-    p.job.mpad = p.job.tok_tiles * tok + 8;
-    p.job.n_steps = n_steps;
-    p.wgs = p.job.tok_tiles * row_tiles * ks;
-    p.x_bytes = up256((size_t)n_steps * 12 * p.job.mpad * sizeof(uint4));
-    p.part_bytes = ks > 1 ? up256((size_t)ks * tokens * m.rows * sizeof(float)) : 0;
+    pg_fit(m, tokens, tok, ks, p);
+}
+
+// Tokens per piece of a product that is given less workspace than its plan takes: pieces of whole tiles, as equal as
+// they come, all with the plan's column shares.  The shares alone decide in which order a sum is taken, so every token's
+// results are those of the whole product bit for bit, and a piece of fewer tokens takes less (a plan of its own would
+// share its columns more finely and could take more).  Narrower tiles where not even one fits; 0: none does.
+static uint32_t pg_piece(PgPlan &p, size_t ws_bytes) {
+    const PgJob &j = p.job;
+    if (p.x_bytes + p.part_bytes <= ws_bytes) return j.tokens;
+    const size_t column = (size_t)j.n_steps * 12 * sizeof(uint4), fixed = 8 * column + 512;  // 512: both parts are rounded up
+    for (uint32_t tok = p.tok; tok >= 32; tok /= 2) {
+        const size_t tile = tok * (column + (j.ksplit > 1 ? (size_t)j.ksplit * j.m.rows * sizeof(float) : 0));
+        if (fixed + tile > ws_bytes) continue;
+        const size_t tiles = ((size_t)j.tokens + tok - 1) / tok, most = (ws_bytes - fixed) / tile, pieces = (tiles + most - 1) / most;
+        p.tok = tok;
+        return (uint32_t)((tiles + pieces - 1) / pieces) * tok;
+    }
+    return 0;
 }
 
 template <uint32_t T, int TOK>
@@ -822,23 +845,31 @@ static hipError_t launch_pg_main(hipStream_t stream, const PgPlan &p) {
 }
 
 static hipError_t launch_pg(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *y, void *ws, size_t ws_bytes) {
-    PgPlan p;
-    pg_plan(m, tokens, p);
-    if (p.x_bytes + p.part_bytes > ws_bytes) return hipErrorInvalidValue;
-    p.job.x = x;
-    p.job.y = y;
-    p.job.xb = static_cast<uint4 *>(ws);
-    p.job.part = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + p.x_bytes);
-    hipLaunchKernelGGL(pg_split_kernel, dim3((p.job.mpad + PG_XS_TOK - 1) / PG_XS_TOK, (p.job.n_steps * PG_K + PG_XS_COLS - 1) / PG_XS_COLS),
-                       dim3(256), 0, stream, p.job);
-    hipError_t e;
-    if (m.type == T_F16)
-        e = p.tok == 128 ? launch_pg_main<T_F16, 128>(stream, p) : p.tok == 64 ? launch_pg_main<T_F16, 64>(stream, p) : launch_pg_main<T_F16, 32>(stream, p);
-    else
-        e = p.tok == 128 ? launch_pg_main<T_F32, 128>(stream, p) : p.tok == 64 ? launch_pg_main<T_F32, 64>(stream, p) : launch_pg_main<T_F32, 32>(stream, p);
-    if (e != hipSuccess || p.job.ksplit < 2) return e;
-    const size_t total = (size_t)tokens * m.rows, vec = (total + 3) / 4, blocks = (vec + 255) / 256;
-    hipLaunchKernelGGL(fg_reduce_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, stream, p.job.part, y, total, p.job.ksplit);
+    PgPlan plan;
+    pg_plan(m, tokens, plan);
+    const uint32_t piece = pg_piece(plan, ws_bytes);
+    if (piece == 0) return launch_fg(stream, m, tokens, x, y, ws, ws_bytes);  // rows so long that 32 tokens of them do not fit
+    for (uint32_t t = 0, n; t < tokens; t += n) {
+        n = tokens - t < piece ? tokens - t : piece;
+        PgPlan p;
+        pg_fit(m, n, plan.tok, plan.job.ksplit, p);
+        p.job.x = x + (size_t)t * m.cols;
+        p.job.y = y + (size_t)t * m.rows;
+        p.job.xb = static_cast<uint4 *>(ws);
+        p.job.part = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + p.x_bytes);
+        hipLaunchKernelGGL(pg_split_kernel, dim3((p.job.mpad + PG_XS_TOK - 1) / PG_XS_TOK, (p.job.n_steps * PG_K + PG_XS_COLS - 1) / PG_XS_COLS),
+                           dim3(256), 0, stream, p.job);
+        hipError_t e;
+        if (m.type == T_F16)
+            e = p.tok == 128 ? launch_pg_main<T_F16, 128>(stream, p) : p.tok == 64 ? launch_pg_main<T_F16, 64>(stream, p) : launch_pg_main<T_F16, 32>(stream, p);
+        else
+            e = p.tok == 128 ? launch_pg_main<T_F32, 128>(stream, p) : p.tok == 64 ? launch_pg_main<T_F32, 64>(stream, p) : launch_pg_main<T_F32, 32>(stream, p);
+        if (e != hipSuccess) return e;
+        if (p.job.ksplit < 2) continue;
+        const size_t total = (size_t)n * m.rows, vec = (total + 3) / 4, blocks = (vec + 255) / 256;
+        hipLaunchKernelGGL(fg_reduce_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, stream, p.job.part, p.job.y, total,
+                           p.job.ksplit);
+    }
     return hipGetLastError();
 }
 
@@ -900,7 +931,7 @@ static void mm_classes(const MatView *mats, const uint32_t *tokens, const float 
     }
 }
 
-size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_t n) {
+size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_t n, bool least) {
     size_t need = 0;
     for (uint32_t g = 0; g < n;) {
         if (tokens[g] == 0 || mats[g].rows == 0) { g++; continue; }
@@ -908,7 +939,7 @@ size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_
         if (run == 0) {
             if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
                 size_t bytes;
-                if (pg_takes(mats[g], tokens[g])) {
+                if (pg_takes(mats[g], tokens[g]) && !least) {
                     PgPlan p;
                     pg_plan(mats[g], tokens[g], p);
                     bytes = p.x_bytes + p.part_bytes;

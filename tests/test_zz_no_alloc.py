@@ -98,7 +98,7 @@ def test_noalloc_plain_dtypes_with_shared_columns(gpu, hip, ty):
 @pytest.mark.parametrize("tokens", [801, 1700])
 def test_noalloc_plain_dtype_whose_cut_activations_exceed_the_workspace(gpu, hip, tokens):
     """The three bf16 parts of 801 x 14336 activations alone are 74 MB: the call goes out in pieces.  Against the
-    allocating call, whose sums may be shared differently: twice the bound of either."""
+    allocating call, twice the bound of either (the same bits: the next test)."""
     rng = np.random.default_rng(tokens)
     rows, cols = 40, 14336
     w = K.random_packed(K.F16, rows, cols, rng)
@@ -116,6 +116,38 @@ def test_noalloc_plain_dtype_whose_cut_activations_exceed_the_workspace(gpu, hip
     mag = K.abs_product(K.F16, rows, cols, w, x).ravel()
     assert np.all(np.abs(got.astype(np.float64) - ref) <= 2 * K.single_kernel_bound(cols, mag))
     m.close(); xd.free(); yd.free()
+
+
+@pytest.mark.parametrize("ty,rows,cols,tokens", [(K.F32, 4096, 4096, 1537), (K.F16, 14336, 4096, 3073), (K.F32, 300, 14336, 2100),
+                                                 (K.F16, 9, 131072, 200), (K.F32, 3, 400004, 40)])
+def test_noalloc_plain_dtype_in_pieces_of_one_plan(gpu, hip, ty, rows, cols, tokens):
+    """Every piece of a product that goes out in pieces fits: the last, smaller one shares its columns as the others do and
+    not as a product of its size would (768 of 1537 tokens by 4096x4096 would take 66 MB, 1536 of 3073 by 14336x4096
+    204 MB).  The sums are then those of lnh_gemm_device, bit for bit; a few rows and tokens against float64.  Rows so long
+    that narrower tiles than the plan's have to do, and so long that none fits (which leaves the f32 instruction)."""
+    rng = np.random.default_rng(tokens)
+    w = K.random_packed(ty, rows, cols, rng)
+    x = rng.standard_normal((tokens, cols), np.float32)
+    m = gpu.upload_packed(ty, rows, cols, w)
+    xd = hip.DeviceBuffer.from_numpy(x.ravel())
+    ya, yb = hip.DeviceBuffer(tokens * rows * 4), hip.DeviceBuffer(tokens * rows * 4)
+    ya.fill_byte(0xff)
+    hip.device_synchronize()
+    gpu.gemm_device_noalloc(m, tokens, xd.ptr, ya.ptr)
+    gpu.gemm_device(m, tokens, xd.ptr, yb.ptr)
+    gpu.synchronize()
+    a, b = ya.to_numpy(np.float32).reshape(tokens, rows), yb.to_numpy(np.float32).reshape(tokens, rows)
+    for buf in (xd, ya, yb):
+        buf.free()
+    m.close()
+    if cols < 400000:
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    rs, ts = sorted({0, min(127, rows - 1), min(128, rows - 1), rows - 1}), sorted({t for t in (0, 31, 32, 640, 767, 768, 769, tokens - 1) if t < tokens})
+    rb = K.row_bytes(ty, cols)
+    exact, mag = O.gemm_f64_mag(ty, cols, len(ts), np.concatenate([w[r * rb:(r + 1) * rb] for r in rs]), x[ts].ravel(), len(rs))
+    exact, bound = exact.reshape(len(ts), -1), K.single_kernel_bound(cols, mag.reshape(len(ts), -1))
+    for y in (a, b):
+        assert np.all(np.abs(y[np.ix_(ts, rs)] - exact) <= bound)
 
 
 @pytest.mark.parametrize("ty,tokens", [(K.Q4_K, 24), (K.Q5_1, 7), (K.Q8_0, 70), (K.F16, 5)])
