@@ -142,7 +142,11 @@ int lnh_gemm_shared(lnh_exec *exec, size_t n_mats, const lnh_matrix *const *mats
  * LNH_ERR_INVALID before anything is launched - run the largest shape once
  * before capturing; a workspace that captured launches point at stays
  * allocated until the executor is destroyed, also after a later call has
- * made the executor move to a larger one).  Calls of one executor must therefore be enqueued on
+ * made the executor move to a larger one).  So do products of several tokens by an F32 / F16 matrix: always where the
+ * matrix has so few rows that its columns are shared between workgroups, and, where there are more than 32 tokens
+ * (F16: 16), 6 bytes per activation value, up to 1 GB.  Without the latter (the stream is being captured, or the
+ * memory is not to be had) they run in pieces of fewer tokens or on a slower kernel, whose sums are in another order.
+ * Calls of one executor must therefore be enqueued on
  * one stream at a time; calls that overlap on different streams race on it.
  * Every device buffer a call reads (device_x, device_x2, device_residual, device_norm_w; in this and the following
  * sections) must be 16-byte aligned, as anything hipMalloc returns is: LNH_ERR_INVALID otherwise. */
@@ -157,7 +161,7 @@ int lnh_gemm_grouped_device(lnh_exec *exec, size_t n_groups, const lnh_matrix *c
  * that GPU until the process ends) instead of the executor's grow-on-demand allocation: the call
  * never allocates or frees.  A product by a quantized matrix that needs more fails with LNH_ERR_INVALID
  * (the message states the need) before anything is launched; one by an F32 / F16 matrix goes out in pieces of
- * fewer tokens instead, with the same sums (rows of some 270000 columns and more take another kernel, whose sums
+ * fewer tokens instead, with the same sums (rows of some 150000 columns and more take another kernel, whose sums
  * are taken in another order).  Refused likewise is a product of three or more tokens by a
  * quantized matrix whose multi-token layout has not been made yet (lnh_matrix_prepare, or any earlier such product
  * through an allocating entry point, makes it).  Every call on one GPU, from any executor, uses the

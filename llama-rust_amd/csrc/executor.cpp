@@ -168,25 +168,30 @@ bool ensure_pinned(lnh_exec *e, size_t in_floats, size_t out_floats) {
 // goes: a caller may have captured launches that point at it into a HIP graph (a decode step that is replayed
 // while another call, a longer prompt say, makes the workspace grow), and work already queued may still use
 // it.  Growth is by at least half, so everything retired together is smaller than twice the live buffer.
-int ensure_workspace(lnh_exec *e, hipStream_t s, size_t bytes) {
+// `least`: what the call can do with (more slowly) where `bytes` cannot be had.
+int ensure_workspace(lnh_exec *e, hipStream_t s, size_t bytes, size_t least) {
     if (bytes <= e->ws_cap) return LNH_OK;
     // Growing allocates, which a stream under capture cannot record: refuse before anything is launched
     // instead of leaving the caller with a broken capture.
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (s && hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing != hipStreamCaptureStatusNone)
+    if (s && hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing != hipStreamCaptureStatusNone) {
+        if (least <= e->ws_cap) return LNH_OK;
         return fail(e, LNH_ERR_INVALID,
                     "the multi-token workspace must grow to " + std::to_string(bytes) +
                         " bytes while the stream is being captured: run the largest product once before capturing, "
                         "or use lnh_gemm_device_noalloc");
+    }
     (void)hipGetLastError();
-    size_t want = bytes > e->ws_cap + e->ws_cap / 2 ? bytes : e->ws_cap + e->ws_cap / 2;
-    want += want / 4;
+    const size_t grown = bytes > e->ws_cap + e->ws_cap / 2 ? bytes : e->ws_cap + e->ws_cap / 2;
+    const size_t sizes[3] = {grown + grown / 4, bytes, least};
     void *fresh = nullptr;
-    hipError_t h = hipMalloc(&fresh, want);
-    if (h != hipSuccess) {
-        (void)hipGetLastError();
-        want = bytes;
+    size_t want = 0;
+    hipError_t h = hipErrorOutOfMemory;
+    for (int i = 0; i < 3 && h != hipSuccess; i++) {
+        want = sizes[i];
+        if (want <= e->ws_cap) return LNH_OK;
         h = hipMalloc(&fresh, want);
+        if (h != hipSuccess) (void)hipGetLastError();
     }
     if (h != hipSuccess) return hip_fail(e, h, "HIP workspace allocation");
     if (e->d_ws) e->ws_retired.push_back(e->d_ws);
@@ -257,7 +262,8 @@ int launch_products(lnh_exec *e, hipStream_t s, size_t n, const lnh_matrix *cons
             if (rt != LNH_OK) return rt;
         }
     }
-    int rc = ensure_workspace(e, s, nh::gemm_workspace_bytes(views.data(), toks.data(), (uint32_t)n));
+    int rc = ensure_workspace(e, s, nh::gemm_workspace_bytes(views.data(), toks.data(), (uint32_t)n),
+                              nh::gemm_workspace_bytes(views.data(), toks.data(), (uint32_t)n, true));
     if (rc != LNH_OK) return rc;
     hipError_t h = nh::launch_gemm_groups(s, views.data(), tiled.data(), toks.data(), xs, ys, (uint32_t)n, e->d_ws, e->ws_cap);
     if (h != hipSuccess) return hip_fail(e, h, "HIP kernel launch");
@@ -873,8 +879,8 @@ int gemm_act(lnh_exec *e, size_t n_mats, const lnh_matrix *const *mats, const ln
         const int rt = ensure_tiled(e, s, mats[i], &tiled[i]);
         if (rt != LNH_OK) return rt;
     }
-    int rc = ensure_workspace(e, s, nh::gemm_act_workspace_bytes(tiled, (uint32_t)n_mats, (uint32_t)tokens,
-                                                                 ep.kind != nh::ACT_EPILOGUE_NONE, plain));
+    const size_t ws_bytes = nh::gemm_act_workspace_bytes(tiled, (uint32_t)n_mats, (uint32_t)tokens, ep.kind != nh::ACT_EPILOGUE_NONE, plain);
+    int rc = ensure_workspace(e, s, ws_bytes, ws_bytes);
     if (rc != LNH_OK) return rc;
     const hipError_t h = nh::launch_gemm_act(s, tiled, (uint32_t)n_mats, (uint32_t)tokens, plain ? nullptr : x->dev,
                                              plain ? 0 : x->max_tokens, dx, norm.w ? &norm : nullptr, dys, ep, e->d_ws, e->ws_cap);

@@ -27,10 +27,10 @@ hipError_t launch_retile(hipStream_t stream, const MatView &tiled, const MatView
 // Products of three or more tokens by a quantized matrix run on the matrix cores (two tokens: two
 // single-token launches),
 // read the tiled copy of the matrix and need device workspace: ws must hold gemm_workspace_bytes() for the same
-// arguments (hipErrorInvalidValue otherwise).  The workspace is only used by
+// arguments, at the least (hipErrorInvalidValue otherwise).  The workspace is only used by
 // work queued on `stream`, so calls on one stream may share it.
 // Products of F32 / F16 weights cut the activations of many tokens into the workspace; given less than that takes they
-// go out in pieces of fewer tokens.  least: what a call cannot do without.
+// go out in pieces of fewer tokens or on a kernel that cuts nothing.  least: what a call cannot do without.
 size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_t n, bool least = false);
 hipError_t launch_gemm(hipStream_t stream, const MatView &m, const MatView &tiled, uint32_t tokens, const float *x,
                        float *y, void *ws, size_t ws_bytes);

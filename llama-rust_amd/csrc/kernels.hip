@@ -689,7 +689,8 @@ static hipError_t launch_mm(hipStream_t stream, MmPlan &p, void *ws, size_t ws_b
     }
 }
 
-// F32 / F16 weights, up to 32 tokens: gemm_fmfma_kernel (+ fg_reduce_kernel when columns are shared).
+// F32 / F16 weights, up to 32 tokens, and more where there is no workspace to cut the activations into:
+// gemm_fmfma_kernel (+ fg_reduce_kernel when columns are shared).
 struct FgPlan {
     FgJob job;
     int tt;
@@ -697,8 +698,8 @@ struct FgPlan {
     size_t part_bytes;
 };
 static void fg_plan(const MatView &m, uint32_t tokens, FgPlan &p) {
-    p.tt = tokens > 16 ? 1 : 0;   // 0: a 16-token tile
-    const uint32_t tile_tok = p.tt == 0 ? 16u : 32u;
+    p.tt = tokens > 32 ? 2 : tokens > 16 ? 1 : 0;   // 0: a 16-token tile
+    const uint32_t tile_tok = p.tt == 0 ? 16u : 32u * (uint32_t)p.tt;
     const uint32_t tok_tiles = (tokens + tile_tok - 1) / tile_tok, row_tiles = (m.rows + FG_ROWS - 1) / FG_ROWS;
     const uint32_t tiles = tok_tiles * row_tiles, n_steps = (m.cols + FG_K - 1) / FG_K;
     // about two workgroups per CU (16-token tiles measured at 1 / 2 / 3 / 4 per CU: F16 4096x14336, 8 tokens, 51 / 40 / 40 / 44 us)
@@ -742,9 +743,9 @@ static hipError_t launch_fg(hipStream_t stream, const MatView &m, uint32_t token
     p.job.part = static_cast<float *>(ws);
     hipError_t e;
     if (m.type == T_F16)
-        e = p.tt == 1 ? launch_fg_main<T_F16, 1>(stream, p) : launch_fg_main<T_F16, 0>(stream, p);
+        e = p.tt == 2 ? launch_fg_main<T_F16, 2>(stream, p) : p.tt == 1 ? launch_fg_main<T_F16, 1>(stream, p) : launch_fg_main<T_F16, 0>(stream, p);
     else
-        e = p.tt == 1 ? launch_fg_main<T_F32, 1>(stream, p) : launch_fg_main<T_F32, 0>(stream, p);
+        e = p.tt == 2 ? launch_fg_main<T_F32, 2>(stream, p) : p.tt == 1 ? launch_fg_main<T_F32, 1>(stream, p) : launch_fg_main<T_F32, 0>(stream, p);
     if (e != hipSuccess || p.job.ksplit < 2) return e;
     const size_t total = (size_t)tokens * m.rows, vec = (total + 3) / 4, blocks = (vec + 255) / 256;
     hipLaunchKernelGGL(fg_reduce_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, stream, p.job.part, y, total,
@@ -812,20 +813,31 @@ static void pg_plan(const MatView &m, uint32_t tokens, PgPlan &p) {
     pg_fit(m, tokens, tok, ks, p);
 }
 
+// The most workspace such a product asks for: cut activations take 6 bytes a value, held as long as the executor lives,
+// where the f32 instruction takes none.  Pieces of this size cost nothing (16384 tokens by 4096x14336, 1.4 GB whole:
+// F16 10.2 -> 9.2 ms in two pieces, F32 14.0 -> 13.4), of a quarter of it 7-10 % (8192 tokens in three pieces: F16 4.84 ->
+// 5.31 ms, F32 6.99 -> 7.45), the last round of workgroups of each piece being partly empty.
+constexpr size_t PG_WS_BYTES = (size_t)1 << 30;
+
 // Tokens per piece of a product that is given less workspace than its plan takes: pieces of whole tiles, as equal as
 // they come, all with the plan's column shares.  The shares alone decide in which order a sum is taken, so every token's
 // results are those of the whole product bit for bit, and a piece of fewer tokens takes less (a plan of its own would
-// share its columns more finely and could take more).  Narrower tiles where not even one fits; 0: none does.
+// share its columns more finely and could take more).  Narrower tiles where not even one fits.  0: pieces would have
+// fewer than 64 tokens, and reading the weights that often costs more than the f32 instruction does (F16 4096x14336:
+// 51 us per 32 tokens, 55 per 64; the f32 instruction 78 per 64 of 128).
 static uint32_t pg_piece(PgPlan &p, size_t ws_bytes) {
     const PgJob &j = p.job;
+    if (ws_bytes > PG_WS_BYTES) ws_bytes = PG_WS_BYTES;
     if (p.x_bytes + p.part_bytes <= ws_bytes) return j.tokens;
     const size_t column = (size_t)j.n_steps * 12 * sizeof(uint4), fixed = 8 * column + 512;  // 512: both parts are rounded up
     for (uint32_t tok = p.tok; tok >= 32; tok /= 2) {
         const size_t tile = tok * (column + (j.ksplit > 1 ? (size_t)j.ksplit * j.m.rows * sizeof(float) : 0));
         if (fixed + tile > ws_bytes) continue;
         const size_t tiles = ((size_t)j.tokens + tok - 1) / tok, most = (ws_bytes - fixed) / tile, pieces = (tiles + most - 1) / most;
+        const uint32_t piece = (uint32_t)((tiles + pieces - 1) / pieces) * tok;
+        if (piece < 64) return 0;
         p.tok = tok;
-        return (uint32_t)((tiles + pieces - 1) / pieces) * tok;
+        return piece;
     }
     return 0;
 }
@@ -848,7 +860,7 @@ static hipError_t launch_pg(hipStream_t stream, const MatView &m, uint32_t token
     PgPlan plan;
     pg_plan(m, tokens, plan);
     const uint32_t piece = pg_piece(plan, ws_bytes);
-    if (piece == 0) return launch_fg(stream, m, tokens, x, y, ws, ws_bytes);  // rows so long that 32 tokens of them do not fit
+    if (piece == 0) return launch_fg(stream, m, tokens, x, y, ws, ws_bytes);
     for (uint32_t t = 0, n; t < tokens; t += n) {
         n = tokens - t < piece ? tokens - t : piece;
         PgPlan p;
@@ -939,14 +951,15 @@ size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_
         if (run == 0) {
             if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
                 size_t bytes;
+                FgPlan f;
+                fg_plan(mats[g], tokens[g], f);
+                bytes = f.part_bytes;
                 if (pg_takes(mats[g], tokens[g]) && !least) {
                     PgPlan p;
                     pg_plan(mats[g], tokens[g], p);
-                    bytes = p.x_bytes + p.part_bytes;
-                } else {
-                    FgPlan p;
-                    fg_plan(mats[g], tokens[g], p);
-                    bytes = p.part_bytes;
+                    const size_t want = p.x_bytes + p.part_bytes;
+                    // f.part_bytes also then: pg_piece may find that not even a tile fits
+                    bytes = want <= PG_WS_BYTES ? want : PG_WS_BYTES > bytes ? PG_WS_BYTES : bytes;
                 }
                 need = bytes > need ? bytes : need;
             }

@@ -331,6 +331,45 @@ def test_workspace_growth_under_stream_capture_is_refused_not_recorded(pkg):
     g.close()
 
 
+@pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,tokens,before", [(300, 256, 40, 0), (5000, 1032, 420, 0), (5000, 1032, 420, 130), (5000, 1032, 420, 33)])
+def test_plain_dtype_captured_without_its_workspace(pkg, ty, rows, cols, tokens, before):
+    """F16 / F32 products whose columns are not shared can be recorded into a graph by an executor that has run nothing yet
+    or only a product of fewer tokens: the plan that cuts the activations into a workspace gives way to pieces that fit,
+    or to the kernel that needs none.  Replayed with new inputs and the program's own eager work in between, each replay
+    within the bound of the eager result."""
+    hip = importlib.import_module("llama-rust_amd.hiprt")
+    g = pkg.HipGemv(0)
+    rng = np.random.default_rng(rows)
+    w = K.random_packed(ty, rows, cols, rng)
+    m = g.upload_packed(ty, rows, cols, w)
+    xd = hip.DeviceBuffer(tokens * cols * 4)
+    ya, yb = hip.DeviceBuffer(tokens * rows * 4), hip.DeviceBuffer(tokens * rows * 4)
+    stream = hip.Stream()
+    if before:
+        g.gemm_device(m, before, xd.ptr, yb.ptr)
+        g.synchronize()
+    graph = hip.Graph(stream, lambda s: g.gemm_device(m, tokens, xd.ptr, ya.ptr, s.ptr))
+    for replay in range(3):
+        x = rng.normal(0, 1, tokens * cols).astype(np.float32)
+        xd.upload(x)
+        ya.fill_byte(0xff)
+        hip.device_synchronize()
+        graph.launch()
+        stream.synchronize()
+        g.gemm_device(m, tokens, xd.ptr, yb.ptr)   # eager: from now on the executor has the workspace
+        g.synchronize()
+        exact, mag = O.gemm_f64_mag(ty, cols, tokens, w, x, rows)
+        bound = K.single_kernel_bound(cols, mag).reshape(tokens, rows)
+        for y in (ya, yb):
+            assert np.all(np.abs(y.to_numpy(np.float32).reshape(tokens, rows) - exact.reshape(tokens, rows)) <= bound), f"replay {replay}"
+    graph.destroy()
+    for b in (xd, ya, yb):
+        b.free()
+    m.close()
+    g.close()
+
+
 def test_q4k_matrix_beyond_32_bit_plane_offsets_is_refused(pkg, gpu):
     """The Q4_K single-token kernel addresses a plane with 32-bit byte offsets: an upload whose code plane
     would reach 4 GiB is refused by shape, before any byte of it is read (the buffer here is a stub)."""
