@@ -15,6 +15,7 @@
 
 #include "../../include/native_hip.h"
 #include "early_gemm.h"
+#include "host_range.h"
 #include "kernels.h"
 
 static_assert(LNH_NOALLOC_WORKSPACE_BYTES == nh::STATIC_SCRATCH_BYTES, "header and device array disagree");
@@ -352,17 +353,24 @@ int check_gemm(lnh_exec *e, const lnh_matrix *m, size_t tokens, bool have_lens, 
     return LNH_OK;
 }
 
-// Whether a kernel of this device can read or write the caller's buffer in place: pinned memory, whole aligned 16-byte
-// vectors.  Asked for buffers where a staging copy costs more than the question.
+// Whether a kernel of this device can read or write the caller's buffer in place: whole aligned 16-byte vectors in one
+// pinned mapping.  Asked (1 us) for buffers where a staging copy costs more than the question.
 constexpr size_t IN_PLACE_MIN_FLOATS = 16384;
 float *in_place(const float *p, size_t floats) {
     if (floats < IN_PLACE_MIN_FLOATS || floats % 4 != 0 || misaligned(p)) return nullptr;
-    hipPointerAttribute_t at;
-    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
-        (void)hipGetLastError();  // an ordinary pointer
-        return nullptr;
-    }
-    return at.type == hipMemoryTypeHost && !misaligned(at.devicePointer) ? static_cast<float *>(at.devicePointer) : nullptr;
+    void *const there = nh::device_view(p, floats * sizeof(float), [](const void *host, nh::HostMapping *m) {
+        hipPointerAttribute_t at;
+        hipDeviceptr_t base = nullptr;
+        if (hipPointerGetAttributes(&at, host) != hipSuccess || at.type != hipMemoryTypeHost || !at.devicePointer ||
+            hipMemGetAddressRange(&base, &m->size, at.devicePointer) != hipSuccess) {
+            (void)hipGetLastError();  // an ordinary pointer
+            return false;
+        }
+        m->device = at.devicePointer;
+        m->base = base;
+        return true;
+    });
+    return misaligned(there) ? nullptr : static_cast<float *>(there);
 }
 
 void copy_floats(lnh_exec *e, float *dst, const float *src, size_t n) {

@@ -178,3 +178,17 @@ def test_cpp_mirror_header_compiles_against_the_c_abi(pkg, tmp_path):
     subprocess.run([cxx, "-std=c++17", "-Wall", "-Wextra", "-Werror", pkg.SELFTEST_SRC, "-o", str(out), "-L" + pkg.HERE,
                     "-lnative_hip"], check=True)
     assert out.exists()
+
+
+def test_host_only_parts(tmp_path):
+    """Header parts of the library that need no device (tests/cpp/host_parts.cpp), built by the host compiler alone."""
+    import os
+    import shutil
+    import subprocess
+    cxx = shutil.which(os.environ.get("CXX", "g++"))
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    src, out = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "host_parts.cpp"), tmp_path / "host_parts"
+    subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Wextra", "-Werror", "-pthread", src, "-o", str(out)], check=True)
+    r = subprocess.run([str(out)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "OK", r.stdout + r.stderr
