@@ -7,7 +7,9 @@
 //   - items are handed out one by one from a single word that also holds the call's number and item count, and run()
 //     returns when every item is done, not when every worker has woken up: a late worker finds the word spent and
 //     goes back to sleep.
-// A pool belongs to one object and is driven by one thread at a time; it ends with its owner.
+// A pool belongs to one object and is driven by one thread at a time; it ends with its owner.  All pools of a process
+// together have a bounded number of workers: a pool that finds fewer left, or whose threads the system refuses, has as
+// many as it got, down to none (the calling thread then does all the work).
 #ifndef NATIVE_HIP_HOST_POOL_H
 #define NATIVE_HIP_HOST_POOL_H
 
@@ -20,6 +22,7 @@
 #include <climits>
 #include <cstddef>
 #include <cstdint>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -33,8 +36,22 @@ class HostPool {
         const unsigned hw = std::thread::hardware_concurrency();
         return hw < 2 ? 1 : (hw > 16 ? 16 : hw);
     }
-    explicit HostPool(size_t workers = default_threads() - 1) {
-        for (size_t i = 0; i < workers; i++) threads_.emplace_back([this] { loop(); });
+    // Workers of all pools together: four whole pools.  A program that calls from more threads than that keeps its
+    // processors busy without them.
+    static size_t most_workers() { return 4 * (default_threads() - 1); }
+    // Never throws: this is reached from C entry points, and a thread that cannot be made is no failure of the call.
+    explicit HostPool(size_t workers = default_threads() - 1) noexcept {
+        size_t used = live().load(std::memory_order_relaxed), want;
+        do {
+            const size_t left = most_workers() > used ? most_workers() - used : 0;
+            want = workers < left ? workers : left;
+        } while (!live().compare_exchange_weak(used, used + want, std::memory_order_relaxed));
+        try {
+            threads_.reserve(want);
+            while (threads_.size() < want) threads_.emplace_back([this] { loop(); });
+        } catch (const std::exception &) {  // the system's limit on threads or memory: those made so far do
+        }
+        live().fetch_sub(want - threads_.size(), std::memory_order_relaxed);
     }
     HostPool(const HostPool &) = delete;
     HostPool &operator=(const HostPool &) = delete;
@@ -42,6 +59,7 @@ class HostPool {
         stop_.store(true, std::memory_order_relaxed);
         ring(INT_MAX);
         for (auto &t : threads_) t.join();
+        live().fetch_sub(threads_.size(), std::memory_order_relaxed);
     }
     size_t threads() const { return threads_.size() + 1; }
 
@@ -63,6 +81,11 @@ class HostPool {
     }
 
   private:
+    static std::atomic<size_t> &live() {
+        static std::atomic<size_t> count{0};
+        return count;
+    }
+
     static constexpr size_t MAX_ITEMS = (1u << 20) - 1;
     static constexpr int SPIN_US = 60;  // about the time a product call of a host session keeps its caller away
 

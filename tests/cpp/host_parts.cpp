@@ -1,7 +1,16 @@
 // Checks of the library's host-only parts (llama-rust_amd/csrc/*.h that need no device), for the host compiler alone.
 // Prints "OK" and returns 0, or says what failed and returns 1.
-#include <cstdio>
+#include <sys/resource.h>
+#include <sys/wait.h>
+#include <unistd.h>
 
+#include <atomic>
+#include <cstdio>
+#include <memory>
+#include <thread>
+#include <vector>
+
+#include "../../llama-rust_amd/csrc/host_pool.h"
 #include "../../llama-rust_amd/csrc/host_range.h"
 
 static int failures = 0;
@@ -36,8 +45,96 @@ static void host_range() {
     CHECK(nh::device_view(host + 4096, 16, [](const void *, nh::HostMapping *) { return true; }) == nullptr);
 }
 
+// Every item exactly once, seen by the caller afterwards, over calls of changing size that follow each other closely or
+// after the workers have gone to sleep.
+static void pool_items(nh::HostPool &pool) {
+    std::vector<int> seen;
+    const size_t sizes[] = {0, 1, 2, 3, 15, 16, 17, 64, 1000, 5, 2, 40000};
+    for (int round = 0; round < 300; round++) {
+        const size_t n = sizes[(size_t)round % 12];
+        seen.assign(n, 0);
+        pool.run(n, [&](size_t i) { seen[i]++; });
+        size_t wrong = 0;
+        for (size_t i = 0; i < n; i++) wrong += seen[i] != 1;
+        CHECK(wrong == 0);
+        if (round % 50 == 49) usleep(2000);
+    }
+    for (size_t n : {1, 7, 96, 97, 1000, 100003})
+        for (size_t grain : {1, 10, 96, 200000}) {
+            seen.assign(n, 0);
+            std::atomic<size_t> pieces{0};
+            pool.run_ranges(n, grain, [&](size_t begin, size_t end) {
+                for (size_t i = begin; i < end; i++) seen[i]++;
+                pieces++;
+            });
+            size_t wrong = 0;
+            for (size_t i = 0; i < n; i++) wrong += seen[i] != 1;
+            CHECK(wrong == 0);
+            CHECK(pieces >= 1 && pieces <= 4 * pool.threads() && pieces <= (n + grain - 1) / grain);
+        }
+    size_t calls = 0;
+    pool.run_ranges(0, 16, [&](size_t, size_t) { calls++; });
+    CHECK(calls == 0);
+    std::atomic<uint64_t> sum{0};  // more items than one word of the pool counts
+    const size_t many = (1u << 20) + 5;
+    pool.run(many, [&](size_t i) { sum.fetch_add(i, std::memory_order_relaxed); });
+    CHECK(sum == (uint64_t)many * (many - 1) / 2);
+}
+
+static void pools() {
+    {
+        nh::HostPool pool(3), none(0);
+        CHECK(none.threads() == 1);
+        pool_items(pool);
+        pool_items(none);
+    }
+    // pools of several threads at once, more of them than there are workers for
+    std::vector<std::unique_ptr<nh::HostPool>> held;
+    size_t workers = 0;
+    for (int i = 0; i < 9; i++) {
+        held.push_back(std::make_unique<nh::HostPool>(nh::HostPool::most_workers() / 4 + 1));
+        workers += held.back()->threads() - 1;
+    }
+    CHECK(workers == nh::HostPool::most_workers());
+    std::vector<std::thread> callers;
+    for (auto &p : held) callers.emplace_back([&p] { pool_items(*p); });
+    for (auto &t : callers) t.join();
+    held.clear();
+    nh::HostPool again(nh::HostPool::most_workers());  // given back
+    CHECK(again.threads() == nh::HostPool::most_workers() + 1);
+}
+
+// A pool in a process that may have few or no further threads: no exception, no end of the process.
+static void pool_without_threads() {
+    const pid_t child = fork();
+    if (child == 0) {
+        long pages = 0;
+        if (std::FILE *f = std::fopen("/proc/self/statm", "r")) {
+            if (std::fscanf(f, "%ld", &pages) != 1) pages = 0;
+            std::fclose(f);
+        }
+        const rlim_t limit = (rlim_t)pages * (rlim_t)sysconf(_SC_PAGESIZE) + (20u << 20);  // a few stacks, not sixteen
+        const rlimit r = {limit, limit};
+        if (pages == 0 || setrlimit(RLIMIT_AS, &r) != 0) _exit(2);
+        {
+            nh::HostPool pool(16);
+            if (pool.threads() > 16) _exit(3);
+            size_t seen[64] = {};
+            pool.run(64, [&](size_t i) { seen[i]++; });
+            for (size_t s : seen)
+                if (s != 1) _exit(4);
+        }
+        _exit(0);
+    }
+    int status = -1;
+    CHECK(child > 0 && waitpid(child, &status, 0) == child);
+    CHECK(WIFEXITED(status) && WEXITSTATUS(status) == 0);
+}
+
 int main() {
     host_range();
+    pool_without_threads();  // first: a forked child has only the thread that forked
+    pools();
     if (failures == 0) std::printf("OK\n");
     return failures != 0;
 }
