@@ -16,6 +16,7 @@
 #include <cstring>
 #include <type_traits>
 
+#include "device_once.h"
 #include "kernels.h"
 
 namespace nh {
@@ -27,6 +28,14 @@ namespace nh {
 #include "plain_gemm.inc"
 
 // ------------------------------------------------------------------ launchers
+
+// Lifts a kernel's limit on dynamic LDS on the current GPU to `bytes`, the first time it is launched there.
+static hipError_t allow_lds(DeviceOnce &once, const void *kernel, size_t bytes) {
+    int device = -1;
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    return once.run(device, [&] { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes); });
+}
 
 static bool g_nibble_bf16 = false;  // the packed fp8 -> bf16 convert turns nibble bytes into the integers 0..15
 static bool g_nibble_i4 = false;    // the signed 4-bit convert with a byte select gives (n - 8) / 16 for nibble n ^ 8
@@ -568,12 +577,10 @@ static hipError_t launch_mm_main(hipStream_t stream, const MmBatch &b) {
     }
     constexpr size_t lds = 2 * MmStage<T, TT>::BYTES;  // two pipeline stages
     auto kern = gemm_mfma_kernel<T, TT, VQ, FB, INLINE, NORM>;
-    static bool configured = false;
-    if (lds > 48 * 1024 && !configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)lds);
+    if constexpr (lds > 48 * 1024) {
+        static DeviceOnce limit;
+        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
         if (e != hipSuccess) return e;
-        configured = true;
     }
     hipLaunchKernelGGL(kern, dim3(b.total_wgs), dim3(256), lds, stream, b);
     return hipGetLastError();
@@ -723,11 +730,10 @@ template <uint32_t T, int TT>
 static hipError_t launch_fg_main(hipStream_t stream, const FgPlan &p) {
     constexpr size_t lds = (size_t)2 * (FG_ROWS + (TT == 0 ? 16 : 32 * TT)) * FG_LD * sizeof(float);
     auto kern = gemm_fmfma_kernel<T, TT>;
-    static bool configured = false;
-    if (lds > 48 * 1024 && !configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if constexpr (lds > 48 * 1024) {
+        static DeviceOnce limit;
+        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
         if (e != hipSuccess) return e;
-        configured = true;
     }
     hipLaunchKernelGGL(kern, dim3(p.wgs), dim3(256), lds, stream, p.job);
     return hipGetLastError();
@@ -846,11 +852,10 @@ template <uint32_t T, int TOK>
 static hipError_t launch_pg_main(hipStream_t stream, const PgPlan &p) {
     constexpr size_t lds = 2 * PgTraits<T, TOK>::STAGE;
     auto kern = gemm_plain_kernel<T, TOK>;
-    static bool configured = false;
-    if (lds > 48 * 1024 && !configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if constexpr (lds > 48 * 1024) {
+        static DeviceOnce limit;
+        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
         if (e != hipSuccess) return e;
-        configured = true;
     }
     hipLaunchKernelGGL(kern, dim3(p.wgs), dim3(256), lds, stream, p.job);
     return hipGetLastError();

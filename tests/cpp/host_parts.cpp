@@ -10,6 +10,7 @@
 #include <thread>
 #include <vector>
 
+#include "../../llama-rust_amd/csrc/device_once.h"
 #include "../../llama-rust_amd/csrc/host_pool.h"
 #include "../../llama-rust_amd/csrc/host_range.h"
 
@@ -131,9 +132,37 @@ static void pool_without_threads() {
     CHECK(WIFEXITED(status) && WEXITSTATUS(status) == 0);
 }
 
+// Once for every device, again after a failure, and never skipped by a thread for which it has not been done.
+static void device_once() {
+    nh::DeviceOnce once;
+    int calls = 0;
+    auto works = [&] { return ++calls, 0; };
+    auto fails = [&] { return ++calls, 7; };
+    CHECK(once.run(0, fails) == 7 && once.run(0, works) == 0 && calls == 2);
+    CHECK(once.run(0, fails) == 0 && calls == 2);
+    CHECK(once.run(3, fails) == 7 && once.run(3, works) == 0 && once.run(63, works) == 0 && calls == 5);
+    CHECK(once.run(3, works) == 0 && once.run(0, works) == 0 && once.run(63, works) == 0 && calls == 5);
+    CHECK(once.run(64, works) == 0 && once.run(64, works) == 0 && once.run(-1, works) == 0 && calls == 8);  // not remembered
+    for (int round = 0; round < 200; round++) {
+        nh::DeviceOnce shared;
+        int set[4] = {0, 0, 0, 0};  // not atomic: the flag is what orders it for the threads that skip
+        std::atomic<int> missing{0}, first{0};
+        std::vector<std::thread> threads;
+        for (int t = 0; t < 4; t++)
+            threads.emplace_back([&, t] {
+                const int d = t % 2;
+                shared.run(d, [&] { return first.fetch_add(1), set[2 * d + t / 2] = 1, 0; });
+                if (shared.run(d, [] { return 1; }) != 0) missing++;
+            });
+        for (auto &t : threads) t.join();
+        CHECK(missing == 0 && first >= 2 && first <= 4 && set[0] + set[1] >= 1 && set[2] + set[3] >= 1);
+    }
+}
+
 int main() {
-    host_range();
     pool_without_threads();  // first: a forked child has only the thread that forked
+    host_range();
+    device_once();
     pools();
     if (failures == 0) std::printf("OK\n");
     return failures != 0;
