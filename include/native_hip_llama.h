@@ -86,9 +86,9 @@ int lnm_session_new_device(lnm_model *model, size_t kv_block, const uint32_t *bl
 int lnm_session_new_device_batch(lnm_model *model, size_t kv_block, size_t n_sequences, size_t max_positions,
                                  lnm_session **out);
 /* Greedy decode of all sequences from scratch: `prompts` holds the prompts one after the other, prompt_lens[b]
- * tokens for sequence b (at least 1); out[b * n_new + i] is token i of sequence b.  Prompts run one sequence
- * after the other (all tokens but the last, in chunks of up to 512 that several prompts may share, K and V only), then n_new steps of all
- * sequences together, step 0 taking every prompt's last token. */
+ * tokens for sequence b (at least 1); out[b * n_new + i] is token i of sequence b.  The prompts (all tokens but the
+ * last of each, K and V only) run as one series of tokens in chunks of up to 512, each of which may end one prompt and
+ * hold others; then n_new steps of all sequences together, step 0 taking every prompt's last token. */
 int lnm_batch_generate_greedy(lnm_session *session, const uint32_t *prompts, const size_t *prompt_lens, size_t n_new,
                               uint32_t *out, double *prefill_seconds, double *decode_seconds);
 void lnm_session_free(lnm_session *session);

@@ -499,12 +499,15 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     const uint32_t n_steps = mats[0].cols / 32;
     // Columns are shared between workgroups as far as that shortens the launch: every share costs a partial
     // result written and read back.  A CU holds two workgroups of these kernels, and one alone already gets 0.63-0.7
-    // of what the two get together (measured on the 16-token kernel: a step of 0.48 us alone, 0.76 us each
-    // together), so what counts is how evenly the steps fall on the CUs.  The launch is priced in steps of a
+    // of what the two get together, so what counts is how evenly the steps fall on the CUs.  The launch is priced in steps of a
     // workgroup that shares its CU: whole rounds of 2 x CUs workgroups, then the rest (alone on their CUs if they
     // are at most one per CU), two more steps per workgroup for its start and end; the shares at what the launch
-    // that sums them costs (their bytes at 3 TB/s + 3.5 us).  The constants are fitted to 4096x14336 / 14336x4096
-    // products of 8 to 512 tokens and to the grouped products of a routed layer (8 experts, 9 to 21 tokens each).
+    // that sums them costs (their bytes at 3 TB/s + 3.5 us).  The constants were fitted when a 16-token workgroup had
+    // four wavefronts (a step of 0.48 us alone, 0.76 us each together; eight wavefronts now halve its steps) and the
+    // 64-token Q4_K kernel walked single steps, to 4096x14336 / 14336x4096 products of 8 to 512 tokens and to the grouped
+    // products of a routed layer.  Against the best of all share counts, over seven shapes from 300x1024 to 14336x4096
+    // with 4 to 512 tokens, they lose on average Q4_0 0.5, Q6_K 0.6, Q8_0 1.1, Q4_K 1.6 %; most for Q4_K with up to 16
+    // tokens, where half as many shares are better (4096x14336, 16 tokens: 32 shares 21.1 us, 16 shares 17.5).
     uint32_t launch_tiles = 0;
     size_t share_bytes = 0;  // one share of every job
     for (uint32_t j = 0; j < n; j++) {
@@ -784,16 +787,19 @@ static void pg_fit(const MatView &m, uint32_t tokens, uint32_t tok, uint32_t ks,
 }
 // Whether a product of F32 / F16 weights takes gemm_plain_kernel.  Up to 16 tokens the launch that cuts the activations
 // costs more than the faster matrix instruction gives (F16 4096x14336, 8 tokens: 40 us on the f32 instruction, 44 here);
-// up to 32 only the two parts of F16 weights are worth it, for matrices large enough to hide that launch (52 -> 46 us;
-// 1000x2048 13.3 -> 14.1; F32 56 -> 61).
+// up to 32 only the two parts of F16 weights are worth it, for matrices large enough to hide that launch (4096x14336, 20
+// tokens 55 -> 46 us; 1000x2048 13.3 -> 14.1; F32 56 -> 61).
 static bool pg_takes(const MatView &m, uint32_t tokens) {
     return tokens > 32 || (tokens > 16 && m.type == T_F16 && (size_t)m.rows * m.cols >= ((size_t)1 << 23));
 }
 // Token tile and column shares, priced together: a step of a workgroup that shares its CU with another and of one that
 // has it alone (us, F16, measured on 4096x14336 with 512 tokens: the wider tile reads and cuts its weights for more
 // tokens), two steps for a workgroup's start and end, and what the launch that sums the shares costs (3 TB/s + 3.5 us).
-// Wide tiles win where there is work for the whole chip (512 tokens: 444 / 334 / 312 us with tiles of 32 / 64 / 128),
-// narrow ones where rows and tokens are few (300x1000, 128 tokens: 14.4 / 15.9 / 21.3 us).
+// Wide tiles win where there is work for the whole chip (512 tokens: 394 / 325 / 296 us with tiles of 32 / 64 / 128, F32
+// 563 / 459 / 438), narrow ones where rows and tokens are few (300x1000, 128 tokens: 16.7 / 18.8 / 26.4 us, F32 18.1 /
+// 20.8 / 28.1).  F32's steps cost more in about the same proportions, so F16's prices do for both: against the best of
+// all tiles and shares, over seven shapes from 300x1024 to 14336x4096 with 40 to 512 tokens, either loses 1.1 % on
+// average and 6.5 (4096x4096, 128 tokens) resp. 5.9 % (14336x4096, 128 tokens) at worst.
 static void pg_plan(const MatView &m, uint32_t tokens, PgPlan &p) {
     static constexpr uint32_t tile[3] = {32, 64, 128};
     static constexpr double shared_us[3] = {0.47, 0.69, 1.25}, alone_us[3] = {0.55, 0.8, 1.39};
