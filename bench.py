@@ -255,8 +255,8 @@ def other_workloads(pkg, hip, gpu, stream, rng, cpu):
                 m.close()
             xd.free(); yd.free()
 
-    # F16 and F32 weights, 4096x14336 (the two dtypes whose products never reach the matrix cores: one token on the
-    # streaming GEMV kernel, more on a vector-ALU tile kernel)
+    # F16 and F32 weights, 4096x14336: one token on the streaming GEMV kernel, up to 32 on the f32 matrix instruction, more as
+    # products of exact bf16 parts (six per multiply-add for F16 weights, nine for F32)
     for ty, nm in ((F16, "f16"), (F32, "f32")):
         rows, cols, n = D, FF, 4
         ws = [synth_matrix(ty, rows, cols, rng) for _ in range(n)]
@@ -270,10 +270,11 @@ def other_workloads(pkg, hip, gpu, stream, rng, cpu):
             flops = 2.0 * rows * cols * tokens
             out[f"gemm_{nm}_{rows}x{cols}_m{tokens}"] = {
                 "call_us": round(us, 2), "tflops": round(flops / us / 1e6, 1),
-                "fp32_frac": round(flops / us / 1e6 / FP32_PEAK_TFLOPS, 4) if tokens > 1 else None,
+                "fp32_frac": round(flops / us / 1e6 / FP32_PEAK_TFLOPS, 4) if 1 < tokens <= 32 else None,
+                "mfma_frac": round((6 if ty == F16 else 9) * flops / us / 1e6 / BF16_MFMA_PEAK_TFLOPS, 4) if tokens > 32 else None,
                 "weight_gbs": round(rows * row_bytes(ty, cols) / us / 1e3, 1),
                 "hbm_frac": round(algorithmic_bytes(ty, rows, cols, tokens) / us / 1e3 / HBM_PEAK_GBS, 4),
-                "bound": "fp32" if tokens >= 128 else "hbm", "cpu_us": None}
+                "bound": "mfma" if tokens >= 128 else "hbm", "cpu_us": None}
         for m in ms:
             m.close()
         xd.free(); yd.free()
