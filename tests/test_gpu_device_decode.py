@@ -208,12 +208,12 @@ def test_fused_and_unfused_device_sessions_agree(pkg, llama, tmp_path, monkeypat
     assert ta.tolist() == tb.tolist()
 
 
-@pytest.mark.parametrize("n_prompt", [3, 17, 140, 300])
+@pytest.mark.parametrize("n_prompt", [3, 17, 140, 300, 513, 520, 1100])
 def test_prompt_as_batches_equals_prompt_step_by_step(pkg, llama, tmp_path, monkeypatch, n_prompt):
-    """All prompt tokens but the last run through the multi-token kernels in chunks of up to 128 (K and V into
+    """All prompt tokens but the last run through the multi-token kernels in chunks of up to 512 (K and V into
     the cache, nothing else kept); LLAMA_HIP_DECODE_STEP_PREFILL runs them as single steps like decode.  Same
-    tokens, logits to 1e-4, also across chunk boundaries (140: 128 + 11; 300: 128 + 128 + 43), for a prompt
-    continued by a second one in the same session, and against the host session."""
+    tokens, logits to 1e-4, also for a whole chunk (513: 512), across chunk boundaries (520: 320 + 199; 1100: 384 + 384
+    + 331), for a prompt continued by a second one in the same session, and against the host session."""
     path = tmp_path / "small.gguf"
     llama.write_synthetic_llama(path, n_layer=3, n_embd=512, n_head=8, n_head_kv=2, n_ff=1536, n_vocab=2048, seed=35)
     m = llama.Llama(path=path)
@@ -247,18 +247,18 @@ def test_batch_session_equals_independent_sessions(pkg, llama, tmp_path, n_seq, 
                                 block_type=block_type, seed=41)
     m = llama.Llama(path=path)
     rng = np.random.default_rng(100 + n_seq)
-    lens = [1, 150, 7, 33, 2, 64, 19, 5] + [int(v) for v in rng.integers(1, 40, 32)]
+    lens = [1, 550, 7, 33, 2, 64, 19, 5] + [int(v) for v in rng.integers(1, 40, 32)]
     prompts = [rng.integers(0, 2048, lens[b]).tolist() for b in range(n_seq)]
-    n_new, cap = 14, 176
+    n_new, cap = 14, 576
     bs = m.batch_session(n_seq, cap)
     together, _, _ = bs.generate_greedy(prompts, n_new)
     for b in range(n_seq):
         alone, _, _ = m.session(device_positions=cap).generate_greedy(prompts[b], n_new)
         assert together[b].tolist() == alone.tolist(), f"sequence {b} of {n_seq}"
     # A second generation in the same session starts every sequence afresh.  In between the executor's workspace
-    # has grown (128-token prompt chunks above, a 300-token host batch here): the session's captured step still
+    # has grown (prompt chunks of up to 512 tokens above, an 800-token host batch here): the session's captured step still
     # points at the workspace it was captured with, which therefore must not have been freed.
-    m.session().forward(rng.integers(0, 2048, 300).tolist())
+    m.session().forward(rng.integers(0, 2048, 800).tolist())
     again, _, _ = bs.generate_greedy(prompts[::-1], n_new)
     assert again[::-1].tolist() == together.tolist()
 

@@ -508,6 +508,24 @@ def test_plain_dtypes_multiply_infinities_and_nan_like_f32(gpu, ty, rows, cols, 
     assert np.all(np.abs(y[finite] - want[finite]) <= K.single_kernel_bound(cols, mag[finite]))
 
 
+@pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
+def test_plain_dtypes_cut_activations_near_the_smallest_numbers(gpu, ty):
+    """The parts of an activation reach down to bf16's smallest number, 2^-133: what an activation below 2^-110 has under
+    that is lost, nothing else (bound: a sequential f32 sum's, plus 2^-133 per unit of weight)."""
+    rng = np.random.default_rng(133)
+    rows, cols, tokens = 160, 64, 40
+    w = rng.uniform(-1, 1, (rows, cols)).astype(np.float32) * np.float32(2.0 ** (15 if ty == K.F16 else 40))
+    w = w.astype(np.float16).astype(np.float32) if ty == K.F16 else w
+    x = (rng.normal(0, 1, (tokens, cols)) * 2.0 ** rng.integers(-118, -104, (tokens, 1))).astype(np.float32)
+    m = gpu.upload_packed(ty, rows, cols, np.ascontiguousarray((w.astype(np.float16) if ty == K.F16 else w).view(np.uint8).reshape(-1)))
+    y = np.zeros(tokens * rows, np.float32)
+    gpu.gemm_resident(m, tokens, x.ravel(), y)
+    m.close()
+    exact, mag = product_by_ieee_rules(w, x)
+    lost = 2.0 ** -133 * np.abs(w.astype(np.float64)).sum(axis=1)
+    assert np.all(np.abs(y.reshape(tokens, rows) - exact) <= K.single_kernel_bound(cols, mag) + lost[None, :])
+
+
 @pytest.mark.parametrize("ty", O.ALL_TYPES, ids=lambda t: O.TYPE_NAMES[t])
 def test_random_gemv_and_gemm_within_bounds(pkg, gpu, ty):
     """Signed scales, every code value, int8 -128, token counts across the kernel switch points."""
