@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <type_traits>
 
 #include "device_once.h"
@@ -44,10 +45,13 @@ static size_t g_lds_limit = 64 * 1024;
 
 // The launchers' view of the device is held once per process.  Every executor reports what it found on its
 // device; the first report sets it, a later one that differs is refused by the caller (one kind of GPU per
-// process: a second kind would need these per device).
+// process: a second kind would need these per device).  Executors may be made on several threads at once; a thread's
+// launches come after its own report, so they need no lock.
+static std::mutex g_report;
 static bool g_limits_set = false;
 bool set_device_limits(int cu_count, size_t lds_per_block) {
     if (cu_count <= 0 || lds_per_block == 0) return false;
+    std::lock_guard<std::mutex> lock(g_report);
     if (g_limits_set) return cu_count == g_cu_count && lds_per_block == g_lds_limit;
     g_cu_count = cu_count;
     g_lds_limit = lds_per_block;
@@ -85,12 +89,10 @@ static hipError_t launch_gemv_t(hipStream_t stream, const MatView *mats, float *
     const size_t lds = ((size_t)b.x_pad + (T == T_F32 || T == T_F16 ? 0 : 2 * (size_t)b.n_chunks)) * sizeof(float);
     if (lds > g_lds_limit) return hipErrorInvalidValue;
     auto kern = gemv_kernel<T, R>;
-    static size_t configured = 0;  // per instantiation
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)g_lds_limit);
+    if (lds > 48 * 1024) {
+        static DeviceOnce limit;  // per instantiation
+        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), g_lds_limit);
         if (e != hipSuccess) return e;
-        configured = g_lds_limit;
     }
     size_t per_cu = g_lds_limit * 2 / (lds ? lds : 1);  // 160 KB of LDS per CU
     if (per_cu < 1) per_cu = 1;
@@ -168,6 +170,7 @@ static float g_nib_mul = 0.f;  // 1 / (value of fp8 byte 0x01); 0 = fp8 unpack n
 static bool g_converts_set = false;
 bool set_nibble_converts(float unit, bool bf16_exact, bool i4_exact) {
     const float mul = unit > 0.f ? 1.0f / unit : 0.f;
+    std::lock_guard<std::mutex> lock(g_report);
     if (g_converts_set) return mul == g_nib_mul && bf16_exact == g_nibble_bf16 && i4_exact == g_nibble_i4;
     g_nib_mul = mul;
     g_nibble_bf16 = bf16_exact;
@@ -200,13 +203,10 @@ static hipError_t launch_q4k_lb(hipStream_t stream, const GemvBatch &b, uint32_t
     } else {
         kern = one ? gemv_q4k_kernel<LB, NW, true, PL, true, PRO> : gemv_q4k_kernel<LB, NW, true, PL, false, PRO>;
     }
-    static size_t configured[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    size_t &conf = configured[4 * (b.pair != 0) + 2 * fp8 + one];
-    if (lds > 48 * 1024 && lds > conf) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)g_lds_limit);
+    if (lds > 48 * 1024) {
+        static DeviceOnce limit[8];
+        const hipError_t e = allow_lds(limit[4 * (b.pair != 0) + 2 * fp8 + one], reinterpret_cast<const void *>(kern), g_lds_limit);
         if (e != hipSuccess) return e;
-        conf = g_lds_limit;
     }
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), lds, stream, b, fp8 ? g_nib_mul : 1.0f);
     return hipGetLastError();
@@ -321,12 +321,10 @@ static hipError_t launch_gemv_q4k(hipStream_t stream, const MatView *mats, float
 template <int LB, int NW>
 static hipError_t launch_q6k_lb(hipStream_t stream, const GemvBatch &b, uint32_t units, size_t lds) {
     auto kern = gemv_q6k_kernel<LB, NW>;
-    static size_t configured = 0;
-    if (lds > 48 * 1024 && lds > configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)g_lds_limit);
+    if (lds > 48 * 1024) {
+        static DeviceOnce limit;
+        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), g_lds_limit);
         if (e != hipSuccess) return e;
-        configured = g_lds_limit;
     }
     size_t per_cu = g_lds_limit * 2 / (lds ? lds : 1);
     if (per_cu < 1) per_cu = 1;
@@ -373,11 +371,10 @@ static hipError_t launch_b32_lb(hipStream_t stream, const GemvBatch &b, uint32_t
     const bool fp8 = T == T_Q4_0 && g_nibble_i4;  // which of the two instantiations
     const void *kern = fp8 ? reinterpret_cast<const void *>(gemv_b32_kernel<T, LB, NW, true>)
                            : reinterpret_cast<const void *>(gemv_b32_kernel<T, LB, NW, false>);
-    static size_t configured[2] = {0, 0};
-    if (lds > 48 * 1024 && lds > configured[fp8]) {
-        hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g_lds_limit);
+    if (lds > 48 * 1024) {
+        static DeviceOnce limit[2];
+        const hipError_t e = allow_lds(limit[fp8], kern, g_lds_limit);
         if (e != hipSuccess) return e;
-        configured[fp8] = g_lds_limit;
     }
     size_t per_cu = g_lds_limit * 2 / (lds ? lds : 1);  // 160 KB of LDS per CU
     if (per_cu < 1) per_cu = 1;
@@ -1295,6 +1292,7 @@ static void *g_scratch_ptr[SCRATCH_MAX_DEVICES];  // per device ordinal, null un
 
 hipError_t static_scratch_init(int device) {
     if (device < 0 || device >= SCRATCH_MAX_DEVICES) return hipErrorInvalidDevice;
+    std::lock_guard<std::mutex> lock(g_report);
     if (g_scratch_ptr[device]) return hipSuccess;
     void *ptr = nullptr;
     const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));  // of the current device
