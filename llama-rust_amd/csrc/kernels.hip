@@ -59,16 +59,12 @@ bool set_device_limits(int cu_count, size_t lds_per_block) {
     return true;
 }
 
-// Jobs must share x, dtype and column count.  hipErrorInvalidValue = "does not fit this
-// kernel" (x too long for LDS); the caller then uses the tiled kernel.
-template <uint32_t T, int R>
-static hipError_t launch_gemv_t(hipStream_t stream, const MatView *mats, float *const *ys, uint32_t n_jobs,
-                                const float *x, bool accumulate) {
+template <uint32_t T, int LB, int R, int K, bool SPLIT>
+static hipError_t launch_rows(hipStream_t stream, const MatView *mats, float *const *ys, uint32_t n_jobs, const float *x, bool accumulate) {
     constexpr int E = Geo<T>::E;
+    constexpr uint32_t GROUP = 64 / LB * R;
     GemvBatch b;
-    const uint32_t cols = mats[0].cols;
-    b.n_chunks = (cols + E - 1) / E;
-    b.x_pad = b.n_chunks * E;
+    b.n_chunks = (mats[0].cols + E - 1) / E;
     b.x = x;
     b.n_jobs = n_jobs;
     uint32_t rgs = 0;
@@ -77,7 +73,7 @@ static hipError_t launch_gemv_t(hipStream_t stream, const MatView *mats, float *
         b.job[j].y = ys[j];
         b.job[j].rg_begin = rgs;
         b.job[j].pad = 0;
-        rgs += (mats[j].rows + R - 1) / R;
+        rgs += (mats[j].rows + GROUP - 1) / GROUP;
     }
     for (uint32_t j = n_jobs; j < GEMV_MAX_JOBS; j++) b.job[j] = b.job[0];
     b.total_rgs = rgs;
@@ -86,19 +82,23 @@ static hipError_t launch_gemv_t(hipStream_t stream, const MatView *mats, float *
     b.x2 = nullptr;
     b.eps = 0.f;
     b.pair = 0;
-    const size_t lds = ((size_t)b.x_pad + (T == T_F32 || T == T_F16 ? 0 : 2 * (size_t)b.n_chunks)) * sizeof(float);
+    const size_t rest = ((T == T_Q5_1 ? (size_t)b.n_chunks : 0) + (SPLIT ? GEMV_WAVES * GROUP : 0)) * sizeof(float);
+    b.x_pad = rows_x_slots<T>(b.n_chunks);
+    if ((size_t)b.x_pad * E * sizeof(float) + rest > g_lds_limit) b.x_pad = b.n_chunks;
+    const size_t lds = (size_t)b.x_pad * E * sizeof(float) + rest;
     if (lds > g_lds_limit) return hipErrorInvalidValue;
-    auto kern = gemv_kernel<T, R>;
+    const bool i4 = T == T_Q4_0 && g_nibble_i4;
+    auto kern = i4 ? gemv_rows_kernel<T, LB, R, K, SPLIT, T == T_Q4_0> : gemv_rows_kernel<T, LB, R, K, SPLIT, false>;
     if (lds > 48 * 1024) {
-        static DeviceOnce limit;  // per instantiation
-        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), g_lds_limit);
+        static DeviceOnce limit[2];  // per instantiation
+        const hipError_t e = allow_lds(limit[i4], reinterpret_cast<const void *>(kern), g_lds_limit);
         if (e != hipSuccess) return e;
     }
     size_t per_cu = g_lds_limit * 2 / (lds ? lds : 1);  // 160 KB of LDS per CU
     if (per_cu < 1) per_cu = 1;
     if (per_cu > 2) per_cu = 2;                          // 16 wavefronts per CU
-    uint32_t grid = (uint32_t)((size_t)g_cu_count * per_cu);
-    const uint32_t needed = (rgs + GEMV_WAVES - 1) / GEMV_WAVES;
+    uint32_t grid = SPLIT ? rgs : (uint32_t)((size_t)g_cu_count * per_cu);
+    const uint32_t needed = SPLIT ? rgs : (rgs + GEMV_WAVES - 1) / GEMV_WAVES;
     if (grid > needed) grid = needed;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(GEMV_WAVES * 64), lds, stream, b);
     return hipGetLastError();
@@ -212,10 +212,9 @@ static hipError_t launch_q4k_lb(hipStream_t stream, const GemvBatch &b, uint32_t
     return hipGetLastError();
 }
 
-// Jobs of a lane-per-unit launch: lb lanes per row, 64 / lb rows per wavefront step.
+// Jobs of a lane-per-unit launch, in row groups of rg_rows rows.
 static uint32_t fill_unit_jobs(GemvBatch &b, const MatView *mats, float *const *ys, uint32_t n_jobs, const float *x,
-                               uint32_t lb) {
-    const uint32_t rg_rows = 64 / lb;
+                               uint32_t rg_rows) {
     b.x = x;
     b.x2 = nullptr;
     b.eps = 0.f;
@@ -272,7 +271,7 @@ static hipError_t launch_gemv_q4k_pro(hipStream_t stream, const MatView *mats, f
         const bool halves = lbb <= 16 && full_steps <= (size_t)10 * g_cu_count;
         const uint32_t lb = halves ? 2 * lbb : lbb;
         GemvBatch b;
-        const uint32_t rgs = fill_unit_jobs(b, mats, ys, n_jobs, x, lb);
+        const uint32_t rgs = fill_unit_jobs(b, mats, ys, n_jobs, x, 64 / lb);
         b.unit0 = win.first(w);
         b.units = units;
         b.accumulate = accumulate || w > 0;
@@ -336,19 +335,61 @@ static hipError_t launch_q6k_lb(hipStream_t stream, const GemvBatch &b, uint32_t
     return hipGetLastError();
 }
 
+template <int LBB, int PL, int NW>
+static hipError_t launch_q6k_part(hipStream_t stream, GemvBatch &b, const MatView *mats, float *const *ys, uint32_t n_jobs, const float *x) {
+    constexpr int LANES = LBB * 8 / PL;
+    constexpr uint32_t rows = LANES > 64 ? NW / (LANES / 64) : NW * 64 / LANES;
+    const uint32_t groups = fill_unit_jobs(b, mats, ys, n_jobs, x, rows);
+    constexpr size_t lds = (size_t)PL * 8 * (LANES * 4 + 4) * sizeof(float);
+    auto kern = gemv_q6k_part_kernel<LBB, PL, NW>;
+    if constexpr (lds > 48 * 1024) {
+        if (lds > g_lds_limit) return hipErrorInvalidValue;
+        static DeviceOnce limit;
+        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kern, dim3(groups), dim3(NW * 64), lds, stream, b);
+    return hipGetLastError();
+}
+
 static hipError_t launch_gemv_q6k(hipStream_t stream, const MatView *mats, float *const *ys, uint32_t n_jobs,
                                   const float *x, bool accumulate) {
     const uint32_t nb = mats[0].nb;
+    size_t rows = 0;
+    for (uint32_t j = 0; j < n_jobs; j++) rows += mats[j].rows;
     const UnitWindows win(nb, 64);
     for (uint32_t w = 0; w < win.n; w++) {
         const uint32_t units = win.count(w, nb);
         uint32_t lb = 1;
         while (lb < 64 && lb < units) lb <<= 1;
         GemvBatch b;
-        const uint32_t rgs = fill_unit_jobs(b, mats, ys, n_jobs, x, lb);
         b.unit0 = win.first(w);
         b.units = units;
         b.accumulate = accumulate || w > 0;
+        // One step per wavefront, on the graph: 512x1024 4.2 -> 2.9 us, 4096x4096 6.2 -> 5.4, 2048x11008 9.8 -> 7.9, 128256x4096
+        // 71.2 -> 66.9; between those sizes the loop is faster (14336x4096 11.2 against 11.8, 32000x4096 20.3 against 21.0).
+        hipError_t part = hipErrorInvalidValue;
+        const size_t lanes = rows * lb;
+        auto small = [&](auto tag) {
+            constexpr int LBB = decltype(tag)::value;
+            part = lanes > 65536 ? launch_q6k_part<LBB, 4, 4>(stream, b, mats, ys, n_jobs, x) : launch_q6k_part<LBB, 2, 4>(stream, b, mats, ys, n_jobs, x);
+        };
+        if (lanes <= 131072) {
+            switch (lb) {
+            case 1: small(std::integral_constant<int, 1>{}); break;
+            case 2: small(std::integral_constant<int, 2>{}); break;
+            case 4: small(std::integral_constant<int, 4>{}); break;
+            case 8: small(std::integral_constant<int, 8>{}); break;
+            case 16: small(std::integral_constant<int, 16>{}); break;
+            case 32: small(std::integral_constant<int, 32>{}); break;
+            default: part = launch_q6k_part<64, 4, 8>(stream, b, mats, ys, n_jobs, x); break;
+            }
+        } else if (lb == 16 && lanes >= 1000000) {
+            part = launch_q6k_part<16, 8, 4>(stream, b, mats, ys, n_jobs, x);
+        }
+        if (part == hipSuccess) continue;
+        if (part != hipErrorInvalidValue) return part;
+        const uint32_t rgs = fill_unit_jobs(b, mats, ys, n_jobs, x, 64 / lb);
         const size_t lds = (size_t)(64 * (lb * 4 + 4)) * sizeof(float);
         if (lds > g_lds_limit) return hipErrorInvalidValue;
         hipError_t e;
@@ -366,66 +407,78 @@ static hipError_t launch_gemv_q6k(hipStream_t stream, const MatView *mats, float
     return hipSuccess;
 }
 
-template <uint32_t T, int LB, int NW>
-static hipError_t launch_b32_lb(hipStream_t stream, const GemvBatch &b, uint32_t units, size_t lds) {
-    const bool fp8 = T == T_Q4_0 && g_nibble_i4;  // which of the two instantiations
-    const void *kern = fp8 ? reinterpret_cast<const void *>(gemv_b32_kernel<T, LB, NW, true>)
-                           : reinterpret_cast<const void *>(gemv_b32_kernel<T, LB, NW, false>);
-    if (lds > 48 * 1024) {
+template <uint32_t T, int LBB, int PL, int NW>
+static hipError_t launch_b32(hipStream_t stream, GemvBatch &b, const MatView *mats, float *const *ys, uint32_t n_jobs, const float *x) {
+    using G = B32Geo<T>;
+    constexpr int LANES = LBB * 8 / PL;
+    // a row group of the launch-wide numbering is a workgroup's rows
+    constexpr uint32_t rows = LANES > 64 ? NW / (LANES / 64) : NW * 64 / LANES;
+    const uint32_t groups = fill_unit_jobs(b, mats, ys, n_jobs, x, rows);
+    constexpr size_t lds = (size_t)(PL * G::XV * (LANES * 4 + 4) + (T == T_Q5_1 ? PL * LANES : 0)) * sizeof(float);
+    const bool i4 = T == T_Q4_0 && g_nibble_i4;
+    auto kern = i4 ? gemv_b32_kernel<T, LBB, PL, NW, T == T_Q4_0> : gemv_b32_kernel<T, LBB, PL, NW, false>;
+    if constexpr (lds > 48 * 1024) {
+        if (lds > g_lds_limit) return hipErrorInvalidValue;
         static DeviceOnce limit[2];
-        const hipError_t e = allow_lds(limit[fp8], kern, g_lds_limit);
+        const hipError_t e = allow_lds(limit[i4], reinterpret_cast<const void *>(kern), lds);
         if (e != hipSuccess) return e;
     }
-    size_t per_cu = g_lds_limit * 2 / (lds ? lds : 1);  // 160 KB of LDS per CU
-    if (per_cu < 1) per_cu = 1;
-    constexpr size_t wpc = T == T_Q8_0 ? 32 : 16;       // wavefronts per CU (measured: Q8_0 +5 % at 32, Q4_0 -4 %)
-    if (per_cu > wpc / NW) per_cu = wpc / NW;
-    uint32_t grid = (uint32_t)((size_t)g_cu_count * per_cu);
-    const uint32_t needed = (units + NW - 1) / NW;
-    if (grid > needed) grid = needed;
-    if (fp8)
-        hipLaunchKernelGGL((gemv_b32_kernel<T, LB, NW, true>), dim3(grid), dim3(NW * 64), lds, stream, b);
-    else
-        hipLaunchKernelGGL((gemv_b32_kernel<T, LB, NW, false>), dim3(grid), dim3(NW * 64), lds, stream, b);
+    hipLaunchKernelGGL(kern, dim3(groups), dim3(NW * 64), lds, stream, b);
     return hipGetLastError();
 }
 
-// hipErrorInvalidValue: rows are not whole units (block-order layout).
+// How a window's rows are cut.  Parts of a unit where rows are few or short: their lanes make the wavefronts (and the
+// bytes in flight) that whole units would not.  Whole units where both are plenty, for the row work they share.
+// Quarters / halves / whole units, us: Q4_0 512x4096 2.85 / 3.3 / -, 14336x4096 8.9 / 9.0 / -, 32000x4096 17.3 / 16.1 / -,
+// 4096x8192 6.4 / 6.6 / 7.1, 4096x14336 11.0 / 11.3 / 11.1, 16384x14336 35.7 / 35.2 / 31.0; Q8_0 512x4096 - / 3.0 / 3.2,
+// 4096x4096 6.0 / 5.6 / 5.5, 16384x8192 32.2 / 27.1 / 25.6.
+template <uint32_t T>
+static hipError_t launch_b32_window(hipStream_t stream, GemvBatch &b, size_t rows, const MatView *mats, float *const *ys, uint32_t n,
+                                    const float *x) {
+    const bool few = rows < 2048;
+    // quarters of units would make more than 48 wavefronts per CU
+    auto plenty = [&](uint32_t lbb) { return rows * lbb > (size_t)768 * g_cu_count; };
+    auto quarters_or_halves = [&](auto tag) {
+        constexpr int LBB = decltype(tag)::value;
+        return plenty(LBB) ? launch_b32<T, LBB, 4, 4>(stream, b, mats, ys, n, x) : launch_b32<T, LBB, 2, 4>(stream, b, mats, ys, n, x);
+    };
+    if (b.units <= 1) return quarters_or_halves(std::integral_constant<int, 1>{});
+    if (b.units <= 2) return quarters_or_halves(std::integral_constant<int, 2>{});
+    if (b.units <= 4) return quarters_or_halves(std::integral_constant<int, 4>{});
+    if (b.units <= 8) return quarters_or_halves(std::integral_constant<int, 8>{});
+    if (b.units <= 16) {
+        if (few || plenty(16)) return quarters_or_halves(std::integral_constant<int, 16>{});
+        return launch_b32<T, 16, 2, 8>(stream, b, mats, ys, n, x);
+    }
+    if (b.units <= 32) {
+        if constexpr (T == T_Q8_0)
+            return few ? launch_b32<T, 32, 4, 4>(stream, b, mats, ys, n, x) : launch_b32<T, 32, 8, 4>(stream, b, mats, ys, n, x);
+        else
+            return few ? launch_b32<T, 32, 2, 4>(stream, b, mats, ys, n, x) : launch_b32<T, 32, 4, 8>(stream, b, mats, ys, n, x);
+    }
+    if (b.units <= 64)
+        return rows < 3072 ? launch_b32<T, 64, 4, 8>(stream, b, mats, ys, n, x) : launch_b32<T, 64, 8, 8>(stream, b, mats, ys, n, x);
+    if constexpr (T == T_Q8_0)  // its units are half as long
+        return rows < 8192 ? launch_b32<T, 128, 8, 8>(stream, b, mats, ys, n, x) : launch_b32<T, 128, 8, 16>(stream, b, mats, ys, n, x);
+    return hipErrorInvalidValue;
+}
+
+// Rows of whole units (piece-major planes).
 template <uint32_t T>
 static hipError_t launch_gemv_b32(hipStream_t stream, const MatView *mats, float *const *ys, uint32_t n_jobs,
                                   const float *x, bool accumulate) {
     using G = B32Geo<T>;
     const uint32_t cols = mats[0].cols;
-    if (!piece_major(T, cols)) return hipErrorInvalidValue;
     const uint32_t nu = cols / G::UC;
-    // up to 64 lanes per row, and as many unit columns per lane as keep x within LDS
-    const size_t iter_lds = (size_t)((G::UC / 4) * (64 * 4 + 4) + G::NBLK * 64) * sizeof(float);
-    const uint32_t max_iter = (uint32_t)(g_lds_limit / iter_lds) ? (uint32_t)(g_lds_limit / iter_lds) : 1;
-    const UnitWindows win(nu, 64 * max_iter);
+    size_t rows = 0;
+    for (uint32_t j = 0; j < n_jobs; j++) rows += mats[j].rows;
+    const UnitWindows win(nu, 16384 / G::UC);  // x of a window within LDS
     for (uint32_t w = 0; w < win.n; w++) {
-        const uint32_t units = win.count(w, nu);
-        uint32_t lb = 1;
-        while (lb < 64 && lb < units) lb <<= 1;
-        const uint32_t n_iter = (units + lb - 1) / lb;
         GemvBatch b;
-        const uint32_t rgs = fill_unit_jobs(b, mats, ys, n_jobs, x, lb);
         b.unit0 = win.first(w);
-        b.units = units;
+        b.units = win.count(w, nu);
         b.accumulate = accumulate || w > 0;
-        const size_t lds = (size_t)n_iter * ((G::UC / 4) * (lb * 4 + 4) + G::NBLK * lb) * sizeof(float);
-        if (lds > g_lds_limit) return hipErrorInvalidValue;
-        hipError_t e;
-        switch (lb) {
-        case 1: e = launch_b32_lb<T, 1, 4>(stream, b, rgs, lds); break;
-        case 2: e = launch_b32_lb<T, 2, 4>(stream, b, rgs, lds); break;
-        case 4: e = launch_b32_lb<T, 4, 4>(stream, b, rgs, lds); break;
-        case 8: e = launch_b32_lb<T, 8, 4>(stream, b, rgs, lds); break;
-        case 16: e = launch_b32_lb<T, 16, 4>(stream, b, rgs, lds); break;
-        case 32: e = launch_b32_lb<T, 32, 8>(stream, b, rgs, lds); break;
-        default:  // 16 wavefronts per workgroup measured 3 % faster for Q8_0, 12 % slower for the nibble dtypes
-            e = T == T_Q8_0 ? launch_b32_lb<T, 64, 16>(stream, b, rgs, lds) : launch_b32_lb<T, 64, 8>(stream, b, rgs, lds);
-            break;
-        }
+        const hipError_t e = launch_b32_window<T>(stream, b, rows, mats, ys, n_jobs, x);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -444,18 +497,32 @@ static hipError_t launch_multi_t(hipStream_t stream, const MatView *mats, float 
     if constexpr (T == T_Q4_K) return launch_gemv_q4k(stream, mats, ys, n, x, accumulate);
     if constexpr (T == T_Q6_K) return launch_gemv_q6k(stream, mats, ys, n, x, accumulate);
     if constexpr (T == T_Q8_0 || T == T_Q4_0 || T == T_Q5_0 || T == T_Q5_1) {
-        hipError_t e = launch_gemv_b32<T>(stream, mats, ys, n, x, accumulate);
-        if (e != hipErrorInvalidValue) return e;
-        (void)hipGetLastError();
+        if (piece_major(T, mats[0].cols)) return launch_gemv_b32<T>(stream, mats, ys, n, x, accumulate);
     }
-    // Rows per lane: four share the lane's activations, but a wavefront owns whole row groups, so
-    // matrices with few rows take fewer rows per group to give every wavefront of the chip one.
-    size_t rows = 0;
-    for (uint32_t j = 0; j < n; j++) rows += mats[j].rows;
-    const size_t wavefronts = (size_t)g_cu_count * 16;
-    if (rows >= 4 * wavefronts) return launch_gemv_t<T, 4>(stream, mats, ys, n, x, accumulate);
-    if (rows >= 2 * wavefronts) return launch_gemv_t<T, 2>(stream, mats, ys, n, x, accumulate);
-    return launch_gemv_t<T, 1>(stream, mats, ys, n, x, accumulate);
+    if constexpr (T != T_Q4_K && T != T_Q6_K) {
+        // The wavefronts of a workgroup share a row where rows are long and too few to keep the chip busy one per wavefront, or
+        // long enough that the last wavefronts would run alone (shared / one per wavefront, us: Q4_0 512x11040 5.0 / 6.3,
+        // 4864x11040 11.9 / 13.2, 16384x11040 29 / 23.9; F16 2048x4096 5.45 / 6.3, 16384x4096 21.1 / 22.7; F32 16384x4096
+        // 38.6 / 42.0, 16384x2080 26.7 / 22.1).  Sums are formed in an order that depends on this choice.
+        size_t rows = 0;
+        for (uint32_t j = 0; j < n; j++) rows += mats[j].rows;
+        const uint32_t chunks = (mats[0].cols + Geo<T>::E - 1) / Geo<T>::E;
+        constexpr bool PLAIN = T == T_F32 || T == T_F16;
+        if constexpr (PLAIN) {
+            if (chunks >= 1024 || (chunks >= 512 && rows < 8192)) {
+                if (T == T_F32 || rows < 1024) return launch_rows<T, 64, 2, 2, true>(stream, mats, ys, n, x, accumulate);
+                return launch_rows<T, 32, 2, 1, true>(stream, mats, ys, n, x, accumulate);
+            }
+            if (chunks < 128 && rows >= 8192) return launch_rows<T, 32, T == T_F32 ? 2 : 1, T == T_F32 ? 1 : 2, false>(stream, mats, ys, n, x, accumulate);
+            if (T == T_F32 && chunks >= 128) return launch_rows<T, 64, 1, 4, false>(stream, mats, ys, n, x, accumulate);
+            return launch_rows<T, 64, 1, 2, false>(stream, mats, ys, n, x, accumulate);
+        } else {
+            constexpr int K = T == T_Q8_0 ? 2 : 1;  // chunks of 32 columns
+            if (chunks * Geo<T>::E >= 4096 && rows < 8192) return launch_rows<T, 32, 2, 1, true>(stream, mats, ys, n, x, accumulate);
+            if (chunks <= 16 * K && rows >= 8192) return launch_rows<T, 16, 2, K, false>(stream, mats, ys, n, x, accumulate);
+            return launch_rows<T, 32, 1, K, false>(stream, mats, ys, n, x, accumulate);
+        }
+    }
 }
 
 // ---- MFMA GEMM: planning and launch

@@ -547,6 +547,44 @@ def test_random_gemv_and_gemm_within_bounds(pkg, gpu, ty):
         m.close()
 
 
+# Rows and columns on both sides of every rule that picks a single-token kernel, and of the lanes, parts and steps inside it.
+_LONG = 20480  # columns of x that fill a workgroup's LDS
+_SINGLE_TOKEN = {
+    K.F32: [(1, 1), (3, 33), (64, 511), (65, 513), (1023, 2047), (1024, 2052), (8191, 515), (8192, 509), (8193, 2048), (8200, 4099),
+            (5, _LONG), (5, _LONG + 4)],
+    K.F16: [(1, 1), (3, 33), (64, 1023), (65, 1025), (1023, 4096), (1024, 4100), (8191, 1030), (8192, 1016), (8193, 4095), (8200, 8193),
+            (5, _LONG), (5, _LONG + 8)],
+    K.Q6_K: [(1, 256), (3, 512), (63, 1280), (257, 2304), (100, 4352), (31, 8448), (7, 16384), (9, 16640), (65537, 256), (131073, 256),
+             (4097, 4096), (8193, 4096), (2049, 8192), (2048, 11008), (2049, 16384), (62501, 4096)],
+}
+_BLOCKS = [(1, 32), (3, 96), (64, 288), (63, 512 + 32), (2049, 4064), (2047, 4128), (8191, 4128), (8192, 4128), (8191, 480), (8192, 480),
+           (8193, 576), (5, _LONG - 32 * 20 - 32), (3, _LONG + 32)]  # rows that are not whole units
+_UNITS = [(1, 1), (2, 2), (5, 3), (63, 4), (65, 5), (100, 9), (2047, 16), (2048, 16), (2047, 17), (2048, 32), (12289, 16), (24577, 8),
+          (100, 33), (3071, 40), (3072, 64), (7, 65), (33, 127), (3, 129)]
+
+
+@pytest.mark.parametrize("ty", O.ALL_TYPES, ids=lambda t: O.TYPE_NAMES[t])
+def test_single_token_products_on_both_sides_of_every_rule(pkg, gpu, ty):
+    """Every output within the product's own bounds."""
+    if ty in (K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0):
+        unit = 128 if ty == K.Q8_0 else 256
+        shapes = _BLOCKS + [(r, n * unit) for r, n in _UNITS]
+    else:
+        shapes = _SINGLE_TOKEN.get(ty, [(1, 256), (5, 768), (2049, 4096), (3, 16640)])
+    rng = np.random.default_rng(70 + ty)
+    for rows, cols in shapes:
+        w = K.random_packed(ty, rows, cols, rng, scale=0.02)
+        x = rng.normal(0, 1, cols).astype(np.float32)
+        m = gpu.upload_packed(ty, rows, cols, w)
+        y = np.full(rows, np.nan, np.float32)
+        gpu.gemv_resident(m, x, y)
+        exact, mag = O.gemm_f64_mag(ty, cols, 1, w, x, rows)
+        err = np.abs(y.astype(np.float64) - exact[0])
+        bad = np.flatnonzero(~(err <= np.minimum(K.single_kernel_bound(cols, mag[0]), K.observed_envelope_u(cols) * K.U * mag[0])))
+        assert bad.size == 0, f"{rows}x{cols}: {bad.size} outputs, first {bad[0]}: {y[bad[0]]} for {exact[0][bad[0]]}"
+        m.close()
+
+
 @pytest.mark.parametrize("rows,cols,tokens", [(1, 256, 33), (255, 512, 64), (256, 768, 65), (257, 4352, 97), (600, 14336, 128),
                                               (4099, 1280, 129)])
 def test_q4_k_products_of_more_than_32_tokens(gpu, rows, cols, tokens):
