@@ -562,16 +562,14 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     bool any_split = false;
     const uint32_t n_steps = mats[0].cols / 32;
     // Columns are shared between workgroups as far as that shortens the launch: every share costs a partial
-    // result written and read back.  A CU holds two workgroups of these kernels, and one alone already gets 0.63-0.7
-    // of what the two get together, so what counts is how evenly the steps fall on the CUs.  The launch is priced in steps of a
-    // workgroup that shares its CU: whole rounds of 2 x CUs workgroups, then the rest (alone on their CUs if they
-    // are at most one per CU), two more steps per workgroup for its start and end; the shares at what the launch
-    // that sums them costs (their bytes at 3 TB/s + 3.5 us).  The constants were fitted when a 16-token workgroup had
-    // four wavefronts (a step of 0.48 us alone, 0.76 us each together; eight wavefronts now halve its steps) and the
-    // 64-token Q4_K kernel walked single steps, to 4096x14336 / 14336x4096 products of 8 to 512 tokens and to the grouped
-    // products of a routed layer.  Against the best of all share counts, over seven shapes from 300x1024 to 14336x4096
-    // with 4 to 512 tokens, they lose on average Q4_0 0.5, Q6_K 0.6, Q8_0 1.1, Q4_K 1.6 %; most for Q4_K with up to 16
-    // tokens, where half as many shares are better (4096x14336, 16 tokens: 32 shares 21.1 us, 16 shares 17.5).
+    // result written and read back.  A CU holds two workgroups of these kernels, and one alone already gets 0.53-0.7
+    // of what two get together (the 16-token kernel's eight wavefronts least), so what counts is how evenly the steps fall
+    // on the CUs.  The launch is priced in steps of a workgroup that shares its CU: whole rounds of 2 x CUs workgroups, then
+    // the rest (alone on their CUs if they are at most one per CU), two more steps per workgroup for its start and end; the
+    // shares at what the launch that sums them costs.  The constants are fitted to the times of all share counts, over five
+    // dtypes and ten shapes from 256x1024 to 4096x14336 and 11008x2048 with 3 to 512 tokens: against the best count of each,
+    // the plan loses 0.2 % on average with up to 16 tokens (4.6 at most; 1.1 and 15 with the 64-token kernel's constants: Q4_K
+    // 4096x14336 at 3 tokens 18.4 -> 16.0 us, 6144x4096 at 6 tokens 13.5 -> 12.6), none up to 32 and 0.3 above.
     uint32_t launch_tiles = 0;
     size_t share_bytes = 0;  // one share of every job
     for (uint32_t j = 0; j < n; j++) {
@@ -584,15 +582,16 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     if (ks_max > 32) ks_max = 32;
     if (ks_max < 1) ks_max = 1;
     const uint32_t slots = (uint32_t)(2 * g_cu_count), alone = (uint32_t)g_cu_count;
-    const double step_us = p.tt == 2 ? 1.5 : 0.7;
+    const double step_us = p.tile16 ? 0.8 : p.tt == 2 ? 1.7 : 0.7, alone_cost = p.tile16 ? 0.53 : 0.7;
+    const double bytes_per_us = p.tile16 ? 6.0e6 : p.tt == 2 ? 4.0e6 : 3.0e6;
     uint32_t ks_launch = 1;
     double best = 0.0;
     for (uint32_t ks = 1; ks <= ks_max; ks++) {
         const uint64_t wg = (uint64_t)(launch_tiles ? launch_tiles : 1) * ks;
         const double len = (double)((n_steps + ks - 1) / ks) + 2.0;
         const uint64_t rounds = wg / slots, rest = wg % slots;
-        double cost = (double)rounds * len + (rest == 0 ? 0.0 : rest <= alone ? 0.7 * len : len);
-        if (ks > 1) cost += ((double)ks * (double)share_bytes / 3.0e6 + 3.5) / step_us;
+        double cost = (double)rounds * len + (rest == 0 ? 0.0 : rest <= alone ? alone_cost * len : len);
+        if (ks > 1) cost += ((double)ks * (double)share_bytes / bytes_per_us + 3.5) / step_us;
         if (ks == 1 || cost < best) {
             best = cost;
             ks_launch = ks;
