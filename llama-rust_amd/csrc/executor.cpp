@@ -15,6 +15,7 @@
 
 #include "../../include/native_hip.h"
 #include "early_gemm.h"
+#include "head_step.h"
 #include "host_range.h"
 #include "kernels.h"
 
@@ -807,7 +808,7 @@ namespace {
 // lnh_gemm_act_device (x) and lnh_gemm_plain_act_device (dx): the product's activations split or plain.
 int gemm_act(lnh_exec *e, size_t n_mats, const lnh_matrix *const *mats, const lnh_act *x, const float *dx, size_t tokens,
              float *const *dys, int epilogue, float *d_residual, const float *d_norm_w, float eps, float *d_xn, lnh_act *next,
-             void *stream) {
+             void *stream, const nh::ActEpilogue *argmax = nullptr) {
     if (!e) return LNH_ERR_INVALID;
     if (!mats || (!x && !dx) || n_mats == 0) return fail(e, LNH_ERR_INVALID, "matrix list or activations are null");
     if (misaligned(dx) || misaligned(d_residual) || misaligned(d_norm_w)) return fail(e, LNH_ERR_INVALID, "device input buffers must be 16-byte aligned");
@@ -872,6 +873,7 @@ int gemm_act(lnh_exec *e, size_t n_mats, const lnh_matrix *const *mats, const ln
         break;
     default: return fail(e, LNH_ERR_INVALID, "unknown epilogue");
     }
+    if (argmax) ep = *argmax;
     ep.residual = d_residual;
     ep.norm_w = d_norm_w;
     ep.eps = eps;
@@ -923,6 +925,43 @@ int lnh_gemm_plain_act_device(lnh_exec *e, size_t n_mats, const lnh_matrix *cons
     if (e && !dx) return fail(e, LNH_ERR_INVALID, "buffer pointer is null");
     return gemm_act(e, n_mats, mats, nullptr, dx, tokens, dys, epilogue, d_residual, d_norm_w, eps, d_xn, next, stream);
 }
+
+}  // extern "C"
+
+namespace nh {
+
+size_t head_candidates(const lnh_matrix *m) { return m ? head_candidates(m->view) : 0; }
+
+int head_device(lnh_exec *e, const lnh_matrix *m, const float *dx, const float *norm_w, float eps, float *dy, float *cand_v,
+                uint32_t *cand_i, void *stream) {
+    size_t inputs, outputs;
+    const int rc = check_gemm(e, m, 1, false, 0, 0, &inputs, &outputs);
+    if (rc != LNH_OK) return rc;
+    if (!dx || !norm_w || !dy || !cand_v || !cand_i) return fail(e, LNH_ERR_INVALID, "buffer pointer is null");
+    if (misaligned(dx) || misaligned(norm_w)) return fail(e, LNH_ERR_INVALID, "device input buffers must be 16-byte aligned");
+    const hipError_t h = launch_head(stream ? static_cast<hipStream_t>(stream) : e->stream, m->view, dx, norm_w, eps, dy, cand_v, cand_i);
+    if (h == hipErrorInvalidValue) {
+        (void)hipGetLastError();
+        return fail(e, LNH_ERR_UNSUPPORTED, "no output-head launch for this dtype or row length");
+    }
+    return h == hipSuccess ? LNH_OK : hip_fail(e, h, "HIP kernel launch");
+}
+
+int head_act_device(lnh_exec *e, const lnh_matrix *m, const lnh_act *x, size_t tokens, float *dy, float *cand_v, uint32_t *cand_i,
+                    uint32_t n_cand, void *stream) {
+    if (e && (!x || !dy || !cand_v || !cand_i || n_cand == 0)) return fail(e, LNH_ERR_INVALID, "buffer pointer is null");
+    ActEpilogue ep;
+    ep.kind = ACT_EPILOGUE_ARGMAX;
+    ep.y = dy;
+    ep.cand_v = cand_v;
+    ep.cand_i = cand_i;
+    ep.n_cand = n_cand;
+    return gemm_act(e, 1, &m, x, nullptr, tokens, &dy, LNH_EPILOGUE_NONE, nullptr, nullptr, 0.f, nullptr, nullptr, stream, &ep);
+}
+
+}  // namespace nh
+
+extern "C" {
 
 int lnh_gemm_grouped_device(lnh_exec *e, size_t n_groups, const lnh_matrix *const *mats, const size_t *tokens,
                             const float *dx, float *dy, void *stream) {

@@ -55,7 +55,7 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
 //                         of one per token.  tokens <= ACT_DEFER_MAX_TOKENS.
 // ws must hold gemm_act_workspace_bytes() for the same arguments.  hipErrorInvalidValue = not this path's case,
 // nothing launched.
-enum { ACT_EPILOGUE_NONE = 0, ACT_EPILOGUE_ADD_RMSNORM = 1, ACT_EPILOGUE_SWIGLU = 2, ACT_EPILOGUE_ADD_DEFER = 3 };
+enum { ACT_EPILOGUE_NONE = 0, ACT_EPILOGUE_ADD_RMSNORM = 1, ACT_EPILOGUE_SWIGLU = 2, ACT_EPILOGUE_ADD_DEFER = 3, ACT_EPILOGUE_ARGMAX = 4 };
 constexpr size_t ACT_NORM_MAX_ROW_BYTES = 48 * 1024;  // ADD_RMSNORM: rows of at most 12288 floats
 constexpr uint32_t ACT_DEFER_MAX_TOKENS = 32;         // the products whose main launch cuts plain rows itself
 constexpr size_t ACT_DEFER_PARTIAL_BYTES = ACT_DEFER_MAX_TOKENS * 16 * sizeof(float);
@@ -68,7 +68,14 @@ struct ActEpilogue {
     float *partial = nullptr;  // ADD_DEFER
     void *next_act = nullptr;
     uint32_t next_type = 0, next_cols = 0, next_max_tokens = 0;
+    float *y = nullptr, *cand_v = nullptr;  // ARGMAX: the rows, and n_cand candidates of each
+    uint32_t *cand_i = nullptr, n_cand = 0;
 };
+// y = W rmsnorm(x) * norm_w for one token, and the largest output of each of head_candidates(m) workgroups with its row.
+// head_candidates: 0 where no such launch exists (then launch_head is hipErrorInvalidValue).
+uint32_t head_candidates(const MatView &m);
+hipError_t launch_head(hipStream_t stream, const MatView &m, const float *x, const float *norm_w, float eps, float *y, float *cand_v,
+                       uint32_t *cand_i);
 size_t act_bytes(uint32_t type, uint32_t cols, uint32_t max_tokens);
 hipError_t launch_act_split(hipStream_t stream, void *act, uint32_t type, uint32_t cols, uint32_t max_tokens, uint32_t tokens,
                             const float *x);

@@ -82,6 +82,8 @@ static hipError_t launch_rows(hipStream_t stream, const MatView *mats, float *co
     b.x2 = nullptr;
     b.eps = 0.f;
     b.pair = 0;
+    b.cand_v = nullptr;
+    b.cand_i = nullptr;
     const size_t rest = ((T == T_Q5_1 ? (size_t)b.n_chunks : 0) + (SPLIT ? GEMV_WAVES * GROUP : 0)) * sizeof(float);
     b.x_pad = rows_x_slots<T>(b.n_chunks);
     if ((size_t)b.x_pad * E * sizeof(float) + rest > g_lds_limit) b.x_pad = b.n_chunks;
@@ -219,6 +221,8 @@ static uint32_t fill_unit_jobs(GemvBatch &b, const MatView *mats, float *const *
     b.x2 = nullptr;
     b.eps = 0.f;
     b.pair = 0;
+    b.cand_v = nullptr;
+    b.cand_i = nullptr;
     b.n_jobs = n_jobs;
     b.n_chunks = 0;
     b.x_pad = mats[0].cols;
@@ -317,12 +321,32 @@ static hipError_t launch_gemv_q4k(hipStream_t stream, const MatView *mats, float
     }
 }
 
+// An output head's launch: what its kernels add to the product, and how many workgroups (candidates) it has.
+struct Q6kHead {
+    const float *norm_w = nullptr;
+    float eps = 0.f;
+    float *cand_v = nullptr;  // null: only the count is wanted
+    uint32_t *cand_i = nullptr;
+    uint32_t groups = 0;
+    void set(GemvBatch &b) const {
+        b.x2 = norm_w;
+        b.eps = eps;
+        b.cand_v = cand_v;
+        b.cand_i = cand_i;
+    }
+    bool planned(uint32_t grid) {
+        groups = grid;
+        return cand_v == nullptr;
+    }
+};
+
 template <int LB, int NW>
-static hipError_t launch_q6k_lb(hipStream_t stream, const GemvBatch &b, uint32_t units, size_t lds) {
-    auto kern = gemv_q6k_kernel<LB, NW>;
+static hipError_t launch_q6k_lb(hipStream_t stream, const GemvBatch &b, uint32_t units, size_t lds, Q6kHead *head) {
+    auto kern = head ? gemv_q6k_kernel<LB, NW, true> : gemv_q6k_kernel<LB, NW>;
+    if (head) lds += NW * sizeof(float);
     if (lds > 48 * 1024) {
-        static DeviceOnce limit;
-        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), g_lds_limit);
+        static DeviceOnce limit[2];
+        const hipError_t e = allow_lds(limit[head != nullptr], reinterpret_cast<const void *>(kern), g_lds_limit);
         if (e != hipSuccess) return e;
     }
     size_t per_cu = g_lds_limit * 2 / (lds ? lds : 1);
@@ -331,33 +355,38 @@ static hipError_t launch_q6k_lb(hipStream_t stream, const GemvBatch &b, uint32_t
     uint32_t grid = (uint32_t)((size_t)g_cu_count * per_cu);
     const uint32_t needed = (units + NW - 1) / NW;
     if (grid > needed) grid = needed;
+    if (head && head->planned(grid)) return hipSuccess;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), lds, stream, b);
     return hipGetLastError();
 }
 
 template <int LBB, int PL, int NW>
-static hipError_t launch_q6k_part(hipStream_t stream, GemvBatch &b, const MatView *mats, float *const *ys, uint32_t n_jobs, const float *x) {
+static hipError_t launch_q6k_part(hipStream_t stream, GemvBatch &b, const MatView *mats, float *const *ys, uint32_t n_jobs, const float *x,
+                                  Q6kHead *head) {
     constexpr int LANES = LBB * 8 / PL;
     constexpr uint32_t rows = LANES > 64 ? NW / (LANES / 64) : NW * 64 / LANES;
     const uint32_t groups = fill_unit_jobs(b, mats, ys, n_jobs, x, rows);
-    constexpr size_t lds = (size_t)PL * 8 * (LANES * 4 + 4) * sizeof(float);
-    auto kern = gemv_q6k_part_kernel<LBB, PL, NW>;
+    if (head) head->set(b);
+    constexpr size_t lds = ((size_t)PL * 8 * (LANES * 4 + 4) + NW) * sizeof(float);
+    auto kern = head ? gemv_q6k_part_kernel<LBB, PL, NW, true> : gemv_q6k_part_kernel<LBB, PL, NW>;
     if constexpr (lds > 48 * 1024) {
         if (lds > g_lds_limit) return hipErrorInvalidValue;
-        static DeviceOnce limit;
-        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
+        static DeviceOnce limit[2];
+        const hipError_t e = allow_lds(limit[head != nullptr], reinterpret_cast<const void *>(kern), lds);
         if (e != hipSuccess) return e;
     }
+    if (head && head->planned(groups)) return hipSuccess;
     hipLaunchKernelGGL(kern, dim3(groups), dim3(NW * 64), lds, stream, b);
     return hipGetLastError();
 }
 
 static hipError_t launch_gemv_q6k(hipStream_t stream, const MatView *mats, float *const *ys, uint32_t n_jobs,
-                                  const float *x, bool accumulate) {
+                                  const float *x, bool accumulate, Q6kHead *head = nullptr) {
     const uint32_t nb = mats[0].nb;
     size_t rows = 0;
     for (uint32_t j = 0; j < n_jobs; j++) rows += mats[j].rows;
     const UnitWindows win(nb, 64);
+    if (head && win.n != 1) return hipErrorInvalidValue;  // the norm needs all of x in one workgroup
     for (uint32_t w = 0; w < win.n; w++) {
         const uint32_t units = win.count(w, nb);
         uint32_t lb = 1;
@@ -372,7 +401,7 @@ static hipError_t launch_gemv_q6k(hipStream_t stream, const MatView *mats, float
         const size_t lanes = rows * lb;
         auto small = [&](auto tag) {
             constexpr int LBB = decltype(tag)::value;
-            part = lanes > 65536 ? launch_q6k_part<LBB, 4, 4>(stream, b, mats, ys, n_jobs, x) : launch_q6k_part<LBB, 2, 4>(stream, b, mats, ys, n_jobs, x);
+            part = lanes > 65536 ? launch_q6k_part<LBB, 4, 4>(stream, b, mats, ys, n_jobs, x, head) : launch_q6k_part<LBB, 2, 4>(stream, b, mats, ys, n_jobs, x, head);
         };
         if (lanes <= 131072) {
             switch (lb) {
@@ -382,29 +411,47 @@ static hipError_t launch_gemv_q6k(hipStream_t stream, const MatView *mats, float
             case 8: small(std::integral_constant<int, 8>{}); break;
             case 16: small(std::integral_constant<int, 16>{}); break;
             case 32: small(std::integral_constant<int, 32>{}); break;
-            default: part = launch_q6k_part<64, 4, 8>(stream, b, mats, ys, n_jobs, x); break;
+            default: part = launch_q6k_part<64, 4, 8>(stream, b, mats, ys, n_jobs, x, head); break;
             }
         } else if (lb == 16 && lanes >= 1000000) {
-            part = launch_q6k_part<16, 8, 4>(stream, b, mats, ys, n_jobs, x);
+            part = launch_q6k_part<16, 8, 4>(stream, b, mats, ys, n_jobs, x, head);
         }
         if (part == hipSuccess) continue;
         if (part != hipErrorInvalidValue) return part;
         const uint32_t rgs = fill_unit_jobs(b, mats, ys, n_jobs, x, 64 / lb);
+        if (head) head->set(b);
         const size_t lds = (size_t)(64 * (lb * 4 + 4)) * sizeof(float);
         if (lds > g_lds_limit) return hipErrorInvalidValue;
         hipError_t e;
         switch (lb) {
-        case 1: e = launch_q6k_lb<1, 4>(stream, b, rgs, lds); break;
-        case 2: e = launch_q6k_lb<2, 4>(stream, b, rgs, lds); break;
-        case 4: e = launch_q6k_lb<4, 4>(stream, b, rgs, lds); break;
-        case 8: e = launch_q6k_lb<8, 4>(stream, b, rgs, lds); break;
-        case 16: e = launch_q6k_lb<16, 4>(stream, b, rgs, lds); break;
-        case 32: e = launch_q6k_lb<32, 8>(stream, b, rgs, lds); break;
-        default: e = launch_q6k_lb<64, 16>(stream, b, rgs, lds); break;  // measured 7 % faster than 8 wavefronts
+        case 1: e = launch_q6k_lb<1, 4>(stream, b, rgs, lds, head); break;
+        case 2: e = launch_q6k_lb<2, 4>(stream, b, rgs, lds, head); break;
+        case 4: e = launch_q6k_lb<4, 4>(stream, b, rgs, lds, head); break;
+        case 8: e = launch_q6k_lb<8, 4>(stream, b, rgs, lds, head); break;
+        case 16: e = launch_q6k_lb<16, 4>(stream, b, rgs, lds, head); break;
+        case 32: e = launch_q6k_lb<32, 8>(stream, b, rgs, lds, head); break;
+        default: e = launch_q6k_lb<64, 16>(stream, b, rgs, lds, head); break;  // measured 7 % faster than 8 wavefronts
         }
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+uint32_t head_candidates(const MatView &m) {
+    if (m.type != T_Q6_K || m.rows == 0) return 0;
+    Q6kHead head;
+    float *y = nullptr;
+    return launch_gemv_q6k(nullptr, &m, &y, 1, nullptr, false, &head) == hipSuccess ? head.groups : 0;
+}
+hipError_t launch_head(hipStream_t stream, const MatView &m, const float *x, const float *norm_w, float eps, float *y, float *cand_v,
+                       uint32_t *cand_i) {
+    if (m.type != T_Q6_K || !cand_v || !cand_i) return hipErrorInvalidValue;
+    Q6kHead head;
+    head.norm_w = norm_w;
+    head.eps = eps;
+    head.cand_v = cand_v;
+    head.cand_i = cand_i;
+    return launch_gemv_q6k(stream, &m, &y, 1, x, false, &head);
 }
 
 template <uint32_t T, int LBB, int PL, int NW>
@@ -1219,6 +1266,7 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     }
     if (ep.kind == ACT_EPILOGUE_ADD_DEFER && (!ep.residual || !ep.partial || tokens > ACT_DEFER_MAX_TOKENS || ep.next_act || ep.xn_out))
         return hipErrorInvalidValue;
+    if (ep.kind == ACT_EPILOGUE_ARGMAX && (!ep.y || !ep.cand_v || !ep.cand_i || ep.n_cand == 0)) return hipErrorInvalidValue;
     if (ep.kind == ACT_EPILOGUE_SWIGLU && (!ep.next_act || tiled[1].rows != rows)) return hipErrorInvalidValue;
     if (norm && p.tt == 2) return hipErrorInvalidValue;  // cannot happen up to ACT_DEFER_MAX_TOKENS tokens
 
@@ -1278,6 +1326,11 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     auto shares = [&](uint32_t j) { return b.job[j].ksplit > 1 ? b.job[j].part : b.job[j].y; };
     auto count = [&](uint32_t j) { return b.job[j].ksplit > 1 ? b.job[j].ksplit : 1u; };
     const uint32_t nt = ep.next_act ? ep.next_type : (uint32_t)T_Q8_0;  // without next activations the column order is never used
+    if (ep.kind == ACT_EPILOGUE_ARGMAX) {
+        hipLaunchKernelGGL(mm_epi_argmax_kernel, dim3(ep.n_cand, tokens), dim3(256), 0, stream, shares(0), count(0), total, rows, ep.y,
+                           ep.cand_v, ep.cand_i);
+        return hipGetLastError();
+    }
     if (ep.kind == ACT_EPILOGUE_ADD_DEFER) {
         hipLaunchKernelGGL(mm_epi_add_partial_kernel, dim3(tokens, 4), dim3(256), 0, stream, shares(0), count(0), total, rows,
                            ep.residual, ep.partial);

@@ -32,6 +32,7 @@
 #include "../../include/native_hip.h"
 #include "../../include/native_hip_llama.h"
 #include "gguf.h"
+#include "head_step.h"
 #include "host_pool.h"
 
 namespace {

@@ -405,3 +405,48 @@ def test_paired_swiglu_is_refused_where_it_is_not_built(pkg):
         gpu.synchronize()
         assert set(dh.to_numpy(np.uint8).tolist()) == {0x5a}
     gpu.close()
+
+
+@pytest.mark.parametrize("n_embd,n_vocab,embd_type", [(256, 38, 12), (512, 2048, 14), (1024, 40000, 8), (2048, 9000, 2), (8192, 700, 1), (16384, 300, 6),
+                                                      (4096, 62600, 7)])
+def test_output_head_with_its_norm_and_candidates(pkg, llama, tmp_path, monkeypatch, n_embd, n_vocab, embd_type):
+    """One vocabulary and width per kernel and part size of the Q6_K head: logits and tokens of a session whose norm,
+    product and argmax are launches of their own.  The head's second half repeats its first, so every logit has an equal one
+    n_vocab / 2 rows on, which must never be picked."""
+    path = tmp_path / "head.gguf"
+    llama.write_synthetic_llama(path, n_layer=1, n_embd=n_embd, n_head=n_embd // 128, n_head_kv=1, n_ff=256, n_vocab=n_vocab,
+                                embd_type=embd_type, seed=n_vocab, weight_std=0.05)
+    blob = np.fromfile(path, np.uint8)
+    (start, end), = [(s, e) for name, _, _, s, e in llama.gguf_tensors(blob) if name == "output.weight"]
+    half = (end - start) // 2
+    blob[start + half:end] = blob[start:start + half]
+    m = llama.Llama(blob=blob)
+    prompt = np.random.default_rng(n_vocab).integers(0, n_vocab, 2).tolist()
+    fused = m.session(device_positions=24)
+    logits = fused.forward(prompt)
+    tokens = m.session(device_positions=24).generate_greedy(prompt, 10)[0].tolist()
+    monkeypatch.setenv("LLAMA_HIP_DECODE_UNFUSED", "1")
+    assert logits_close(logits, m.session(device_positions=24).forward(prompt))
+    assert tokens == m.session(device_positions=24).generate_greedy(prompt, 10)[0].tolist()
+    assert max(tokens) < n_vocab // 2 and tokens[0] == llama.argmax(logits)
+
+
+@pytest.mark.parametrize("n_new", [1, 7, 8, 9, 16, 17])
+def test_steps_replayed_together_equal_single_steps(pkg, llama, tmp_path, monkeypatch, n_new):
+    """Step counts around the eight that one replay holds, of both kinds of device session, against the same steps
+    enqueued kernel by kernel; a second run continues where the first stopped."""
+    path = tmp_path / "steps.gguf"
+    llama.write_synthetic_llama(path, n_layer=2, n_embd=256, n_head=4, n_head_kv=2, n_ff=512, n_vocab=512, seed=4, weight_std=0.1)
+    m = llama.Llama(path=path)
+    rng = np.random.default_rng(n_new)
+    prompts = [rng.integers(0, 512, n).astype(np.uint32) for n in (2, 5, 11)]
+
+    def run():
+        one, several = m.session(device_positions=64), m.batch_session(3, 64)
+        out = [one.generate_greedy(prompts[1].tolist(), n_new)[0].tolist()]
+        out.append(one.generate_greedy([out[0][-1]], n_new)[0].tolist())
+        return out + several.generate_greedy(prompts, n_new)[0].tolist()
+
+    replayed = run()
+    monkeypatch.setenv("LLAMA_HIP_DECODE_EAGER", "1")
+    assert replayed == run()
