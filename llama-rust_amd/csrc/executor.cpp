@@ -959,6 +959,16 @@ int head_act_device(lnh_exec *e, const lnh_matrix *m, const lnh_act *x, size_t t
     return gemm_act(e, 1, &m, x, nullptr, tokens, &dy, LNH_EPILOGUE_NONE, nullptr, nullptr, 0.f, nullptr, nullptr, stream, &ep);
 }
 
+int router_device(lnh_exec *e, const lnh_matrix *m, size_t tokens, const float *x, float *x_device, float *logits, void *stream) {
+    size_t inputs, outputs;
+    const int rc = check_gemm(e, m, tokens, false, 0, 0, &inputs, &outputs);
+    if (rc != LNH_OK) return rc;
+    if (!x || !x_device || !logits) return fail(e, LNH_ERR_INVALID, "buffer pointer is null");
+    if (!skinny_takes(m->view)) return LNH_ERR_UNSUPPORTED;
+    const hipError_t h = launch_skinny(stream ? static_cast<hipStream_t>(stream) : e->stream, m->view, (uint32_t)tokens, x, x_device, logits);
+    return h == hipSuccess ? LNH_OK : hip_fail(e, h, "HIP kernel launch");
+}
+
 }  // namespace nh
 
 extern "C" {

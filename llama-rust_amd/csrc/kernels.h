@@ -71,6 +71,10 @@ struct ActEpilogue {
     float *y = nullptr, *cand_v = nullptr;  // ARGMAX: the rows, and n_cand candidates of each
     uint32_t *cand_i = nullptr, n_cand = 0;
 };
+// F32 / F16 weights of a few rows (a router): y = W x, and the rows of x to x_copy where that is not null.  x and y may lie in
+// pinned host memory.
+bool skinny_takes(const MatView &m);
+hipError_t launch_skinny(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *x_copy, float *y);
 // y = W rmsnorm(x) * norm_w for one token, and the largest output of each of head_candidates(m) workgroups with its row.
 // head_candidates: 0 where no such launch exists (then launch_head is hipErrorInvalidValue).
 uint32_t head_candidates(const MatView &m);

@@ -1006,6 +1006,16 @@ static hipError_t launch_pg(hipStream_t stream, const MatView &m, uint32_t token
     return hipGetLastError();
 }
 
+bool skinny_takes(const MatView &m) { return (m.type == T_F32 || m.type == T_F16) && m.rows <= SKINNY_ROWS; }
+hipError_t launch_skinny(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *x_copy, float *y) {
+    if (!skinny_takes(m) || m.rows == 0 || tokens == 0) return hipErrorInvalidValue;
+    void (*kern)(MatView, const float *, float *, float *);
+    if (m.type == T_F32) kern = m.rows <= 8 ? gemm_skinny_kernel<T_F32, 8> : gemm_skinny_kernel<T_F32, 16>;
+    else kern = m.rows <= 8 ? gemm_skinny_kernel<T_F16, 8> : gemm_skinny_kernel<T_F16, 16>;
+    hipLaunchKernelGGL(kern, dim3(tokens), dim3(256), 0, stream, m, x, x_copy, y);
+    return hipGetLastError();
+}
+
 // Single-token products, and whatever the other paths do not take.
 static hipError_t launch_plain(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *y) {
     auto run = [&](auto tag) -> hipError_t {
@@ -1070,7 +1080,7 @@ size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_
         if (tokens[g] == 0 || mats[g].rows == 0) { g++; continue; }
         const uint32_t run = mm_run(mats, tokens, n, g);
         if (run == 0) {
-            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
+            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1 && !skinny_takes(mats[g])) {
                 size_t bytes;
                 FgPlan f;
                 fg_plan(mats[g], tokens[g], f);
@@ -1112,7 +1122,8 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
                 for (uint32_t t = 0; t < tokens[g] && e == hipSuccess; t++)
                     e = launch_plain(stream, mats[g], 1, xs[g] + (size_t)t * mats[g].cols, ys[g] + (size_t)t * mats[g].rows);
             } else if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
-                e = pg_takes(mats[g], tokens[g]) ? launch_pg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes)
+                if (skinny_takes(mats[g])) e = launch_skinny(stream, mats[g], tokens[g], xs[g], nullptr, ys[g]);
+                else e = pg_takes(mats[g], tokens[g]) ? launch_pg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes)
                                                 : launch_fg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes);
             } else {
                 e = launch_plain(stream, mats[g], tokens[g], xs[g], ys[g]);

@@ -750,7 +750,11 @@ int expert_products(lnm_model *m, std::vector<Mat> &parts, const std::vector<siz
 __global__ void dd_swiglu_kernel(float *gate, const float *up, uint32_t n);  // with the device session's kernels below
 
 // packed[i] = x[row_of[i]]: the rows of every expert's bucket, contiguous (grouped_one_expert, decode.rs:10062-10116).
-__global__ __launch_bounds__(256) void moe_gather_kernel(const float *x, const uint32_t *row_of, uint32_t d, float *packed) {
+// row_of and the n_rest words behind it lie in pinned host memory; the first workgroups leave the latter on the device.
+__global__ __launch_bounds__(256) void moe_gather_kernel(const float *x, const uint32_t *row_of, uint32_t d, float *packed, uint32_t *rest,
+                                                         uint32_t n_rest) {
+    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+    if (r < n_rest) rest[r] = row_of[gridDim.x + r];
     const float4 *src = reinterpret_cast<const float4 *>(x + (size_t)row_of[blockIdx.x] * d);
     float4 *dst = reinterpret_cast<float4 *>(packed + (size_t)blockIdx.x * d);
     for (uint32_t i = threadIdx.x; i < d / 4; i += blockDim.x) dst[i] = src[i];
@@ -853,21 +857,33 @@ int moe_ffn_on_device(lnm_model *m, Layer &l, size_t n, const float *x, float *f
             if (armed) (void)hipStreamSynchronize(s);
         }
     } drain{ms->stream, true};
-    // rows up, router product, logits back
-    std::memcpy(ms->h_io, x, n * d * sizeof(float));
-    e = hipMemcpyAsync(ms->d_io, ms->h_io, n * d * sizeof(float), hipMemcpyHostToDevice, ms->stream);
-    if (e != hipSuccess) return hip_fail(e);
+    // rows up, router product, logits back.  Where the router is a few rows of plain weights, launches that read the pinned rows,
+    // leave them on the device and write the pinned logits: one for every 256 KB, which the GPU reads while the next are copied.
     if (ensure_resident(m, l.gate_inp) != 0) return 1;
-    if (lnh_gemm_device(m->exec, l.gate_inp.resident, n, ms->d_io, d_logits, ms->stream) != 0)
+    const size_t piece = d < 65536 ? 65536 / d : 1;
+    int routed = LNH_OK;
+    for (size_t t = 0; t < n && routed == LNH_OK; t += piece) {
+        const size_t rows = n - t < piece ? n - t : piece;
+        std::memcpy(ms->h_io + t * d, x + t * d, rows * d * sizeof(float));
+        routed = nh::router_device(m->exec, l.gate_inp.resident, rows, ms->h_io + t * d, ms->d_io + t * d, h_logits + t * ne, ms->stream);
+    }
+    if (routed == LNH_ERR_UNSUPPORTED) {
+        std::memcpy(ms->h_io, x, n * d * sizeof(float));
+        e = hipMemcpyAsync(ms->d_io, ms->h_io, n * d * sizeof(float), hipMemcpyHostToDevice, ms->stream);
+        if (e != hipSuccess) return hip_fail(e);
+        if (lnh_gemm_device(m->exec, l.gate_inp.resident, n, ms->d_io, d_logits, ms->stream) != 0)
+            return fail(std::string(lnh_last_error(m->exec)) + " (" + l.gate_inp.name + ")");
+        e = hipMemcpyAsync(h_logits, d_logits, n * ne * sizeof(float), hipMemcpyDeviceToHost, ms->stream);
+    } else if (routed != LNH_OK) {
         return fail(std::string(lnh_last_error(m->exec)) + " (" + l.gate_inp.name + ")");
-    e = hipMemcpyAsync(h_logits, d_logits, n * ne * sizeof(float), hipMemcpyDeviceToHost, ms->stream);
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(ms->stream);
     if (e != hipSuccess) return hip_fail(e);
     ms->logits.assign(h_logits, h_logits + n * ne);
     std::vector<size_t> counts;
-    size_t routed = 0;
-    if (moe_route(hp, n, ms, &counts, &routed)) return 1;
-    if (routed != pairs) return fail("routed feed-forward: the buckets do not hold k selections per token");
+    size_t selected = 0;
+    if (moe_route(hp, n, ms, &counts, &selected)) return 1;
+    if (selected != pairs) return fail("routed feed-forward: the buckets do not hold k selections per token");
 
     // bucket order: the row of every packed position; per token its selections in ascending expert order
     std::vector<uint32_t> filled(n, 0);
@@ -884,8 +900,6 @@ int moe_ffn_on_device(lnm_model *m, Layer &l, size_t n, const float *x, float *f
             at++;
         }
     }
-    e = hipMemcpyAsync(d_idx, h_idx, (n_idx + n * k) * sizeof(float), hipMemcpyHostToDevice, ms->stream);  // indices and weights are adjacent
-    if (e != hipSuccess) return hip_fail(e);
     std::vector<const lnh_matrix *> hg, hu, hdn;
     std::vector<size_t> toks;
     for (size_t ex = 0; ex < ne; ex++) {
@@ -897,7 +911,10 @@ int moe_ffn_on_device(lnm_model *m, Layer &l, size_t n, const float *x, float *f
         hdn.push_back(l.down_e[ex].resident);
         toks.push_back(counts[ex]);
     }
-    hipLaunchKernelGGL(moe_gather_kernel, dim3((uint32_t)pairs), dim3(256), 0, ms->stream, ms->d_io, d_idx, (uint32_t)d, ms->d_x);
+    // (n_idx + n k - pairs words behind the rows: the slots and the weights, adjacent; a workgroup per pair takes 256 of them)
+    static_assert(sizeof(float) == sizeof(uint32_t), "weights travel as words");
+    hipLaunchKernelGGL(moe_gather_kernel, dim3((uint32_t)pairs), dim3(256), 0, ms->stream, ms->d_io, h_idx, (uint32_t)d, ms->d_x, d_idx + pairs,
+                       (uint32_t)(2 * n * k));
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e);
     {
         // gate and up of every expert as one batch: the experts of at most 16 rows first, then the others, so that
@@ -931,10 +948,9 @@ int moe_ffn_on_device(lnm_model *m, Layer &l, size_t n, const float *x, float *f
     if (lnh_gemm_grouped_device(m->exec, hdn.size(), hdn.data(), toks.data(), ms->d_g, ms->d_y, ms->stream) != 0)
         return fail(std::string(lnh_last_error(m->exec)) + " (" + l.down_e[0].name + ")");
     hipLaunchKernelGGL(moe_scatter_kernel, dim3((uint32_t)n, (uint32_t)((d + 1023) / 1024)), dim3(256), 0, ms->stream, ms->d_y,
-                       d_idx + pairs, d_w, (uint32_t)k, (uint32_t)d, ms->d_io);
+                       d_idx + pairs, d_w, (uint32_t)k, (uint32_t)d, ms->h_io);  // straight into the pinned rows
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e);
-    e = hipMemcpyAsync(ms->h_io, ms->d_io, n * d * sizeof(float), hipMemcpyDeviceToHost, ms->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ms->stream);
+    e = hipStreamSynchronize(ms->stream);
     if (e != hipSuccess) return hip_fail(e);
     drain.armed = false;  // the stream is idle
     std::memcpy(ffn_out, ms->h_io, n * d * sizeof(float));

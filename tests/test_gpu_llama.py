@@ -131,6 +131,23 @@ def test_small_model_with_experts_generates_the_same_tokens_as_the_cpu_path(pkg,
     assert len(set(toks_c)) >= 15  # the layers matter: no fixed point, no short cycle
 
 
+@pytest.mark.parametrize("n_expert,n_embd,tokens", [(4, 256, 3), (16, 1024, 70), (17, 512, 33)])
+def test_routed_layer_in_pieces_equals_the_cpu_products(pkg, llama, tmp_path, n_expert, n_embd, tokens):
+    """moe_ffn alone: a router that fits the one-launch product in one piece and in two (70 rows of 1024: 64 + 6), and one of
+    more rows, whose input is copied first; more than eight products of a kind in a launch."""
+    path = tmp_path / "moe.gguf"
+    llama.write_synthetic_llama(path, n_layer=1, n_embd=n_embd, n_head=4, n_head_kv=2, n_ff=512, n_vocab=64, block_type=12, embd_type=8,
+                                output_type=8, seed=n_expert, weight_std=0.06, n_expert=n_expert, n_expert_used=2)
+    x = np.random.default_rng(n_expert).normal(0, 1, (tokens, n_embd)).astype(np.float32)
+    cpu = llama.Llama(path=path, products=llama.CALLBACK,
+                      matmul=lambda ty, n_rows, n_cols, n_tokens, w, v: oracle.gemm(ty, n_cols, n_tokens, w, v, n_rows))
+    gpu = llama.Llama(path=path)
+    for _ in range(2):  # the second call reuses the first one's buffers
+        got, want = gpu.moe_ffn(0, x), cpu.moe_ffn(0, x)
+        assert float(np.abs(got - want).max()) <= 1e-4 * float(np.abs(want).max())
+        x = x[::-1].copy()
+
+
 @pytest.mark.parametrize("kind", ["f32", "q4_0", "q4_k", "experts"])
 def test_reference_session_scenario_on_every_path(pkg, llama, tmp_path, kind):
     """langtax/tests/native_cuda_parity.rs:198-249 for its four tiny models (F32, Q4_0, Q4_K weights, a model

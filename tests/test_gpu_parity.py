@@ -430,6 +430,20 @@ def test_plain_dtypes_on_the_matrix_cores_every_tile_and_share_shape(pkg, gpu, t
 
 
 @pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,tokens", [(1, 1, 2), (3, 7, 5), (8, 4096, 64), (8, 4099, 3), (9, 4100, 17), (16, 1023, 2), (16, 8196, 130), (17, 64, 9)])
+def test_plain_dtypes_of_a_few_rows(gpu, ty, rows, cols, tokens):
+    """Routers: up to 16 rows take one launch whatever the tokens; columns that fill no vector, one more row than that."""
+    rng = np.random.default_rng(rows * cols + tokens)
+    w = K.random_packed(ty, rows, cols, rng)
+    x = rng.normal(0, 1, tokens * cols).astype(np.float32)
+    m = gpu.upload_packed(ty, rows, cols, w)
+    y = np.full(tokens * rows, np.nan, np.float32)
+    gpu.gemm_resident(m, tokens, x, y)
+    check(y, ty, cols, tokens, rows, w, x)
+    m.close()
+
+
+@pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("rows,cols,tokens", [(4100, 333, 300), (8200, 330, 257), (4097, 1032, 65), (2050, 8, 33), (4224, 8192, 20),
                                               (3000, 2050, 129), (128, 520, 64), (1, 32, 400), (9000, 64, 513)])
 def test_plain_dtypes_cut_into_bf16_parts(pkg, gpu, ty, rows, cols, tokens):
