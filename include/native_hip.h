@@ -126,7 +126,8 @@ int lnh_gemm_grouped(lnh_exec *exec, size_t n_groups, const lnh_matrix *const *m
  * gemm calls on the same activations at langtax/src/decode.rs:2754-2790 (q, k, v) and
  * 2968-2979 (gate, up).  x holds tokens * cols floats (all matrices have the same column
  * count); y receives the products back to back, matrix after matrix (tokens * rows[i] each).
- * One input copy, one launch for single-token calls, one output copy. */
+ * One input, one launch for single-token calls, one output.  How a launch cuts its rows follows its total size, so a sum may
+ * be taken in another order (other last bits) than in a call of its own. */
 int lnh_gemm_shared(lnh_exec *exec, size_t n_mats, const lnh_matrix *const *mats, size_t tokens, const float *x,
                     size_t x_len, float *y, size_t y_len);
 

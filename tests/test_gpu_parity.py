@@ -979,6 +979,44 @@ def test_shared_input_products_equal_separate_calls(pkg, gpu):
 
 
 # ------------------------------------------------------------------ residency
+@pytest.mark.parametrize("ty,rows_list,cols,tokens", [(K.Q4_K, (1000, 24), 8192, 1), (K.Q8_0, (333,), 8224, 1), (K.Q4_0, (70,), 4096, 2),
+                                                      (K.F16, (130,), 4128, 2), (K.Q6_K, (9,), 16640, 1), (K.F32, (17, 40), 903, 1),
+                                                      (K.Q5_1, (20000, 480), 512, 1), (K.Q4_K, (50,), 512, 3)])
+def test_host_calls_on_both_sides_of_reading_and_writing_pinned_memory(pkg, gpu, ty, rows_list, cols, tokens):
+    """Products whose kernels read x from and write y to pinned memory, and those that still copy one or both: the caller's
+    arrays ordinary, and pinned (then the largest y is written in place).  Twice each, with other inputs."""
+    import ctypes
+    rt = importlib.import_module("llama-rust_amd.hiprt").rt()
+    rt.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+    rt.hipHostFree.argtypes = [ctypes.c_void_p]
+
+    def pinned(n):
+        p = ctypes.c_void_p()
+        assert rt.hipHostMalloc(ctypes.byref(p), 4 * n, 0) == 0
+        return p, np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (n,))
+
+    rng = np.random.default_rng(cols + tokens)
+    ws = [K.random_packed(ty, r, cols, rng, scale=0.02) for r in rows_list]
+    mats = [gpu.upload_packed(ty, r, cols, w) for r, w in zip(rows_list, ws)]
+    (xp, x_pinned), (yp, y_pinned) = pinned(tokens * cols), pinned(tokens * sum(rows_list))
+    for _ in range(2):
+        x = rng.normal(0, 1, tokens * cols).astype(np.float32)
+        x_pinned[:] = x
+        ordinary = np.full(tokens * sum(rows_list), np.nan, np.float32)
+        y_pinned[:] = np.nan
+        gpu.gemm_shared(mats, tokens, x, ordinary)
+        gpu.gemm_shared(mats, tokens, x_pinned, y_pinned)
+        assert ordinary.view(np.uint32).tolist() == y_pinned.view(np.uint32).tolist()
+        off = 0
+        for r, w in zip(rows_list, ws):
+            check(ordinary[off:off + tokens * r], ty, cols, tokens, r, w, x)
+            off += tokens * r
+    for p in (xp, yp):
+        rt.hipHostFree(p)
+    for m in mats:
+        m.close()
+
+
 def test_residency_lru_and_budget(pkg, monkeypatch):
     """langtax/src/native_gpu.rs:161-211: hit moves to the back, admission evicts from the front,
     an over-budget matrix runs once and is not kept, budget 0 disables residency but not the GPU."""
