@@ -268,12 +268,21 @@ static hipError_t launch_gemv_q4k_pro(hipStream_t stream, const MatView *mats, f
         const uint32_t units = win.count(w, nb);
         uint32_t lbb = 1;  // super-blocks per row, rounded up to a power of two
         while (lbb < 64 && lbb < units) lbb <<= 1;
-        // Two lanes per super-block for matrices that would otherwise give the chip fewer than about ten
-        // wavefront steps per CU (measured crossover: 8192 x 4096 gains 11 %, 12288 x 4096 loses 6 %).
+        // Several lanes per super-block for matrices that would otherwise give the chip few wavefront steps per CU.
+        // Quarters up to two (alone on the card, quarters against halves: 512 x 256 2.27 against 2.53 us, 512 x 4096
+        // 2.79 against 3.04, 2048 x 4096 = two steps 3.40 against 3.50; up to five steps they still gain 1 to 3 %
+        // alone, but beside other work they take from it: decode steps of three streams at once, each with a
+        // 4096 x 4096 product per layer = four steps, 962 against 921 us); halves up to ten (8192 x 4096 gains 11 %
+        // over whole blocks, 12288 x 4096 loses 6 %).  Rows of 17 to 32 super-blocks have room for halves only, up to
+        // four steps (512 x 5632 3.30 against 4.49 us, 2048 x 8192 4.55 against 5.08, 2560 x 7168 = five steps
+        // 5.14 against 5.14, 4096 x 8192 6.60 against 6.37).  Rows of one super-block are never taken whole: that
+        // variant spilled (262144 x 256 120 -> 12 us).  The pair epilogue stays with the halves and with the shapes that it took with them.
         size_t full_steps = 0;
         for (uint32_t j = 0; j < n_jobs; j++) full_steps += (mats[j].rows + 64 / lbb - 1) / (64 / lbb);
-        const bool halves = lbb <= 16 && full_steps <= (size_t)10 * g_cu_count;
-        const uint32_t lb = halves ? 2 * lbb : lbb;
+        const size_t cus = g_cu_count;
+        const uint32_t parts = lbb <= 16 ? (full_steps <= 2 * cus && !pro.pair ? 4 : full_steps <= 10 * cus || lbb == 1 ? 2 : 1)
+                                         : (lbb == 32 && full_steps <= 4 * cus ? 2 : 1);
+        const uint32_t lb = parts * lbb;
         GemvBatch b;
         const uint32_t rgs = fill_unit_jobs(b, mats, ys, n_jobs, x, 64 / lb);
         b.unit0 = win.first(w);
@@ -283,21 +292,29 @@ static hipError_t launch_gemv_q4k_pro(hipStream_t stream, const MatView *mats, f
         b.eps = pro.eps;
         b.pair = pro.pair ? 1u : 0u;
         // x slots, the sub-block sums of x, and room for one partial sum per wavefront (RMSNorm prologue)
-        const size_t lds = (size_t)(64 * (lbb * 4 + 4) + lbb * 8 + 16) * sizeof(float);
+        const size_t lds = (size_t)(64 * (lbb * 4 + 4) + (parts > 1 ? parts * lbb * 4 : 0) + lbb * 8 + 16) * sizeof(float);
         if (lds > g_lds_limit) return hipErrorInvalidValue;
         hipError_t e;
-        if (halves) {
+        if (parts == 4) {
+            switch (lbb) {
+            case 1: e = launch_q4k_lb<4, 4, 2, PRO>(stream, b, rgs, lds); break;
+            case 2: e = launch_q4k_lb<8, 4, 2, PRO>(stream, b, rgs, lds); break;
+            case 4: e = launch_q4k_lb<16, 4, 2, PRO>(stream, b, rgs, lds); break;
+            case 8: e = launch_q4k_lb<32, 4, 2, PRO>(stream, b, rgs, lds); break;
+            default: e = launch_q4k_lb<64, 4, 2, PRO>(stream, b, rgs, lds); break;
+            }
+        } else if (parts == 2) {
             switch (lb) {
             case 2: e = launch_q4k_lb<2, 4, 4, PRO>(stream, b, rgs, lds); break;
             case 4: e = launch_q4k_lb<4, 4, 4, PRO>(stream, b, rgs, lds); break;
             case 8: e = launch_q4k_lb<8, 4, 4, PRO>(stream, b, rgs, lds); break;
             case 16: e = launch_q4k_lb<16, 4, 4, PRO>(stream, b, rgs, lds); break;
-            default: e = launch_q4k_lb<32, 4, 4, PRO>(stream, b, rgs, lds); break;
+            case 32: e = launch_q4k_lb<32, 4, 4, PRO>(stream, b, rgs, lds); break;
+            default: e = launch_q4k_lb<64, 4, 4, PRO>(stream, b, rgs, lds); break;
             }
         } else {
             switch (lb) {
             // Short rows: small workgroups, so that even a 1024-row matrix spreads over every CU.
-            case 1: e = launch_q4k_lb<1, 4, 8, PRO>(stream, b, rgs, lds); break;
             case 2: e = launch_q4k_lb<2, 4, 8, PRO>(stream, b, rgs, lds); break;
             case 4: e = launch_q4k_lb<4, 4, 8, PRO>(stream, b, rgs, lds); break;
             case 8: e = launch_q4k_lb<8, 4, 8, PRO>(stream, b, rgs, lds); break;

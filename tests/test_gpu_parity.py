@@ -570,6 +570,8 @@ _SINGLE_TOKEN = {
             (5, _LONG), (5, _LONG + 8)],
     K.Q6_K: [(1, 256), (3, 512), (63, 1280), (257, 2304), (100, 4352), (31, 8448), (7, 16384), (9, 16640), (65537, 256), (131073, 256),
              (4097, 4096), (8193, 4096), (2049, 8192), (2048, 11008), (2049, 16384), (62501, 4096)],
+    K.Q4_K: [(1, 256), (3, 512), (5, 768), (63, 1280), (257, 2304), (100, 4352), (31, 8448), (3, 16640), (81921, 256), (163841, 256),
+             (2048, 4096), (2049, 4096), (10241, 4096), (2048, 7168), (2049, 7168), (2048, 8192)],
 }
 _BLOCKS = [(1, 32), (3, 96), (64, 288), (63, 512 + 32), (2049, 4064), (2047, 4128), (8191, 4128), (8192, 4128), (8191, 480), (8192, 480),
            (8193, 576), (5, _LONG - 32 * 20 - 32), (3, _LONG + 32)]  # rows that are not whole units
@@ -584,7 +586,7 @@ def test_single_token_products_on_both_sides_of_every_rule(pkg, gpu, ty):
         unit = 128 if ty == K.Q8_0 else 256
         shapes = _BLOCKS + [(r, n * unit) for r, n in _UNITS]
     else:
-        shapes = _SINGLE_TOKEN.get(ty, [(1, 256), (5, 768), (2049, 4096), (3, 16640)])
+        shapes = _SINGLE_TOKEN[ty]
     rng = np.random.default_rng(70 + ty)
     for rows, cols in shapes:
         w = K.random_packed(ty, rows, cols, rng, scale=0.02)
