@@ -269,10 +269,10 @@ static hipError_t launch_gemv_q4k_pro(hipStream_t stream, const MatView *mats, f
         uint32_t lbb = 1;  // super-blocks per row, rounded up to a power of two
         while (lbb < 64 && lbb < units) lbb <<= 1;
         // Several lanes per super-block for matrices that would otherwise give the chip few wavefront steps per CU.
-        // Quarters up to two (alone on the card, quarters against halves: 512 x 256 2.27 against 2.53 us, 512 x 4096
-        // 2.79 against 3.04, 2048 x 4096 = two steps 3.40 against 3.50; up to five steps they still gain 1 to 3 %
-        // alone, but beside other work they take from it: decode steps of three streams at once, each with a
-        // 4096 x 4096 product per layer = four steps, 962 against 921 us); halves up to ten (8192 x 4096 gains 11 %
+        // Quarters below one (alone on the card, quarters against halves: 512 x 256 2.27 against 2.53 us, 512 x 4096
+        // 2.79 against 3.04; up to five steps they still gain 9 to 1 % alone, but a [q,k,v] launch and its three separate
+        // products would add in different orders, and beside other work they take from it: decode steps of three
+        // streams at once, each with a 4096 x 4096 product per layer = four steps, 962 against 921 us); halves up to ten (8192 x 4096 gains 11 %
         // over whole blocks, 12288 x 4096 loses 6 %).  Rows of 17 to 32 super-blocks have room for halves only, up to
         // four steps (512 x 5632 3.30 against 4.49 us, 2048 x 8192 4.55 against 5.08, 2560 x 7168 = five steps
         // 5.14 against 5.14, 4096 x 8192 6.60 against 6.37).  Rows of one super-block are never taken whole: that
@@ -280,7 +280,7 @@ static hipError_t launch_gemv_q4k_pro(hipStream_t stream, const MatView *mats, f
         size_t full_steps = 0;
         for (uint32_t j = 0; j < n_jobs; j++) full_steps += (mats[j].rows + 64 / lbb - 1) / (64 / lbb);
         const size_t cus = g_cu_count;
-        const uint32_t parts = lbb <= 16 ? (full_steps <= 2 * cus && !pro.pair ? 4 : full_steps <= 10 * cus || lbb == 1 ? 2 : 1)
+        const uint32_t parts = lbb <= 16 ? (full_steps < cus && !pro.pair ? 4 : full_steps <= 10 * cus || lbb == 1 ? 2 : 1)
                                          : (lbb == 32 && full_steps <= 4 * cus ? 2 : 1);
         const uint32_t lb = parts * lbb;
         GemvBatch b;

@@ -571,7 +571,7 @@ _SINGLE_TOKEN = {
     K.Q6_K: [(1, 256), (3, 512), (63, 1280), (257, 2304), (100, 4352), (31, 8448), (7, 16384), (9, 16640), (65537, 256), (131073, 256),
              (4097, 4096), (8193, 4096), (2049, 8192), (2048, 11008), (2049, 16384), (62501, 4096)],
     K.Q4_K: [(1, 256), (3, 512), (5, 768), (63, 1280), (257, 2304), (100, 4352), (31, 8448), (3, 16640), (81921, 256), (163841, 256),
-             (2048, 4096), (2049, 4096), (10241, 4096), (2048, 7168), (2049, 7168), (2048, 8192)],
+             (1020, 4096), (1021, 4096), (10241, 4096), (2048, 7168), (2049, 7168), (2048, 8192)],
 }
 _BLOCKS = [(1, 32), (3, 96), (64, 288), (63, 512 + 32), (2049, 4064), (2047, 4128), (8191, 4128), (8192, 4128), (8191, 480), (8192, 480),
            (8193, 576), (5, _LONG - 32 * 20 - 32), (3, _LONG + 32)]  # rows that are not whole units
