@@ -272,11 +272,12 @@ static hipError_t launch_gemv_q4k_pro(hipStream_t stream, const MatView *mats, f
         // Quarters below one (alone on the card, quarters against halves: 512 x 256 2.27 against 2.53 us, 512 x 4096
         // 2.79 against 3.04; up to five steps they still gain 9 to 1 % alone, but a [q,k,v] launch and its three separate
         // products would add in different orders, and beside other work they take from it: decode steps of three
-        // streams at once, each with a 4096 x 4096 product per layer = four steps, 962 against 921 us); halves up to ten (8192 x 4096 gains 11 %
-        // over whole blocks, 12288 x 4096 loses 6 %).  Rows of 17 to 32 super-blocks have room for halves only, up to
-        // four steps (512 x 5632 3.30 against 4.49 us, 2048 x 8192 4.55 against 5.08, 2560 x 7168 = five steps
+        // streams at once, each with a 4096 x 4096 product per layer = four steps, 962 against 921 us).  Halves up to
+        // ten (8192 x 4096 gains 11 % over whole blocks, 12288 x 4096 loses 6 %).  Rows of 17 to 32 super-blocks have
+        // room for halves only, up to four steps (512 x 5632 3.30 against 4.49 us, 2048 x 8192 4.55 against 5.08, 2560 x 7168 = five steps
         // 5.14 against 5.14, 4096 x 8192 6.60 against 6.37).  Rows of one super-block are never taken whole: that
-        // variant spilled (262144 x 256 120 -> 12 us).  The pair epilogue stays with the halves and with the shapes that it took with them.
+        // variant spilled (262144 x 256 120 -> 12 us).  The pair epilogue stays with the halves and with the shapes
+        // that it took with them.
         size_t full_steps = 0;
         for (uint32_t j = 0; j < n_jobs; j++) full_steps += (mats[j].rows + 64 / lbb - 1) / (64 / lbb);
         const size_t cus = g_cu_count;
@@ -1033,6 +1034,40 @@ hipError_t launch_skinny(hipStream_t stream, const MatView &m, uint32_t tokens, 
     return hipGetLastError();
 }
 
+template <uint32_t T, int TM, int NW>
+static hipError_t launch_few_t(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *y, uint32_t per_cu) {
+    const bool vec = m.cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    auto kern = vec ? gemm_few_kernel<T, TM, NW, true> : gemm_few_kernel<T, TM, NW, false>;
+    const uint32_t tiles = (m.rows + 15) / 16, most = per_cu * g_cu_count;
+    hipLaunchKernelGGL(kern, dim3(tiles < most ? tiles : most), dim3(NW * 64), 0, stream, m, tokens, x, y);
+    return hipGetLastError();
+}
+// Rows that give less than three quarters of the CUs a tile take the kernel only while they are short: the tile kernels
+// below share long columns between CUs, and one CU draws about 40 GB/s (F16, 4 tokens, against them: 1024x4096 7.9 / 12.0 us,
+// 1024x8192 13.4 / 13.7, 1024x14336 21.5 / 19.0, with 16 tokens 1024x6144 14.0 / 14.4, 1024x8192 16.7 / 14.9; F32
+// 512x2048 5.9 / 10.6, 1024x6144 with 16 tokens 17.2 / 15.3).  17 to 32 tokens take twice the matrix-core time: 512x3072
+// with 20 11.8 / 13.2 (F32 12.8 / 12.8), F32 512x4096 16.1 / 13.9, F32 4096x4096 with 32 18.7 / 23.3, 4096x14336 59.6 / 55.9.
+static bool few_takes(const MatView &m, uint32_t tokens) {
+    if ((m.type != T_F32 && m.type != T_F16) || tokens < 2 || tokens > 32 || pg_takes(m, tokens) || skinny_takes(m)) return false;
+    const bool wide = (m.rows + 15) / 16 >= (uint32_t)g_cu_count * 3 / 4;
+    if (tokens > 16) return m.cols <= (wide ? 8192u : 3072u);
+    return wide || m.cols <= (m.type == T_F16 ? 6144u : 4096u);
+}
+template <uint32_t T> static hipError_t launch_few(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *y) {
+    // A tile for every CU at most: one workgroup of sixteen wavefronts each; else three of eight, which go on from tile
+    // to tile (F16 4096x14336 with 8 tokens 27.2 against 28.1 us, F32 39.0 against 45.6; 14336x4096 32.3 against 28.3).
+    // 32 slots of x for sixteen wavefronts would not fit the LDS.
+    const bool deep = (m.rows + 15) / 16 <= (uint32_t)g_cu_count;
+    auto run = [&](auto tm) -> hipError_t {
+        constexpr int TM = decltype(tm)::value;
+        return deep ? launch_few_t<T, TM, 16>(stream, m, tokens, x, y, 1) : launch_few_t<T, TM, 8>(stream, m, tokens, x, y, 3);
+    };
+    if (tokens <= 4) return run(std::integral_constant<int, 4>{});
+    if (tokens <= 8) return run(std::integral_constant<int, 8>{});
+    if (tokens <= 16) return run(std::integral_constant<int, 16>{});
+    return launch_few_t<T, 32, 8>(stream, m, tokens, x, y, 1);
+}
+
 // Single-token products, and whatever the other paths do not take.
 static hipError_t launch_plain(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *y) {
     auto run = [&](auto tag) -> hipError_t {
@@ -1097,7 +1132,7 @@ size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_
         if (tokens[g] == 0 || mats[g].rows == 0) { g++; continue; }
         const uint32_t run = mm_run(mats, tokens, n, g);
         if (run == 0) {
-            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1 && !skinny_takes(mats[g])) {
+            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1 && !skinny_takes(mats[g]) && !few_takes(mats[g], tokens[g])) {
                 size_t bytes;
                 FgPlan f;
                 fg_plan(mats[g], tokens[g], f);
@@ -1140,6 +1175,9 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
                     e = launch_plain(stream, mats[g], 1, xs[g] + (size_t)t * mats[g].cols, ys[g] + (size_t)t * mats[g].rows);
             } else if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
                 if (skinny_takes(mats[g])) e = launch_skinny(stream, mats[g], tokens[g], xs[g], nullptr, ys[g]);
+                else if (few_takes(mats[g], tokens[g]))
+                    e = mats[g].type == T_F16 ? launch_few<T_F16>(stream, mats[g], tokens[g], xs[g], ys[g])
+                                              : launch_few<T_F32>(stream, mats[g], tokens[g], xs[g], ys[g]);
                 else e = pg_takes(mats[g], tokens[g]) ? launch_pg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes)
                                                 : launch_fg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes);
             } else {

@@ -601,6 +601,38 @@ def test_single_token_products_on_both_sides_of_every_rule(pkg, gpu, ty):
         m.close()
 
 
+@pytest.mark.parametrize("ty", [K.F32, K.F16], ids=["f32", "f16"])
+def test_plain_products_of_few_tokens(pkg, gpu, ty):
+    """Rows around a tile of 16, around what gives every CU one tile and what makes a workgroup go on to another; columns
+    around a wavefront's step, around what sixteen wavefronts take at once and around the rule that leaves long rows to the
+    other kernels; tokens on both sides of every slot count.  An infinity in one row and in one token stays there."""
+    rng = np.random.default_rng(90 + ty)
+    shapes = [(17, 1), (18, 31), (31, 33), (33, 63), (32, 64), (48, 65), (49, 127), (65, 130), (100, 511), (64, 516), (130, 1025),
+              (35, 2052), (20, 3072), (20, 3073), (20, 4096), (20, 4100), (20, 6144), (20, 6152), (3057, 515), (3073, 8200), (4096, 96), (4097, 68),
+              (12305, 40)]
+    for rows, cols in shapes:
+        w = K.random_packed(ty, rows, cols, rng)
+        m = gpu.upload_packed(ty, rows, cols, w)
+        for tokens in (2, 4, 5, 8, 9, 16, 17, 32) if rows * cols < 1 << 21 else (3, 12, 20):
+            x = rng.normal(0, 1, tokens * cols).astype(np.float32)
+            y = np.full(tokens * rows, np.nan, np.float32)
+            gpu.gemm_resident(m, tokens, x, y)
+            check(y, ty, cols, tokens, rows, w, x, f"{O.TYPE_NAMES[ty]} {rows}x{cols} M={tokens}")
+        m.close()
+    rows, cols, tokens = 50, 70, 6
+    wide, esz = K.random_packed(ty, rows, cols, rng).reshape(rows, -1).copy(), (4 if ty == K.F32 else 2)
+    wide[7] = np.frombuffer(np.full(cols, np.inf, np.float32 if esz == 4 else np.float16).tobytes(), np.uint8)
+    m = gpu.upload_packed(ty, rows, cols, wide.ravel())
+    x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    x[3] = np.inf
+    y = np.zeros(tokens * rows, np.float32)
+    gpu.gemm_resident(m, tokens, x.ravel(), y)
+    m.close()
+    touched = np.zeros((tokens, rows), bool)
+    touched[3], touched[:, 7] = True, True
+    assert np.array_equal(~np.isfinite(y.reshape(tokens, rows)), touched)
+
+
 @pytest.mark.parametrize("rows,cols,tokens", [(1, 256, 33), (255, 512, 64), (256, 768, 65), (257, 4352, 97), (600, 14336, 128),
                                               (4099, 1280, 129)])
 def test_q4_k_products_of_more_than_32_tokens(gpu, rows, cols, tokens):
