@@ -741,7 +741,7 @@ def main():
                          "layer_us_one_launch": round(read_merged_us / args.layers, 2),
                          "layer_note": "a layer's 122.9 MB read by four dependent launches (the products' sizes) and by one: "
                                        "the difference is what the three kernel boundaries inside a layer cost a reader"}},
-        "other_kernels": {"gemv_q6k_kernel (head)": {"achieved": round(head_gbs, 1), "unit": "GB/s",
+        "other_kernels": {"gemv_q6k_part_kernel (head)": {"achieved": round(head_gbs, 1), "unit": "GB/s",
                                                      "frac": round(head_gbs / HBM_PEAK_GBS, 4),
                                                      "launch_us": round(head_ms * 1e3, 2)}},
     }
