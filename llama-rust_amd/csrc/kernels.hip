@@ -1045,13 +1045,20 @@ static hipError_t launch_few_t(hipStream_t stream, const MatView &m, uint32_t to
 // Rows that give less than three quarters of the CUs a tile take the kernel only while they are short: the tile kernels
 // below share long columns between CUs, and one CU draws about 40 GB/s (F16, 4 tokens, against them: 1024x4096 7.9 / 12.0 us,
 // 1024x8192 13.4 / 13.7, 1024x14336 21.5 / 19.0, with 16 tokens 1024x6144 14.0 / 14.4, 1024x8192 16.7 / 14.9; F32
-// 512x2048 5.9 / 10.6, 1024x6144 with 16 tokens 17.2 / 15.3).  17 to 32 tokens take twice the matrix-core time: 512x3072
-// with 20 11.8 / 13.2 (F32 12.8 / 12.8), F32 512x4096 16.1 / 13.9, F32 4096x4096 with 32 18.7 / 23.3, 4096x14336 59.6 / 55.9.
+// 512x2048 5.9 / 10.6, 1024x6144 with 16 tokens 17.2 / 15.3).  17 to 32 tokens take twice the matrix-core time:
+// 512x3072 with 20 11.8 / 13.2 (F32 12.8 / 12.8), F32 512x4096 16.1 / 13.9, F32 4096x4096 with 32 18.7 / 23.3, 3072x8192 33.5 / 32.3.
+// F16 matrices of 2^23 weights and more meet launch_pg there: 4096x4096 with 32 16.0 / 25.6, 2048x4096 15.0 / 20.0, 2048x6144
+// 21.0 / 23.3, 2048x8192 with 20 26.5 / 25.5, 4096x8192 with 32 28.2 / 33.3, 8192x4096 29.1 / 32.9, 14336x4096 with 17 54.8 / 49.8,
+// 4096x14336 47.2 / 47.7.
 static bool few_takes(const MatView &m, uint32_t tokens) {
-    if ((m.type != T_F32 && m.type != T_F16) || tokens < 2 || tokens > 32 || pg_takes(m, tokens) || skinny_takes(m)) return false;
-    const bool wide = (m.rows + 15) / 16 >= (uint32_t)g_cu_count * 3 / 4;
-    if (tokens > 16) return m.cols <= (wide ? 8192u : 3072u);
-    return wide || m.cols <= (m.type == T_F16 ? 6144u : 4096u);
+    if ((m.type != T_F32 && m.type != T_F16) || tokens < 2 || tokens > 32 || skinny_takes(m)) return false;
+    const uint32_t tiles = (m.rows + 15) / 16, cus = (uint32_t)g_cu_count;
+    const bool wide = tiles >= cus * 3 / 4;
+    if (tokens <= 16) return wide || m.cols <= (m.type == T_F16 ? 6144u : 4096u);
+    if (m.type == T_F32) return m.cols <= (wide ? 6144u : 3072u);
+    const size_t n = (size_t)m.rows * m.cols;
+    if (n < ((size_t)1 << 23)) return m.cols <= 3072;
+    return n <= ((size_t)1 << 25) && m.cols <= (wide ? 8192u : tiles >= cus / 2 ? 6144u : 3072u);
 }
 template <uint32_t T> static hipError_t launch_few(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *y) {
     // A tile for every CU at most: one workgroup of sixteen wavefronts each; else three of eight, which go on from tile

@@ -609,7 +609,7 @@ def test_plain_products_of_few_tokens(pkg, gpu, ty):
     rng = np.random.default_rng(90 + ty)
     shapes = [(17, 1), (18, 31), (31, 33), (33, 63), (32, 64), (48, 65), (49, 127), (65, 130), (100, 511), (64, 516), (130, 1025),
               (35, 2052), (20, 3072), (20, 3073), (20, 4096), (20, 4100), (20, 6144), (20, 6152), (3057, 515), (3073, 8200), (4096, 96), (4097, 68),
-              (12305, 40)]
+              (12305, 40), (2050, 4100), (2050, 6148), (3073, 6148), (8200, 4104)]
     for rows, cols in shapes:
         w = K.random_packed(ty, rows, cols, rng)
         m = gpu.upload_packed(ty, rows, cols, w)
