@@ -827,7 +827,7 @@ static hipError_t launch_mm(hipStream_t stream, MmPlan &p, void *ws, size_t ws_b
     }
 }
 
-// F32 / F16 weights, up to 32 tokens, and more where there is no workspace to cut the activations into:
+// F32 / F16 weights, up to 32 tokens where rows are few and long, and more where there is no workspace to cut the activations into:
 // gemm_fmfma_kernel (+ fg_reduce_kernel when columns are shared).
 struct FgPlan {
     FgJob job;
@@ -913,7 +913,7 @@ static void pg_fit(const MatView &m, uint32_t tokens, uint32_t tok, uint32_t ks,
     p.x_bytes = up256((size_t)n_steps * 12 * p.job.mpad * sizeof(uint4));
     p.part_bytes = ks > 1 ? up256((size_t)ks * tokens * m.rows * sizeof(float)) : 0;
 }
-// Whether a product of F32 / F16 weights takes gemm_plain_kernel.  Up to 16 tokens the launch that cuts the activations
+// Whether a product of F32 / F16 weights that few_takes leaves takes gemm_plain_kernel.  Up to 16 tokens the launch that cuts the activations
 // costs more than the faster matrix instruction gives (F16 4096x14336, 8 tokens: 40 us on the f32 instruction, 44 here);
 // up to 32 only the two parts of F16 weights are worth it, for matrices large enough to hide that launch (4096x14336, 20
 // tokens 55 -> 46 us; 1000x2048 13.3 -> 14.1; F32 56 -> 61).
