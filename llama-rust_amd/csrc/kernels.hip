@@ -574,7 +574,11 @@ static hipError_t launch_multi_t(hipStream_t stream, const MatView *mats, float 
         const uint32_t chunks = (mats[0].cols + Geo<T>::E - 1) / Geo<T>::E;
         constexpr bool PLAIN = T == T_F32 || T == T_F16;
         if constexpr (PLAIN) {
-            if (chunks >= 1024 || (chunks >= 512 && rows < 8192)) {
+            // The longest rows that fit the LDS leave no room there for the wavefronts' sums: a wavefront each (F32 1100x20480
+            // 15.9 us; the tile kernel, which takes what no launch here does, 1750).
+            constexpr size_t MEET = GEMV_WAVES * 4 * sizeof(float);  // at most four rows per group
+            const bool fits = (size_t)chunks * Geo<T>::E * sizeof(float) + MEET <= g_lds_limit;
+            if (fits && (chunks >= 1024 || (chunks >= 512 && rows < 8192))) {
                 if (T == T_F32 || rows < 1024) return launch_rows<T, 64, 2, 2, true>(stream, mats, ys, n, x, accumulate);
                 return launch_rows<T, 32, 2, 1, true>(stream, mats, ys, n, x, accumulate);
             }

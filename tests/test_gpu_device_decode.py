@@ -190,6 +190,42 @@ def test_prologue_is_refused_where_it_is_not_built(pkg):
     gpu.close()
 
 
+@pytest.mark.parametrize("name,cols", [("F32", 20464), ("F32", 20465), ("F32", 20480), ("F16", 20464), ("F16", 20480)])
+@pytest.mark.parametrize("rows_list", [(40, 24), (1100,)])
+def test_shared_products_take_every_row_that_fits_the_lds(pkg, name, cols, rows_list):
+    """20480 floats are what a workgroup's 80 KB of LDS hold: plain rows up to there are one launch, also where nothing is left
+    beside x for the sums of wavefronts that share a row.  One column more is refused, with y as it was."""
+    import cases as K
+    hip = importlib.import_module("llama-rust_amd.hiprt")
+    ty = getattr(K, name)
+    rng = np.random.default_rng(cols + len(rows_list))
+    gpu = pkg.HipGemv(0)
+    ws = [K.random_packed(ty, r, cols, rng, signed=False, scale=0.02) for r in rows_list]
+    mats = [gpu.upload_packed(ty, r, cols, w) for r, w in zip(rows_list, ws)]
+    x = rng.normal(0, 1.0, cols).astype(np.float32)
+    dx, ys = _device(hip, x), [hip.DeviceBuffer(4 * r) for r in rows_list]
+    for y in ys:
+        y.fill_byte(0xff)
+    for times in (1, 2):
+        gpu.gemv_shared_device(mats, dx.ptr, [y.ptr for y in ys], accumulate=times == 2)
+        gpu.synchronize()
+        for r, w, y in zip(rows_list, ws, ys):
+            exact, mag = oracle.gemm_f64_mag(ty, cols, 1, w, x, r)
+            err = np.abs(y.to_numpy(np.float32).astype(np.float64) - times * exact.ravel())
+            assert np.all(err <= times * K.single_kernel_bound(cols + 1, mag.ravel()))
+    for m in mats:
+        m.close()
+    longer = gpu.upload_packed(ty, 8, 20481, K.random_packed(ty, 8, 20481, rng, signed=False, scale=0.02))
+    dx, y = _device(hip, np.ones(20481)), hip.DeviceBuffer(32)
+    y.fill_byte(0x5a)
+    with pytest.raises(pkg.NativeHipError) as ei:
+        gpu.gemv_shared_device([longer], dx.ptr, [y.ptr])
+    assert ei.value.code == pkg.ERR_UNSUPPORTED
+    gpu.synchronize()
+    assert set(y.to_numpy(np.uint8).tolist()) == {0x5a}
+    gpu.close()
+
+
 def test_fused_and_unfused_device_sessions_agree(pkg, llama, tmp_path, monkeypatch):
     """LLAMA_HIP_DECODE_UNFUSED keeps RMSNorm and SiLU*up as kernels of their own: same tokens, logits to 1e-4."""
     path = tmp_path / "small.gguf"
