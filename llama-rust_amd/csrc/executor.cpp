@@ -17,6 +17,7 @@
 #include "early_gemm.h"
 #include "head_step.h"
 #include "host_range.h"
+#include "host_route.h"
 #include "kernels.h"
 
 static_assert(LNH_NOALLOC_WORKSPACE_BYTES == nh::STATIC_SCRATCH_BYTES, "header and device array disagree");
@@ -250,14 +251,14 @@ int ensure_tiled(lnh_exec *e, hipStream_t s, const lnh_matrix *m, nh::MatView *v
     return LNH_OK;
 }
 
+nh::HostProduct host_product(const lnh_matrix *m, size_t tokens) { return {tokens, m->view.rows, m->view.cols, m->view.type}; }
+
 // Launch n products; xs/ys are device pointers.
 int launch_products(lnh_exec *e, hipStream_t s, size_t n, const lnh_matrix *const *mats, const size_t *tokens,
                     const float *const *xs, float *const *ys) {
-    // Single-token products of one input (q, k, v; gate, up) go out as one launch.
-    bool together = n > 1 && n <= 8;
-    for (size_t g = 0; g < n && together; g++)
-        together = tokens[g] == 1 && xs[g] == xs[0] && mats[g]->view.rows != 0 && mats[g]->view.type == mats[0]->view.type &&
-                   mats[g]->view.cols == mats[0]->view.cols;
+    bool same_x = true;
+    for (size_t g = 1; g < n; g++) same_x = same_x && xs[g] == xs[0];
+    const bool together = n > 1 && nh::launched_together(n, same_x, [&](size_t g) { return host_product(mats[g], tokens[g]); });
     if (together) {
         nh::MatView views[8];
         for (size_t g = 0; g < n; g++) views[g] = mats[g]->view;
@@ -395,14 +396,6 @@ void copy_floats(lnh_exec *e, float *dst, const float *src, size_t n) {
     nh::host_pool(e).run_ranges(n, 32768, [&](size_t begin, size_t end) { std::memcpy(dst + begin, src + begin, (end - begin) * sizeof(float)); });
 }
 
-// A decode step's products, called one by one, spend more time on the copies around them than on their weights: their kernels
-// read a short x from pinned memory as they stage it and write y there, each value once, in one launch instead of three (host
-// calls, us: Q4_K 4096x4096 22.1 -> 17.0, 14336x4096 27.6 -> 21.0, Q6_K 32000x4096 42.7 -> 36.1, Q5_0 4864x896 21.2 -> 15.3).
-// Reading x that way costs the product 2 us with 4096 columns, 3 with 8192 and 8 with 14336 (every workgroup stages all of
-// it), where a launch that copies it first costs 4: longer rows are copied.  More than two tokens are products whose kernels
-// read x more than once and write y in scattered pieces; rows of more than 16384 columns are summed in y by several launches.
-constexpr size_t DIRECT_TOKENS = 2, DIRECT_X_FLOATS = 8192, DIRECT_COLS = 16384;
-
 // A product of host buffers between the enqueueing of its work and the arrival of its result.
 struct HostCall {
     bool staged = false;  // y comes through the executor's pinned staging
@@ -425,14 +418,13 @@ int begin_host(lnh_exec *e, size_t n_groups, const lnh_matrix *const *mats, cons
     if (!pinned && !y) return LNH_ERR_UNSUPPORTED;
     call->staged = pinned && !y_there;
     call->y_total = y_total;
-    bool direct = pinned;
-    for (size_t g = 0; g < n_groups; g++) direct = direct && tokens[g] <= DIRECT_TOKENS && mats[g]->view.cols <= DIRECT_COLS;
     const float *const x_pinned = x_there ? x_there : e->h_in;
     float *const y_pinned = y_there ? y_there : e->h_out;
-    const bool direct_x = direct && x_total <= DIRECT_X_FLOATS;
+    nh::HostRoute direct;
+    if (pinned) direct = nh::host_route(n_groups, shared_x, x_total, y_there != nullptr, [&](size_t g) { return host_product(mats[g], tokens[g]); });
     if (pinned) {
         if (!x_there) copy_floats(e, e->h_in, x, x_total);
-        if (!direct_x) h = nh::launch_copy_small(e->stream, e->d_in, x_pinned, ((x_total + 3) & ~(size_t)3) * sizeof(float));
+        if (!direct.x) h = nh::launch_copy_small(e->stream, e->d_in, x_pinned, ((x_total + 3) & ~(size_t)3) * sizeof(float));
     } else {
         h = hipMemcpyAsync(e->d_in, x, x_total * sizeof(float), hipMemcpyHostToDevice, e->stream);
     }
@@ -441,13 +433,13 @@ int begin_host(lnh_exec *e, size_t n_groups, const lnh_matrix *const *mats, cons
     std::vector<float *> ys(n_groups);
     size_t xo = 0, yo = 0;
     for (size_t g = 0; g < n_groups; g++) {
-        xs[g] = (direct_x ? x_pinned : e->d_in) + xo;
-        ys[g] = (direct ? y_pinned : e->d_out) + yo;
+        xs[g] = (direct.x ? x_pinned : e->d_in) + xo;
+        ys[g] = (direct.y ? y_pinned : e->d_out) + yo;
         if (!shared_x) xo += tokens[g] * mats[g]->view.cols;
         yo += tokens[g] * mats[g]->view.rows;
     }
     rc = launch_products(e, e->stream, n_groups, mats, tokens, xs.data(), ys.data());
-    if (rc == LNH_OK && !direct) {
+    if (rc == LNH_OK && !direct.y) {
         if (pinned)
             h = nh::launch_copy_small(e->stream, y_pinned, e->d_out, ((y_total + 3) & ~(size_t)3) * sizeof(float));
         else

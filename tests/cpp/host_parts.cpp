@@ -13,6 +13,7 @@
 #include "../../llama-rust_amd/csrc/device_once.h"
 #include "../../llama-rust_amd/csrc/host_pool.h"
 #include "../../llama-rust_amd/csrc/host_range.h"
+#include "../../llama-rust_amd/csrc/host_route.h"
 
 static int failures = 0;
 #define CHECK(cond)                                                         \
@@ -44,6 +45,35 @@ static void host_range() {
     CHECK(nh::device_view(host, 8192, find) == nullptr);          // the last part is pinned only
     CHECK(nh::device_view(host + 4096, SIZE_MAX, find) == nullptr);
     CHECK(nh::device_view(host + 4096, 16, [](const void *, nh::HostMapping *) { return true; }) == nullptr);
+}
+
+// Which host calls' kernels use pinned memory; the caller's own y only where one launch writes the whole of it, so that a call
+// of several launches that fails has left it alone.
+static void host_route() {
+    constexpr uint32_t F16 = 1, Q4_0 = 2, Q4_K = 12, Q6_K = 14;
+    auto route = [](const std::vector<nh::HostProduct> &p, bool shared_x, bool y_in_place) {
+        size_t x = 0;
+        for (const nh::HostProduct &q : p) x = shared_x ? q.tokens * q.cols : x + q.tokens * q.cols;
+        const nh::HostRoute r = nh::host_route(p.size(), shared_x, x, y_in_place, [&](size_t g) { return p[g]; });
+        return (r.x ? 1 : 0) + (r.y ? 2 : 0);
+    };
+    for (bool own : {false, true}) {
+        CHECK(route({{1, 20000, 4096, Q4_K}}, false, own) == 3);
+        CHECK(route({{1, 20000, 8192, Q4_K}}, false, own) == 3);
+        CHECK(route({{1, 20000, 8448, Q4_K}}, false, own) == 2);
+        CHECK(route({{1, 20000, 16384, Q4_K}}, false, own) == 2);
+        CHECK(route({{1, 20000, 16640, Q4_K}}, false, own) == 0);
+        CHECK(route({{3, 20000, 256, Q4_K}}, false, own) == 0);
+        CHECK(route({{1, 14336, 4096, Q4_K}, {1, 14336, 4096, Q4_K}}, true, own) == 3);                     // one launch
+        CHECK(route(std::vector<nh::HostProduct>(8, {1, 4096, 4096, Q4_K}), true, own) == 3);
+        CHECK(route({{1, 4096, 4096, Q4_K}, {1, 16384, 4096, Q6_K}}, true, own) == (own ? 0 : 3));          // two dtypes
+        CHECK(route({{1, 8192, 4096, Q4_K}, {1, 8192, 4096, Q4_K}}, false, own) == (own ? 0 : 3));          // two inputs
+        CHECK(route({{1, 8192, 4096, Q4_K}, {1, 0, 4096, Q4_K}}, true, own) == (own ? 0 : 3));
+        CHECK(route(std::vector<nh::HostProduct>(9, {1, 4096, 4096, Q4_K}), true, own) == (own ? 0 : 3));
+        CHECK(route({{2, 8192, 1024, Q4_0}}, false, own) == (own ? 0 : 3));                                 // a launch per token
+        CHECK(route({{2, 8192, 1024, F16}}, false, own) == (own ? 0 : 3));
+        CHECK(route({{1, 8192, 1024, Q4_0}, {2, 8192, 1024, Q4_0}}, false, own) == (own ? 0 : 3));
+    }
 }
 
 // Every item exactly once, seen by the caller afterwards, over calls of changing size that follow each other closely or
@@ -162,6 +192,7 @@ static void device_once() {
 int main() {
     pool_without_threads();  // first: a forked child has only the thread that forked
     host_range();
+    host_route();
     device_once();
     pools();
     if (failures == 0) std::printf("OK\n");
