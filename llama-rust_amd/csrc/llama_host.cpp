@@ -34,6 +34,7 @@
 #include "gguf.h"
 #include "head_step.h"
 #include "host_pool.h"
+#include "step_replays.h"
 
 namespace {
 

@@ -14,6 +14,7 @@
 #include "../../llama-rust_amd/csrc/host_pool.h"
 #include "../../llama-rust_amd/csrc/host_range.h"
 #include "../../llama-rust_amd/csrc/host_route.h"
+#include "../../llama-rust_amd/csrc/step_replays.h"
 
 static int failures = 0;
 #define CHECK(cond)                                                         \
@@ -74,6 +75,45 @@ static void host_route() {
         CHECK(route({{2, 8192, 1024, F16}}, false, own) == (own ? 0 : 3));
         CHECK(route({{1, 8192, 1024, Q4_0}, {2, 8192, 1024, Q4_0}}, false, own) == (own ? 0 : 3));
     }
+}
+
+// Every step once, in whole replays where there is the longer graph, which is made when single replays have lost what it costs
+// and never asked for again where it cannot be made.
+static void step_replays() {
+    constexpr size_t STEPS = nh::StepReplays::STEPS;
+    for (bool can : {true, false}) {
+        nh::StepReplays r;
+        r.set_nodes(20);
+        const size_t worth = r.worth();
+        CHECK(worth > STEPS && worth < 400);
+        size_t steps = 0, singles = 0, wholes = 0, makes = 0;
+        auto run = [&](size_t n) {
+            steps = singles = wholes = 0;
+            const int rc = r.run(n, [&] { return steps++, singles++, 0; }, [&] { return steps += STEPS, wholes++, 0; });
+            CHECK(rc == 0 && steps == n && singles + STEPS * wholes == n);
+        };
+        auto offer = [&] { r.offer([&] { return makes++, can ? 0 : 1; }); };
+        for (size_t i = 0; i < 1000; i++) run(STEPS - 1), offer();  // runs that it could not serve
+        CHECK(makes == 0);
+        run(worth - 1 + STEPS - 1), offer();  // one step short
+        CHECK(makes == 0 && wholes == 0);
+        run(STEPS);
+        CHECK(wholes == 0);
+        offer();
+        CHECK(makes == 1);
+        for (size_t n : {size_t(0), size_t(1), STEPS - 1, STEPS, STEPS + 1, 5 * STEPS, 5 * STEPS + 3, 4 * worth}) {
+            run(n), offer();
+            CHECK(wholes == (can ? n / STEPS : 0));
+        }
+        CHECK(makes == 1);
+    }
+    nh::StepReplays none;  // a graph without nodes is no reason either
+    none.set_nodes(0);
+    none.offer([] { failures++; return 0; });
+    // what fails ends the run
+    nh::StepReplays r;
+    size_t calls = 0;
+    CHECK(r.run(5, [&] { return ++calls == 3 ? 7 : 0; }, [] { return 0; }) == 7 && calls == 3);
 }
 
 // Every item exactly once, seen by the caller afterwards, over calls of changing size that follow each other closely or
@@ -193,6 +233,7 @@ int main() {
     pool_without_threads();  // first: a forked child has only the thread that forked
     host_range();
     host_route();
+    step_replays();
     device_once();
     pools();
     if (failures == 0) std::printf("OK\n");

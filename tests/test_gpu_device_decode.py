@@ -470,7 +470,7 @@ def test_output_head_with_its_norm_and_candidates(pkg, llama, tmp_path, monkeypa
 @pytest.mark.parametrize("n_new", [1, 7, 8, 9, 16, 17])
 def test_steps_replayed_together_equal_single_steps(pkg, llama, tmp_path, monkeypatch, n_new):
     """Step counts around the eight that one replay holds, of both kinds of device session once they have run long enough
-    for that (256 steps), against the same steps enqueued kernel by kernel; a second run continues where the first stopped."""
+    for that (their first runs here are), against the same steps enqueued kernel by kernel; a second run continues where the first stopped."""
     path = tmp_path / "steps.gguf"
     llama.write_synthetic_llama(path, n_layer=2, n_embd=256, n_head=4, n_head_kv=2, n_ff=512, n_vocab=512, seed=4, weight_std=0.1)
     m = llama.Llama(path=path)
@@ -479,10 +479,10 @@ def test_steps_replayed_together_equal_single_steps(pkg, llama, tmp_path, monkey
 
     def run():
         one, several = m.session(device_positions=400), m.batch_session(3, 320)
-        out = [one.generate_greedy(prompts[1].tolist(), 269)[0].tolist()]  # eight at a time begins within this run
+        out = [one.generate_greedy(prompts[1].tolist(), 269)[0].tolist()]  # long enough: eight at a time from the next run on
         for _ in range(2):
             out.append(one.generate_greedy([out[-1][-1]], n_new)[0].tolist())
-        out += several.generate_greedy(prompts, 262)[0].tolist()           # and in the next one here
+        out += several.generate_greedy(prompts, 262)[0].tolist()           # here too
         return out + several.generate_greedy(prompts, n_new)[0].tolist()
 
     replayed = run()
