@@ -1029,6 +1029,14 @@ static hipError_t launch_pg(hipStream_t stream, const MatView &m, uint32_t token
 }
 
 bool skinny_takes(const MatView &m) { return (m.type == T_F32 || m.type == T_F16) && m.rows <= SKINNY_ROWS; }
+// Whether that is also the fastest launch for a product on the device.  A workgroup reads all rows for its one token, so few
+// tokens of long rows leave that reading to few CUs, where the tile kernels share the columns between them (F32, matrices read
+// from memory, skinny / tiles, us: 16x4096 at 2 tokens 7.2 / 11.2, 12x8192 11.3 / 12.0, 12x10240 15.2 / 13.2, 16x14336 21.6 / 16.6, at
+// 16 tokens 19.7 / 16.9, at 32 19.2 / 19.3, 8x16384 at 2 12.8 / 17.4; F16 is half the bytes: 16x14336 at 2 16.1 / 15.8, 16x16384
+// 15.9 / 17.1).
+static bool skinny_pays(const MatView &m, uint32_t tokens) {
+    return skinny_takes(m) && !(m.type == T_F32 && m.rows > 8 && m.cols > 8192 && tokens <= 16);
+}
 hipError_t launch_skinny(hipStream_t stream, const MatView &m, uint32_t tokens, const float *x, float *x_copy, float *y) {
     if (!skinny_takes(m) || m.rows == 0 || tokens == 0) return hipErrorInvalidValue;
     void (*kern)(MatView, const float *, float *, float *);
@@ -1055,7 +1063,7 @@ static hipError_t launch_few_t(hipStream_t stream, const MatView &m, uint32_t to
 // 21.0 / 23.3, 2048x8192 with 20 26.5 / 25.5, 4096x8192 with 32 28.2 / 33.3, 8192x4096 29.1 / 32.9, 14336x4096 with 17 54.8 / 49.8,
 // 4096x14336 47.2 / 47.7.
 static bool few_takes(const MatView &m, uint32_t tokens) {
-    if ((m.type != T_F32 && m.type != T_F16) || tokens < 2 || tokens > 32 || skinny_takes(m)) return false;
+    if ((m.type != T_F32 && m.type != T_F16) || tokens < 2 || tokens > 32 || skinny_pays(m, tokens)) return false;
     const uint32_t tiles = (m.rows + 15) / 16, cus = (uint32_t)g_cu_count;
     const bool wide = tiles >= cus * 3 / 4;
     if (tokens <= 16) return wide || m.cols <= (m.type == T_F16 ? 6144u : 4096u);
@@ -1143,7 +1151,7 @@ size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_
         if (tokens[g] == 0 || mats[g].rows == 0) { g++; continue; }
         const uint32_t run = mm_run(mats, tokens, n, g);
         if (run == 0) {
-            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1 && !skinny_takes(mats[g]) && !few_takes(mats[g], tokens[g])) {
+            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1 && !skinny_pays(mats[g], tokens[g]) && !few_takes(mats[g], tokens[g])) {
                 size_t bytes;
                 FgPlan f;
                 fg_plan(mats[g], tokens[g], f);
@@ -1185,7 +1193,7 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
                 for (uint32_t t = 0; t < tokens[g] && e == hipSuccess; t++)
                     e = launch_plain(stream, mats[g], 1, xs[g] + (size_t)t * mats[g].cols, ys[g] + (size_t)t * mats[g].rows);
             } else if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1) {
-                if (skinny_takes(mats[g])) e = launch_skinny(stream, mats[g], tokens[g], xs[g], nullptr, ys[g]);
+                if (skinny_pays(mats[g], tokens[g])) e = launch_skinny(stream, mats[g], tokens[g], xs[g], nullptr, ys[g]);
                 else if (few_takes(mats[g], tokens[g]))
                     e = mats[g].type == T_F16 ? launch_few<T_F16>(stream, mats[g], tokens[g], xs[g], ys[g])
                                               : launch_few<T_F32>(stream, mats[g], tokens[g], xs[g], ys[g]);

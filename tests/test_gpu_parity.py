@@ -430,9 +430,10 @@ def test_plain_dtypes_on_the_matrix_cores_every_tile_and_share_shape(pkg, gpu, t
 
 
 @pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("rows,cols,tokens", [(1, 1, 2), (3, 7, 5), (8, 4096, 64), (8, 4099, 3), (9, 4100, 17), (16, 1023, 2), (16, 8196, 130), (17, 64, 9)])
+@pytest.mark.parametrize("rows,cols,tokens", [(1, 1, 2), (3, 7, 5), (8, 4096, 64), (8, 4099, 3), (9, 4100, 17), (16, 1023, 2), (16, 8196, 130), (17, 64, 9),
+                                              (9, 8192, 16), (8, 8196, 16), (9, 8196, 16), (9, 8196, 17), (16, 16384, 2)])
 def test_plain_dtypes_of_a_few_rows(gpu, ty, rows, cols, tokens):
-    """Routers: up to 16 rows take one launch whatever the tokens; columns that fill no vector, one more row than that."""
+    """Routers: up to 16 rows take one launch, but for few tokens of long F32 rows; columns that fill no vector, one more row than that."""
     rng = np.random.default_rng(rows * cols + tokens)
     w = K.random_packed(ty, rows, cols, rng)
     x = rng.normal(0, 1, tokens * cols).astype(np.float32)
