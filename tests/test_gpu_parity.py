@@ -979,8 +979,8 @@ def test_grouped_call_with_token_counts_on_both_sides_of_every_kernel_switch(pkg
 
 
 def test_shared_input_products_equal_separate_calls(pkg, gpu):
-    """q, k, v (and gate, up) read the same activations: one call, one input copy.  The values are those
-    of the separate calls bit for bit (same kernels, same order of additions within each row)."""
+    """q, k, v (and gate, up) read the same activations: one call, one input copy.  The values are those of the separate
+    calls, bit for bit where both fall to the same kernel variant, as these shapes do (those that do not: next test)."""
     rng = np.random.default_rng(21)
     for ty, cols, rows_list in [(K.Q4_K, 4096, (4096, 1024, 1024)), (K.Q4_K, 14336, (100, 37, 4099)), (K.Q8_0, 1024, (256, 96)),
                                 (K.Q6_K, 512, (64, 64, 64, 64)), (K.F16, 320, (33, 7))]:
@@ -1011,6 +1011,30 @@ def test_shared_input_products_equal_separate_calls(pkg, gpu):
         gpu.gemm_shared([a, b], 1, np.zeros(256, np.float32), np.zeros(64, np.float32))
     with pytest.raises(pkg.NativeHipError, match="at least one token"):
         gpu.gemm_shared([a], 0, np.zeros(0, np.float32), np.zeros(0, np.float32))
+
+
+@pytest.mark.parametrize("ty,cols,rows_list", [
+    (K.Q4_K, 4096, (1020, 1020)), (K.Q4_K, 2048, (2048, 512, 512)), (K.Q4_K, 4096, (10236, 10)), (K.Q4_K, 8192, (2046, 4)),  # parts of a super-block
+    (K.Q6_K, 4096, (4096, 1024, 1024)), (K.Q6_K, 4096, (8192, 16)),                            # parts, loop over super-blocks
+    (K.Q8_0, 4096, (1500, 1500)), (K.Q4_0, 8192, (1500, 1500)), (K.Q5_1, 16384, (3000, 100)),  # parts of a unit
+    (K.Q5_0, 4128, (4100, 4100)), (K.F16, 4096, (600, 600)), (K.F16, 4096, (4100, 4100)), (K.F32, 480, (4100, 4100))])  # shared rows, lanes per row
+def test_shared_input_products_on_another_side_of_a_rule_than_alone(pkg, gpu, ty, cols, rows_list):
+    """The rules that cut single-token launches count the rows of the whole launch, so a product may be summed in another
+    order in a shared call than alone: other last bits, the same bound against the exact product."""
+    rng = np.random.default_rng(cols + rows_list[0])
+    ws = [K.random_packed(ty, r, cols, rng) for r in rows_list]
+    mats = [gpu.upload_packed(ty, r, cols, w) for r, w in zip(rows_list, ws)]
+    x = rng.normal(0, 1, cols).astype(np.float32)
+    y = np.full(sum(rows_list), np.nan, np.float32)
+    gpu.gemm_shared(mats, 1, x, y)
+    off = 0
+    for r, w, m in zip(rows_list, ws, mats):
+        alone = np.full(r, np.nan, np.float32)
+        gpu.gemm_resident(m, 1, x, alone)
+        check(y[off:off + r], ty, cols, 1, r, w, x, f"shared {pkg.TYPE_NAMES[ty]} rows {r}")
+        check(alone, ty, cols, 1, r, w, x, f"alone {pkg.TYPE_NAMES[ty]} rows {r}")
+        off += r
+        m.close()
 
 
 # ------------------------------------------------------------------ residency
