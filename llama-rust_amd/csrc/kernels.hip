@@ -687,7 +687,7 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
         any_split = any_split || ks > 1;
         total_tok += tokens[j];
     }
-    for (uint32_t j = n; j < MM_MAX_JOBS; j++) b.job[j] = b.job[0];
+    for (uint32_t j = n; j < (uint32_t)MM_FEW_JOBS; j++) b.job[j] = b.job[0];  // launches copy these too
     b.n_jobs = n;
     b.mpad = total_tok + (p.tile16 ? 16 : 64);  // a tile may read up to 15 resp. 63 slots past its job's last token
     b.total_wgs = wgs;
@@ -703,6 +703,25 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     p.part_bytes = part;
 }
 
+// Launches f(arguments, their size as a constant) with room for as many jobs as the batch has.
+template <typename F> static hipError_t with_jobs(const MmBatch &b, F &&f) {
+    if (b.n_jobs > (uint32_t)MM_FEW_JOBS) {
+        f(b, std::integral_constant<int, MM_MAX_JOBS>{});
+    } else {
+        MmFewBatch few;
+        static_cast<MmHead &>(few) = b;
+        std::memcpy(few.job, b.job, sizeof(few.job));
+        f(few, std::integral_constant<int, MM_FEW_JOBS>{});
+    }
+    return hipGetLastError();
+}
+template <uint32_t T> static hipError_t launch_xsplit(hipStream_t stream, const MmBatch &b, uint32_t n_groups) {
+    return with_jobs(b, [&](const auto &args, auto jobs) {
+        hipLaunchKernelGGL((mm_xsplit_kernel<T, decltype(jobs)::value>), dim3((b.mpad + XS_TOK - 1) / XS_TOK, (n_groups + XS_GRP - 1) / XS_GRP),
+                           dim3(256), 0, stream, args, n_groups);
+    });
+}
+
 // INLINE (TT = 1): the jobs' x are plain f32 rows and the kernel cuts them itself.
 template <uint32_t T, int TT, int VQ, bool INLINE = false, bool FB = false, bool NORM = false>
 static hipError_t launch_mm_main(hipStream_t stream, const MmBatch &b) {
@@ -711,14 +730,18 @@ static hipError_t launch_mm_main(hipStream_t stream, const MmBatch &b) {
         if (g_nibble_i4) return launch_mm_main<T, TT, VQ, INLINE, true, NORM>(stream, b);
     }
     constexpr size_t lds = 2 * MmStage<T, TT>::BYTES;  // two pipeline stages
-    auto kern = gemm_mfma_kernel<T, TT, VQ, FB, INLINE, NORM>;
-    if constexpr (lds > 48 * 1024) {
-        static DeviceOnce limit;
-        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(kern, dim3(b.total_wgs), dim3(256), lds, stream, b);
-    return hipGetLastError();
+    hipError_t limits = hipSuccess;
+    const hipError_t e = with_jobs(b, [&](const auto &args, auto jobs) {
+        constexpr int JOBS = decltype(jobs)::value;
+        auto kern = gemm_mfma_kernel<T, TT, VQ, FB, INLINE, NORM, JOBS>;
+        if constexpr (lds > 48 * 1024) {
+            static DeviceOnce limit;  // per instantiation
+            limits = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
+            if (limits != hipSuccess) return;
+        }
+        hipLaunchKernelGGL(kern, dim3(b.total_wgs), dim3(256), lds, stream, args);
+    });
+    return limits != hipSuccess ? limits : e;
 }
 
 // 9 to 16 tokens: only Q6_K gets here, the other dtypes take 16-token tiles
@@ -733,8 +756,9 @@ template <bool FB> static hipError_t launch_mm_q4k64(hipStream_t stream, const M
     if constexpr (!FB) {
         if (b.nibble_bf16) return launch_mm_q4k64<true>(stream, b);
     }
-    hipLaunchKernelGGL(gemm_q4k64_kernel<FB>, dim3(b.total_wgs), dim3(256), 0, stream, b);
-    return hipGetLastError();
+    return with_jobs(b, [&](const auto &args, auto jobs) {
+        hipLaunchKernelGGL((gemm_q4k64_kernel<FB, decltype(jobs)::value>), dim3(b.total_wgs), dim3(256), 0, stream, args);
+    });
 }
 
 // INLINE: the jobs' x are plain f32 rows and the kernel cuts them itself (no mm_xsplit launch before it).
@@ -751,8 +775,9 @@ static hipError_t launch_mm16_lo(hipStream_t stream, const MmBatch &b) {
     using Tr = Mm16Traits<T, NT, LO>;
     constexpr size_t lds = Tr::LDS_BYTES;  // per group of wavefronts two pipeline stages and the exchange slots
     static_assert(lds <= 48 * 1024, "within the default dynamic LDS limit");
-    hipLaunchKernelGGL((gemm_mfma16_kernel<T, FB, INLINE, NORM, NT, LO>), dim3(b.total_wgs), dim3(Tr::THREADS), lds, stream, b);
-    return hipGetLastError();
+    return with_jobs(b, [&](const auto &args, auto jobs) {
+        hipLaunchKernelGGL((gemm_mfma16_kernel<T, FB, INLINE, NORM, NT, LO, decltype(jobs)::value>), dim3(b.total_wgs), dim3(Tr::THREADS), lds, stream, args);
+    });
 }
 template <uint32_t T, bool INLINE = false, bool NORM = false, int NT = 1>
 static hipError_t launch_mm16_main(hipStream_t stream, const MmBatch &b, uint32_t max_tok) {
@@ -775,6 +800,13 @@ static uint32_t mm_reduce_blocks(const MmBatch &b) {
     return (uint32_t)(most < 512 ? most : 512);
 }
 
+static hipError_t launch_mm_reduce(hipStream_t stream, const MmBatch &b) {
+    if (!b.any_split) return hipGetLastError();
+    return with_jobs(b, [&](const auto &args, auto jobs) {
+        hipLaunchKernelGGL(mm_reduce_kernel<decltype(jobs)::value>, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, args);
+    });
+}
+
 template <uint32_t T>
 static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws_bytes) {
     if (p.xb_bytes + p.sx_bytes + p.part_bytes > ws_bytes) return hipErrorInvalidValue;
@@ -792,20 +824,19 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
     if (p.tile16) {  // the 16-token kernel cuts the activations itself
         e = launch_mm16_main<T, true>(stream, b, p.max_tok);
         if (e != hipSuccess) return e;
-        if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
-        return hipGetLastError();
+        return launch_mm_reduce(stream, b);
     }
     if constexpr (T == T_Q4_K) {
         if (p.tile16x2) {
             e = launch_mm16_main<T, true, false, 2>(stream, b, p.max_tok);
             if (e != hipSuccess) return e;
-            if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
-            return hipGetLastError();
+            return launch_mm_reduce(stream, b);
         }
     }
-    if (p.tt == 2)  // 64-token tiles: the activations are cut once, by a launch of their own
-        hipLaunchKernelGGL(mm_xsplit_kernel<T>, dim3((b.mpad + XS_TOK - 1) / XS_TOK, (p.n_groups + XS_GRP - 1) / XS_GRP),
-                           dim3(256), 0, stream, b, p.n_groups);
+    if (p.tt == 2) {  // 64-token tiles: the activations are cut once, by a launch of their own
+        e = launch_xsplit<T>(stream, b, p.n_groups);
+        if (e != hipSuccess) return e;
+    }
     if constexpr (T == T_Q4_K) {
         e = launch_mm_q4k64<false>(stream, b);
     } else {
@@ -815,8 +846,7 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
         else e = launch_mm_main<T, 1, 4, true>(stream, b);
     }
     if (e != hipSuccess) return e;
-    if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
-    return hipGetLastError();
+    return launch_mm_reduce(stream, b);
 }
 
 static hipError_t launch_mm(hipStream_t stream, MmPlan &p, void *ws, size_t ws_bytes) {
@@ -1263,16 +1293,13 @@ hipError_t launch_act_split(hipStream_t stream, void *act, uint32_t type, uint32
     b.job[0].x = x;
     b.job[0].tokens = tokens;
     b.job[0].tok_off = 0;
-    for (uint32_t j = 1; j < MM_MAX_JOBS; j++) b.job[j] = b.job[0];
     b.n_jobs = 1;
     b.xb = v.xb;
     b.sx = v.sx;
     b.mpad = v.mpad;
     return mm_by_type(type, [&](auto t) {
         constexpr uint32_t T = decltype(t)::value;
-        hipLaunchKernelGGL(mm_xsplit_kernel<T>, dim3((b.mpad + XS_TOK - 1) / XS_TOK, (v.n_groups + XS_GRP - 1) / XS_GRP), dim3(256),
-                           0, stream, b, v.n_groups);
-        return hipGetLastError();
+        return launch_xsplit<T>(stream, b, v.n_groups);
     });
 }
 
@@ -1330,7 +1357,6 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
         if (in.mpad != b.mpad) return hipErrorInvalidValue;  // the plan's slots and the buffer's must be the same thing
     } else {
         for (uint32_t j = 0; j < b.n_jobs; j++) b.job[j].x = x_plain;
-        for (uint32_t j = b.n_jobs; j < (uint32_t)MM_MAX_JOBS; j++) b.job[j].x = x_plain;
         if (cut_first) {
             in.xb = static_cast<uint4 *>(ws);
             in.sx = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + p.xb_bytes);
@@ -1380,9 +1406,10 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
             if (p.tile16x2)
                 return x_plain ? launch_mm16_main<T, true, false, 2>(stream, b, p.max_tok) : launch_mm16_main<T, false, false, 2>(stream, b, p.max_tok);
         }
-        if (cut_first)
-            hipLaunchKernelGGL(mm_xsplit_kernel<T>, dim3((b.mpad + XS_TOK - 1) / XS_TOK, (p.n_groups + XS_GRP - 1) / XS_GRP),
-                               dim3(256), 0, stream, b, p.n_groups);
+        if (cut_first) {
+            const hipError_t cut = launch_xsplit<T>(stream, b, p.n_groups);
+            if (cut != hipSuccess) return cut;
+        }
         if constexpr (T == T_Q4_K) {  // up to 32 tokens: above
             return launch_mm_q4k64<false>(stream, b);
         } else {
@@ -1404,8 +1431,7 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     });
     if (e != hipSuccess) return e;
     if (!fused) {
-        if (b.any_split) hipLaunchKernelGGL(mm_reduce_kernel, dim3(mm_reduce_blocks(b), b.n_jobs), dim3(256), 0, stream, b);
-        return hipGetLastError();
+        return launch_mm_reduce(stream, b);
     }
     const size_t total = (size_t)tokens * rows;
     auto shares = [&](uint32_t j) { return b.job[j].ksplit > 1 ? b.job[j].part : b.job[j].y; };

@@ -978,6 +978,26 @@ def test_grouped_call_with_token_counts_on_both_sides_of_every_kernel_switch(pkg
         m.close()
 
 
+@pytest.mark.parametrize("ty", [K.Q4_0, K.Q4_K], ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("n", [8, 9, 16, 17])
+def test_grouped_calls_of_as_many_products_as_a_launch_takes(pkg, gpu, ty, n):
+    """A launch has room for eight or for sixteen products: both full, one more than each; every tile size."""
+    rng = np.random.default_rng(n)
+    cols, rows = 1024, [33 + 17 * g for g in range(n)]
+    ws = [K.random_packed(ty, r, cols, rng) for r in rows]
+    mats = [gpu.upload_packed(ty, r, cols, w) for r, w in zip(rows, ws)]
+    for t in (7, 20, 70):
+        x = rng.normal(0, 1, n * t * cols).astype(np.float32)
+        y = np.full(t * sum(rows), np.nan, np.float32)
+        gpu.gemm_grouped(mats, [t] * n, x, y)
+        at = 0
+        for g, r in enumerate(rows):
+            check(y[at:at + t * r], ty, cols, t, r, ws[g], x[g * t * cols:(g + 1) * t * cols])
+            at += t * r
+    for m in mats:
+        m.close()
+
+
 def test_shared_input_products_equal_separate_calls(pkg, gpu):
     """q, k, v (and gate, up) read the same activations: one call, one input copy.  The values are those of the separate
     calls, bit for bit where both fall to the same kernel variant, as these shapes do (those that do not: next test)."""
