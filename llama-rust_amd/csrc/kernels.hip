@@ -270,14 +270,14 @@ static hipError_t launch_gemv_q4k_pro(hipStream_t stream, const MatView *mats, f
         while (lbb < 64 && lbb < units) lbb <<= 1;
         // Several lanes per super-block for matrices that would otherwise give the chip few wavefront steps per CU.
         // Quarters below one (alone on the card, quarters against halves: 512 x 256 2.27 against 2.53 us, 512 x 4096
-        // 2.79 against 3.04; up to five steps they still gain 9 to 1 % alone, but a [q,k,v] launch and its three separate
-        // products would add in different orders, and beside other work they take from it: decode steps of three
-        // streams at once, each with a 4096 x 4096 product per layer = four steps, 962 against 921 us).  Halves up to
+        // 2.79 against 3.04; up to five steps they still gain 9 to 1 % alone, but beside other work they take from it:
+        // decode steps of three streams at once, each with a 4096 x 4096 product per layer = four steps, 962 against
+        // 921 us).  The steps are those of the whole launch, so a product can be added in another order in a shared
+        // launch than alone (2048 / 512 / 512 x 2048 is; 4096 / 1024 / 1024 x 4096 is not).  Halves up to
         // ten (8192 x 4096 gains 11 % over whole blocks, 12288 x 4096 loses 6 %).  Rows of 17 to 32 super-blocks have
         // room for halves only, up to four steps (512 x 5632 3.30 against 4.49 us, 2048 x 8192 4.55 against 5.08, 2560 x 7168 = five steps
         // 5.14 against 5.14, 4096 x 8192 6.60 against 6.37).  Rows of one super-block are never taken whole: that
-        // variant spilled (262144 x 256 120 -> 12 us).  The pair epilogue stays with the halves and with the shapes
-        // that it took with them.
+        // variant spilled (262144 x 256 120 -> 12 us).  The pair epilogue takes no quarters.
         size_t full_steps = 0;
         for (uint32_t j = 0; j < n_jobs; j++) full_steps += (mats[j].rows + 64 / lbb - 1) / (64 / lbb);
         const size_t cus = g_cu_count;
@@ -415,6 +415,10 @@ static hipError_t launch_gemv_q6k(hipStream_t stream, const MatView *mats, float
         b.accumulate = accumulate || w > 0;
         // One step per wavefront, on the graph: 512x1024 4.2 -> 2.9 us, 4096x4096 6.2 -> 5.4, 2048x11008 9.8 -> 7.9, 128256x4096
         // 71.2 -> 66.9; between those sizes the loop is faster (14336x4096 11.2 against 11.8, 32000x4096 20.3 against 21.0).
+        // The largest ones only with rows of 9 to 16 super-blocks; with others the loop stays although the part kernel takes
+        // 0 to 6 % less there (matrices in turn, loop / part, us: 262144x1024 41.0 / 39.3, 131072x2048 37.6 / 37.6, 256000x2048
+        // 71.0 / 67.3, 128256x5120 122.7 / 115.7, 32000x8192 40.4 / 38.8, 128256x8192 142.9 / 136.9; of 9 to 16 below this
+        // size, 50000x3072 28.5 / 27.6, 65536x4096 38.5 / 37.9).
         hipError_t part = hipErrorInvalidValue;
         const size_t lanes = rows * lb;
         auto small = [&](auto tag) {

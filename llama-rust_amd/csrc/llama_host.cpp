@@ -811,11 +811,12 @@ float moe_weight(const MoeScratch *ms, size_t k, uint32_t t, size_t e) {
     return 0.f;
 }
 
-// The routed feed-forward with the resident products chained on the device: the rows go up once (pinned staging),
-// the router product runs there and only its n x n_expert logits come back for the host's routing; then the
-// bucket order goes up (a few KB), the rows are gathered, gate and up are grouped launches, SiLU(gate) * up an
-// element-wise kernel, down a grouped launch, the scatter a kernel, and the n x n_embd result comes back: two host
-// synchronisations, no expert output ever on the host.  Same products and the same order of additions as moe_ffn's
+// The routed feed-forward with the resident products chained on the device: the router's launches read the rows from
+// pinned staging, 256 KB at a time, leave them on the device and write the n x n_expert logits back to pinned memory
+// for the host's routing (a router of more than 16 rows or of blocks: one copy up, a product, one copy down); the gather
+// reads the bucket order from pinned memory, gate and up are grouped launches, SiLU(gate) * up an element-wise kernel,
+// down a grouped launch, and the scatter writes the n x n_embd result to pinned memory: two host synchronisations, no
+// expert output ever on the host.  Same products and the same order of additions as moe_ffn's
 // host form; SiLU with the device's expf.
 int moe_ffn_on_device(lnm_model *m, Layer &l, size_t n, const float *x, float *ffn_out, MoeScratch *ms, lnm_session *timed) {
     const lnm_hparams &hp = m->hp;
@@ -919,7 +920,7 @@ int moe_ffn_on_device(lnm_model *m, Layer &l, size_t n, const float *x, float *f
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e);
     {
         // gate and up of every expert as one batch: the experts of at most 16 rows first, then the others, so that
-        // products of one tile size lie together and share launches (up to eight each) - with eight products a
+        // products of one tile size lie together and share launches (up to sixteen each) - with so many products a
         // launch has enough tiles to fill the chip without sharing columns, and no launch sums shares
         std::vector<const lnh_matrix *> mats;
         std::vector<size_t> rows;
