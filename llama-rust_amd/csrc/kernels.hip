@@ -1185,7 +1185,8 @@ size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_
         if (tokens[g] == 0 || mats[g].rows == 0) { g++; continue; }
         const uint32_t run = mm_run(mats, tokens, n, g);
         if (run == 0) {
-            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1 && !skinny_pays(mats[g], tokens[g]) && !few_takes(mats[g], tokens[g])) {
+            if ((mats[g].type == T_F32 || mats[g].type == T_F16) && tokens[g] > 1 && !(least ? skinny_takes(mats[g]) : skinny_pays(mats[g], tokens[g])) &&
+                !few_takes(mats[g], tokens[g])) {
                 size_t bytes;
                 FgPlan f;
                 fg_plan(mats[g], tokens[g], f);
@@ -1233,6 +1234,8 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
                                               : launch_few<T_F32>(stream, mats[g], tokens[g], xs[g], ys[g]);
                 else e = pg_takes(mats[g], tokens[g]) ? launch_pg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes)
                                                 : launch_fg(stream, mats[g], tokens[g], xs[g], ys[g], ws, ws_bytes);
+                // no room for the shares of a plan (a stream under capture): the launch that needs none
+                if (e == hipErrorInvalidValue && skinny_takes(mats[g])) e = launch_skinny(stream, mats[g], tokens[g], xs[g], nullptr, ys[g]);
             } else {
                 e = launch_plain(stream, mats[g], tokens[g], xs[g], ys[g]);
             }

@@ -332,9 +332,10 @@ def test_workspace_growth_under_stream_capture_is_refused_not_recorded(pkg):
 
 
 @pytest.mark.parametrize("ty", [K.F16, K.F32], ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("rows,cols,tokens,before", [(300, 256, 40, 0), (5000, 1032, 420, 0), (5000, 1032, 420, 130), (5000, 1032, 420, 33)])
+@pytest.mark.parametrize("rows,cols,tokens,before", [(300, 256, 40, 0), (5000, 1032, 420, 0), (5000, 1032, 420, 130), (5000, 1032, 420, 33),
+                                                     (16, 10240, 4, 0), (9, 8196, 16, 0)])
 def test_plain_dtype_captured_without_its_workspace(pkg, ty, rows, cols, tokens, before):
-    """F16 / F32 products whose columns are not shared can be recorded into a graph by an executor that has run nothing yet
+    """F16 / F32 products whose columns are not shared, or of at most 16 rows, can be recorded into a graph by an executor that has run nothing yet
     or only a product of fewer tokens: the plan that cuts the activations into a workspace gives way to pieces that fit,
     or to the kernel that needs none.  Replayed with new inputs and the program's own eager work in between, each replay
     within the bound of the eager result."""
