@@ -957,9 +957,15 @@ struct PgPlan {
     uint32_t tok, wgs;
     size_t x_bytes, part_bytes;
 };
+// Bytes a token slot takes in the cut activations: twelve vectors a step, for F16 weights a factor per 256 columns.
+static size_t pg_slot_bytes(const MatView &m, uint32_t n_steps) {
+    return (size_t)n_steps * 12 * sizeof(uint4) + (m.type == T_F16 ? (size_t)((m.cols + PG_BLOCK - 1) / PG_BLOCK) * sizeof(float) : 0);
+}
+// Weight rows of a workgroup on tiles of `tok` tokens.
+static uint32_t pg_rows(const MatView &m, uint32_t tok) { return m.type == T_F16 && tok == 128 ? (uint32_t)PhTraits<128>::ROWS : (uint32_t)PG_ROWS; }
 // Sizes of a product of `tokens` tokens on tiles of `tok`, columns shared `ks` ways.
 static void pg_fit(const MatView &m, uint32_t tokens, uint32_t tok, uint32_t ks, PgPlan &p) {
-    const uint32_t row_tiles = (m.rows + PG_ROWS - 1) / PG_ROWS, n_steps = (m.cols + PG_K - 1) / PG_K;
+    const uint32_t rows = pg_rows(m, tok), row_tiles = (m.rows + rows - 1) / rows, n_steps = (m.cols + PG_K - 1) / PG_K;
     p.tok = tok;
     p.job = PgJob{};
     p.job.m = m;
@@ -971,7 +977,7 @@ static void pg_fit(const MatView &m, uint32_t tokens, uint32_t tok, uint32_t ks,
     p.job.mpad = p.job.tok_tiles * tok + 8;
     p.job.n_steps = n_steps;
     p.wgs = p.job.tok_tiles * row_tiles * ks;
-    p.x_bytes = up256((size_t)n_steps * 12 * p.job.mpad * sizeof(uint4));
+    p.x_bytes = up256(pg_slot_bytes(m, n_steps) * p.job.mpad);
     p.part_bytes = ks > 1 ? up256((size_t)ks * tokens * m.rows * sizeof(float)) : 0;
 }
 // Whether a product of F32 / F16 weights that few_takes leaves takes gemm_plain_kernel.  Up to 16 tokens the launch that cuts the activations
@@ -982,24 +988,22 @@ static bool pg_takes(const MatView &m, uint32_t tokens) {
     return tokens > 32 || (tokens > 16 && m.type == T_F16 && (size_t)m.rows * m.cols >= ((size_t)1 << 23));
 }
 // Token tile and column shares, priced together: a step of a workgroup that shares its CU with another and of one that
-// has it alone (us, F16, measured on 4096x14336 with 512 tokens: the wider tile reads and cuts its weights for more
-// tokens), two steps for a workgroup's start and end, and what the launch that sums the shares costs (3 TB/s + 3.5 us).
-// Wide tiles win where there is work for the whole chip (512 tokens: 394 / 325 / 296 us with tiles of 32 / 64 / 128, F32
-// 563 / 459 / 438), narrow ones where rows and tokens are few (300x1000, 128 tokens: 16.7 / 18.8 / 26.4 us, F32 18.1 /
-// 20.8 / 28.1).  F32's steps cost more in about the same proportions, so F16's prices do for both: against the best of
-// all tiles and shares, over seven shapes from 300x1024 to 14336x4096 with 40 to 512 tokens, either loses 1.1 % on
-// average and 6.5 (4096x4096, 128 tokens) resp. 5.9 % (14336x4096, 128 tokens) at worst.
+// has it alone (us, measured on 4096x14336 and 14336x4096; a workgroup of F16's 128-token tile always has its CU alone), two steps
+// for a workgroup's start and end, and what the launch that sums the shares costs (3 TB/s + 3.5 us).
+// Wide tiles win where there is work for the whole chip (4096x14336, 512 tokens on tiles of 32 / 64 / 128: F16 284 / 225 / 197 us, F32
+// 563 / 459 / 438), narrow ones where rows and tokens are few (F32 300x1000, 128 tokens: 18.1 / 20.8 / 28.1 us).
 static void pg_plan(const MatView &m, uint32_t tokens, PgPlan &p) {
     static constexpr uint32_t tile[3] = {32, 64, 128};
-    static constexpr double shared_us[3] = {0.47, 0.69, 1.25}, alone_us[3] = {0.55, 0.8, 1.39};
-    const uint32_t row_tiles = (m.rows + PG_ROWS - 1) / PG_ROWS, n_steps = (m.cols + PG_K - 1) / PG_K;
+    static constexpr double price[2][2][3] = {{{0.47, 0.69, 1.25}, {0.55, 0.8, 1.39}}, {{0.36, 0.5, 1.55}, {0.48, 0.6, 1.5}}};  // [F16][alone]
+    const double *shared_us = price[m.type == T_F16][0], *alone_us = price[m.type == T_F16][1];
+    const uint32_t n_steps = (m.cols + PG_K - 1) / PG_K;
     uint32_t ks_max = n_steps / 8;  // a share is at least 256 columns
     ks_max = ks_max > 32 ? 32 : ks_max < 1 ? 1 : ks_max;
     double best = 0.0;
     uint32_t tok = 0, ks = 1;
     for (int k = 0; k < 3; k++) {
         if (k > 0 && tokens <= tile[k - 1]) break;
-        const uint32_t tiles = (tokens + tile[k] - 1) / tile[k] * row_tiles;
+        const uint32_t rows = pg_rows(m, tile[k]), tiles = (tokens + tile[k] - 1) / tile[k] * ((m.rows + rows - 1) / rows);
         for (uint32_t s = 1; s <= ks_max; s++) {
             const uint64_t wgs = (uint64_t)tiles * s, per_cu = (wgs + (uint32_t)g_cu_count - 1) / (uint32_t)g_cu_count;
             double cost = ((double)((n_steps + s - 1) / s) + 2.0) * (per_cu == 1 ? alone_us[k] : (double)per_cu * shared_us[k]);
@@ -1030,7 +1034,7 @@ static uint32_t pg_piece(PgPlan &p, size_t ws_bytes) {
     const PgJob &j = p.job;
     if (ws_bytes > PG_WS_BYTES) ws_bytes = PG_WS_BYTES;
     if (p.x_bytes + p.part_bytes <= ws_bytes) return j.tokens;
-    const size_t column = (size_t)j.n_steps * 12 * sizeof(uint4), fixed = 8 * column + 512;  // 512: both parts are rounded up
+    const size_t column = pg_slot_bytes(j.m, j.n_steps), fixed = 8 * column + 512;  // 512: both parts are rounded up
     for (uint32_t tok = p.tok; tok >= 32; tok /= 2) {
         const size_t tile = tok * (column + (j.ksplit > 1 ? (size_t)j.ksplit * j.m.rows * sizeof(float) : 0));
         if (fixed + tile > ws_bytes) continue;
@@ -1045,8 +1049,12 @@ static uint32_t pg_piece(PgPlan &p, size_t ws_bytes) {
 
 template <uint32_t T, int TOK>
 static hipError_t launch_pg_main(hipStream_t stream, const PgPlan &p) {
-    constexpr size_t lds = 2 * PgTraits<T, TOK>::STAGE;
-    auto kern = gemm_plain_kernel<T, TOK>;
+    if constexpr (T == T_F16) {  // its LDS is static: no function attribute has to be set
+        hipLaunchKernelGGL(gemm_f16_kernel<TOK>, dim3(p.wgs), dim3(64 * PhTraits<TOK>::WAVES), 0, stream, p.job);
+        return hipGetLastError();
+    }
+    constexpr size_t lds = 2 * PgTraits<TOK>::STAGE;
+    auto kern = gemm_plain_kernel<TOK>;
     if constexpr (lds > 48 * 1024) {
         static DeviceOnce limit;
         const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(kern), lds);
@@ -1068,8 +1076,9 @@ static hipError_t launch_pg(hipStream_t stream, const MatView &m, uint32_t token
         p.job.x = x + (size_t)t * m.cols;
         p.job.y = y + (size_t)t * m.rows;
         p.job.xb = static_cast<uint4 *>(ws);
+        p.job.xf = reinterpret_cast<float *>(p.job.xb + (size_t)p.job.n_steps * 12 * p.job.mpad);
         p.job.part = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + p.x_bytes);
-        hipLaunchKernelGGL(pg_split_kernel, dim3((p.job.mpad + PG_XS_TOK - 1) / PG_XS_TOK, (p.job.n_steps * PG_K + PG_XS_COLS - 1) / PG_XS_COLS),
+        hipLaunchKernelGGL(m.type == T_F16 ? pg_split_kernel<true> : pg_split_kernel<false>, dim3((p.job.mpad + PG_XS_TOK - 1) / PG_XS_TOK, (p.job.n_steps * PG_K + PG_XS_COLS - 1) / PG_XS_COLS),
                            dim3(256), 0, stream, p.job);
         hipError_t e;
         if (m.type == T_F16)
