@@ -65,3 +65,17 @@ def test_numbers_of_every_magnitude(gpu, cols):
     x[69] = x[1][::-1]
     w[:, cols - 1] = np.where(np.arange(rows) % 2, w[:, cols - 1], np.float16(0.0))
     _check(gpu, w, x)
+
+
+def test_small_activations_beside_a_few_large_ones_of_zero_weights(gpu):
+    """The sum is the small ones' alone: they must not be held to what the large ones allow."""
+    rng = np.random.default_rng(3)
+    rows, cols, tokens = 140, 1024, 70
+    w = rng.normal(0, 0.02, (rows, cols)).astype(np.float16)
+    x = np.zeros((tokens, cols), np.float32)
+    for g in range(cols // 256):
+        at = 256 * g + rng.permutation(256)[:10]
+        w[:, at[:7]] = 0
+        x[:, at[:7]] = rng.uniform(0.5, 1, (tokens, 7))
+        x[:, at[7:]] = rng.normal(0, 2.0 ** -32, (tokens, 3))
+    _check(gpu, w, x)

@@ -76,6 +76,22 @@ def test_activations_of_every_magnitude(gpu, ty):
     _check(ty, rows, cols, x, w, _product(gpu, ty, rows, cols, x, w))
 
 
+@pytest.mark.parametrize("ty", [K.Q4_0, K.Q5_0], ids=lambda t: O.TYPE_NAMES[t])
+def test_small_activations_beside_a_few_large_ones_of_zero_weights(gpu, ty):
+    """The sum is the small ones' alone: they must not be held to what the large ones allow."""
+    rng = np.random.default_rng(23 + ty)
+    cols, tokens = 512, 40
+    w = K.random_packed(ty, 1, cols, rng)
+    w32 = O.dequant(ty, cols, w, 1).reshape(-1, 32)
+    x = np.zeros((tokens, cols), np.float32)
+    for g in range(cols // 32):
+        zero, rest = np.flatnonzero(w32[g] == 0), np.flatnonzero(w32[g] != 0)
+        at = rng.permutation(rest)[:3]
+        x[:, 32 * g + at] = rng.normal(0, 2.0 ** -22, (tokens, 3))
+        x[:, 32 * g + zero[:7]] = rng.uniform(0.5, 1, (tokens, len(zero[:7])))
+    _check(ty, 1, cols, x, w, _product(gpu, ty, 1, cols, x, w))
+
+
 @pytest.mark.parametrize("ty", [K.Q4_0, K.Q4_K], ids=lambda t: O.TYPE_NAMES[t])
 def test_infinities_stay_in_their_token(gpu, ty):
     rng = np.random.default_rng(5)
