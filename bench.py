@@ -242,12 +242,10 @@ def other_workloads(pkg, hip, gpu, stream, rng, cpu):
                 check(f"{names[ty]} GEMM {rows}x{cols} M={tokens}", ty, rows, cols, tokens, ws[0], x[:tokens * cols], yd)
                 flops = 2.0 * rows * cols * tokens
                 with_cpu = ty == Q4_0 and rows == D and tokens > 1
-                # three bf16 MFMA products per multiply-add (the f32 activations are split in three); Q4_0 and Q5_0 above
-                # 32 tokens: the time of 1.5 (six 6-bit digits at four times the bf16 rate)
-                per_mad = 1.5 if ty != Q5_1 and tokens > 32 else 3
+                # three bf16 MFMA products per multiply-add (the f32 activations are split in three)
                 out[f"gemm_{names[ty]}_{rows}x{cols}_m{tokens}"] = {
                     "call_us": round(us, 2), "tflops": round(flops / us / 1e6, 1),
-                    "mfma_frac": round(per_mad * flops / us / 1e6 / BF16_MFMA_PEAK_TFLOPS, 4) if tokens > 1 else None,
+                    "mfma_frac": round(3 * flops / us / 1e6 / BF16_MFMA_PEAK_TFLOPS, 4) if tokens > 1 else None,
                     "weight_gbs": round(rows * row_bytes(ty, cols) / us / 1e3, 1),
                     "hbm_frac": round(algorithmic_bytes(ty, rows, cols, tokens) / us / 1e3 / HBM_PEAK_GBS, 4),
                     "bound": "mfma" if tokens >= 128 else "hbm",

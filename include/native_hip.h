@@ -206,8 +206,8 @@ int lnh_gemv_swiglu_device(lnh_exec *exec, const lnh_matrix *gate, const lnh_mat
                            float *device_h, int prologue, const float *device_x2, float eps, void *stream);
 /* Activations kept in the form the multi-token kernels read, for steps that stay on the device.  No counterpart in
  * the reference, whose every product takes and returns plain f32 rows on the host (langtax/src/native_gpu.rs:124-213).
- * A multi-token product is up to three launches: the activations are cut into three bf16 parts (Q4_0, Q5_0 and Q4_K
- * with more than 32 tokens: six 6-bit digits) in the matrix's column order (a launch of its own for more than 32 tokens; the matrix-core launch does it for fewer), the matrix-core launch
+ * A multi-token product is up to three launches: the activations are cut into three bf16 parts in the matrix's column
+ * order (a launch of its own for more than 32 tokens; the matrix-core launch does it for fewer), the matrix-core launch
  * writes one partial result per share of the columns, a last launch sums the shares.
  * Between two products of a decode step lies only element-wise work; lnh_gemm_act_device does that work in the
  * launch that sums the shares and leaves its result already cut for the next matrix, so a chain of products costs

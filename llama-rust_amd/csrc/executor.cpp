@@ -779,7 +779,8 @@ int lnh_act_create(lnh_exec *e, uint32_t type, size_t cols, size_t max_tokens, l
     void *dev = nullptr;
     h = hipMalloc(&dev, bytes + nh::ACT_DEFER_PARTIAL_BYTES);
     if (h != hipSuccess) return hip_fail(e, h, "HIP activation allocation");
-    // slots past the tokens of a call are multiplied like any other and dropped: keep them finite from the start
+    // slots past the tokens of a call are multiplied like any other and dropped, whatever they hold: zeros only so that no run differs
+    // from another
     h = hipMemsetAsync(dev, 0, bytes + nh::ACT_DEFER_PARTIAL_BYTES, e->stream);
     const hipError_t hs = hipStreamSynchronize(e->stream);
     if (h == hipSuccess) h = hs;

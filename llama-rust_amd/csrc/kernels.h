@@ -39,8 +39,8 @@ hipError_t launch_gemm(hipStream_t stream, const MatView &m, const MatView &tile
 hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const MatView *tiled, const uint32_t *tokens,
                               const float *const *xs, float *const *ys, uint32_t n, void *ws, size_t ws_bytes);
 
-// Activations that stay in the form the matrix-core kernels read (three bf16 parts per group of 16 columns, or six
-// 6-bit digits per 32, in the column order of the dtype that will multiply them) between products, for callers whose steps stay on the device:
+// Activations that stay in the form the matrix-core kernels read (three bf16 parts per group of 16 columns, in the
+// column order of the dtype that will multiply them) between products, for callers whose steps stay on the device:
 // act_bytes sizes a buffer for up to max_tokens tokens of `cols` columns under a matrix of dtype `type` (0: not a
 // dtype / shape of the matrix-core path); launch_act_split fills it from plain f32 rows; launch_gemm_act multiplies
 // it by n matrices of that dtype and column count (tiled copies, tokens >= 3) and either writes ys (epilogue NONE:

@@ -615,9 +615,6 @@ struct MmPlan {
 // Most tokens of a job that the 16-token kernel takes (Q6_K fills its rows with 8).
 static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
 
-// Dtypes whose products of more than 32 tokens are gemm_f6_kernel's.
-static bool mm_f6(uint32_t type) { return type == T_Q4_0 || type == T_Q5_0 || type == T_Q4_K; }
-
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Jobs share dtype and column count; every job has at least MM_MIN_TOKENS tokens.
@@ -658,28 +655,21 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     if (ks_max > 32) ks_max = 32;
     if (ks_max < 1) ks_max = 1;
     const uint32_t slots = (uint32_t)(2 * g_cu_count), alone = (uint32_t)g_cu_count;
+    const double step_us = p.tile16 ? 0.8 : p.tt == 2 ? 1.7 : 0.7, alone_cost = p.tile16 ? 0.53 : 0.7;
     const double bytes_per_us = p.tile16 ? 6.0e6 : p.tt == 2 ? 4.0e6 : 3.0e6;
-    auto best_shares = [&](double step_us, double alone_cost, uint32_t most) {
-        uint32_t shares = 1;
-        double best = 0.0;
-        for (uint32_t ks = 1; ks <= most; ks++) {
-            const uint64_t wg = (uint64_t)(launch_tiles ? launch_tiles : 1) * ks;
-            const double len = (double)((n_steps + ks - 1) / ks) + 2.0;
-            const uint64_t rounds = wg / slots, rest = wg % slots;
-            double cost = (double)rounds * len + (rest == 0 ? 0.0 : rest <= alone ? alone_cost * len : len);
-            if (ks > 1) cost += ((double)ks * (double)share_bytes / bytes_per_us + 3.5) / step_us;
-            if (ks == 1 || cost < best) {
-                best = cost;
-                shares = ks;
-            }
+    uint32_t ks_launch = 1;
+    double best = 0.0;
+    for (uint32_t ks = 1; ks <= ks_max; ks++) {
+        const uint64_t wg = (uint64_t)(launch_tiles ? launch_tiles : 1) * ks;
+        const double len = (double)((n_steps + ks - 1) / ks) + 2.0;
+        const uint64_t rounds = wg / slots, rest = wg % slots;
+        double cost = (double)rounds * len + (rest == 0 ? 0.0 : rest <= alone ? alone_cost * len : len);
+        if (ks > 1) cost += ((double)ks * (double)share_bytes / bytes_per_us + 3.5) / step_us;
+        if (ks == 1 || cost < best) {
+            best = cost;
+            ks_launch = ks;
         }
-        return shares;
-    };
-    uint32_t ks_launch = best_shares(p.tile16 ? 0.8 : p.tt == 2 ? 1.7 : 0.7, p.tile16 ? 0.53 : 0.7, ks_max);
-    // gemm_f6_kernel's steps are shorter: 4096x14336 at 512 tokens 120 us in 4 shares, 145 in 2; Q4_K 4099x14336 at 100 tokens 38 in 15,
-    // 45 in 7.  Never more shares than the prices of the bf16 kernels give: a product then needs no more workspace than with those,
-    // which is what callers with a fixed one are refused by.
-    if (p.tt == 2 && mm_f6(mats[0].type)) ks_launch = best_shares(1.1, 0.61, ks_launch);
+    }
     for (uint32_t j = 0; j < n; j++) {
         MmJob &job = b.job[j];
         job.m = mats[j];
@@ -730,7 +720,7 @@ template <typename F> static hipError_t with_jobs(const MmBatch &b, F &&f) {
     return hipGetLastError();
 }
 // Token slots that hold a job's token: those behind them, which a last tile reads too, may hold anything - a slot's contents reach its own
-// token's sums alone, and those are not stored (Q4_K 4099x14336 at 100 tokens, 164 slots, four calls 215 -> 213 us; Q4_0 at 512 595 -> 593).
+// token's sums alone, and those are not stored.
 static uint32_t mm_used_slots(const MmBatch &b) {
     uint32_t used = 0;
     for (uint32_t j = 0; j < b.n_jobs; j++) used = b.job[j].tok_off + b.job[j].tokens > used ? b.job[j].tok_off + b.job[j].tokens : used;
@@ -772,28 +762,14 @@ static hipError_t launch_mm_main_q6k_16(hipStream_t stream, const MmBatch &b) {
     else return hipErrorInvalidValue;
 }
 
-// The kernel of more than 32 tokens and the launch that cuts its activations.
-template <uint32_t T, bool FB = false> static hipError_t launch_mm_64(hipStream_t stream, const MmBatch &b) {
-    if constexpr (f6_type<T>()) {
-        if constexpr (T == T_Q4_0 && !FB) {
-            if (g_nibble_i4) return launch_mm_64<T, true>(stream, b);
-        }
-        return with_jobs(b, [&](const auto &args, auto jobs) {
-            hipLaunchKernelGGL((gemm_f6_kernel<T, FB, decltype(jobs)::value>), dim3(b.total_wgs), dim3(256), 0, stream, args);
-        });
-    } else {
-        return launch_mm_main<T, 2, 4>(stream, b);
+// Q4_K, more than 32 tokens
+template <bool FB> static hipError_t launch_mm_q4k64(hipStream_t stream, const MmBatch &b) {
+    if constexpr (!FB) {
+        if (b.nibble_bf16) return launch_mm_q4k64<true>(stream, b);
     }
-}
-template <uint32_t T> static hipError_t launch_xsplit_64(hipStream_t stream, const MmBatch &b, uint32_t n_groups) {
-    if constexpr (f6_type<T>()) {
-        return with_jobs(b, [&](const auto &args, auto jobs) {
-            hipLaunchKernelGGL((f6_xsplit_kernel<T, decltype(jobs)::value>), dim3((mm_used_slots(b) + XS_TOK - 1) / XS_TOK, (n_groups + XS_GRP - 1) / XS_GRP),
-                               dim3(256), 0, stream, args, n_groups);
-        });
-    } else {
-        return launch_xsplit<T>(stream, b, n_groups);
-    }
+    return with_jobs(b, [&](const auto &args, auto jobs) {
+        hipLaunchKernelGGL((gemm_q4k64_kernel<FB, decltype(jobs)::value>), dim3(b.total_wgs), dim3(256), 0, stream, args);
+    });
 }
 
 // INLINE: the jobs' x are plain f32 rows and the kernel cuts them itself (no mm_xsplit launch before it).
@@ -869,15 +845,16 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
         }
     }
     if (p.tt == 2) {  // 64-token tiles: the activations are cut once, by a launch of their own
-        e = launch_xsplit_64<T>(stream, b, p.n_groups);
+        e = launch_xsplit<T>(stream, b, p.n_groups);
         if (e != hipSuccess) return e;
-        e = launch_mm_64<T>(stream, b);
-    } else if constexpr (T != T_Q4_K) {  // up to 32 tokens: above
-        if (T == T_Q6_K && p.max_tok <= 16) e = launch_mm_main_q6k_16<T, true>(stream, b);
+    }
+    if constexpr (T == T_Q4_K) {
+        e = launch_mm_q4k64<false>(stream, b);
+    } else {
+        if (p.tt == 2) e = launch_mm_main<T, 2, 4>(stream, b);
+        else if (T == T_Q6_K && p.max_tok <= 16) e = launch_mm_main_q6k_16<T, true>(stream, b);
         else if (p.max_tok <= 24) e = launch_mm_main<T, 1, 3, true>(stream, b);
         else e = launch_mm_main<T, 1, 4, true>(stream, b);
-    } else {
-        e = hipErrorInvalidValue;
     }
     if (e != hipSuccess) return e;
     return launch_mm_reduce(stream, b);
@@ -1345,7 +1322,7 @@ hipError_t launch_act_split(hipStream_t stream, void *act, uint32_t type, uint32
     b.mpad = v.mpad;
     return mm_by_type(type, [&](auto t) {
         constexpr uint32_t T = decltype(t)::value;
-        return tokens > 32 ? launch_xsplit_64<T>(stream, b, v.n_groups) : launch_xsplit<T>(stream, b, v.n_groups);
+        return launch_xsplit<T>(stream, b, v.n_groups);
     });
 }
 
@@ -1453,18 +1430,18 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
                 return x_plain ? launch_mm16_main<T, true, false, 2>(stream, b, p.max_tok) : launch_mm16_main<T, false, false, 2>(stream, b, p.max_tok);
         }
         if (cut_first) {
-            const hipError_t cut = launch_xsplit_64<T>(stream, b, p.n_groups);
+            const hipError_t cut = launch_xsplit<T>(stream, b, p.n_groups);
             if (cut != hipSuccess) return cut;
         }
-        if (p.tt == 2) return launch_mm_64<T>(stream, b);
         if constexpr (T == T_Q4_K) {  // up to 32 tokens: above
-            return hipErrorInvalidValue;
+            return launch_mm_q4k64<false>(stream, b);
         } else {
             if (norm) {
                 if (T == T_Q6_K && p.max_tok <= 16) return launch_mm_main_q6k_16<T, true, true>(stream, b);
                 if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true, false, true>(stream, b);
                 return launch_mm_main<T, 1, 4, true, false, true>(stream, b);
             }
+            if (p.tt == 2) return launch_mm_main<T, 2, 4>(stream, b);
             if (x_plain) {  // 32-token tiles cut plain activations themselves
                 if (T == T_Q6_K && p.max_tok <= 16) return launch_mm_main_q6k_16<T, true>(stream, b);
                 if (p.max_tok <= 24) return launch_mm_main<T, 1, 3, true>(stream, b);
@@ -1496,23 +1473,15 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     if (ep.kind == ACT_EPILOGUE_ADD_RMSNORM)
         return mm_by_type(nt, [&](auto t) {
             constexpr uint32_t TN = decltype(t)::value;
-            auto launch = [&](auto f6) {
-                hipLaunchKernelGGL((mm_epi_add_norm_kernel<TN, decltype(f6)::value>), dim3(tokens), dim3(1024), (size_t)rows * sizeof(float), stream,
-                                   shares(0), count(0), total, rows, ep.residual, ep.norm_w, ep.eps, ep.xn_out, next);
-            };
-            if (f6_type<TN>() && tokens > 32) launch(std::bool_constant<f6_type<TN>()>{});
-            else launch(std::false_type{});
+            hipLaunchKernelGGL(mm_epi_add_norm_kernel<TN>, dim3(tokens), dim3(1024), (size_t)rows * sizeof(float), stream, shares(0),
+                               count(0), total, rows, ep.residual, ep.norm_w, ep.eps, ep.xn_out, next);
             return hipGetLastError();
         });
     return mm_by_type(nt, [&](auto t) {  // SiLU(gate) * up
         constexpr uint32_t TN = decltype(t)::value;
         constexpr int GRP = 8;  // 128 columns per workgroup: 16 measured 2-3 % slower on the batch steps, 4 (not Q6_K's order) the same
-        auto launch = [&](auto f6) {
-            hipLaunchKernelGGL((mm_epi_swiglu_kernel<TN, GRP, decltype(f6)::value>), dim3((tokens + XS_TOK - 1) / XS_TOK, (next.n_groups + GRP - 1) / GRP),
-                               dim3(256), 0, stream, shares(0), count(0), shares(1), count(1), total, rows, tokens, next);
-        };
-        if (f6_type<TN>() && tokens > 32) launch(std::bool_constant<f6_type<TN>()>{});
-        else launch(std::false_type{});
+        hipLaunchKernelGGL((mm_epi_swiglu_kernel<TN, GRP>), dim3((tokens + XS_TOK - 1) / XS_TOK, (next.n_groups + GRP - 1) / GRP),
+                           dim3(256), 0, stream, shares(0), count(0), shares(1), count(1), total, rows, tokens, next);
         return hipGetLastError();
     });
 }
