@@ -170,7 +170,8 @@ def test_rows_of_one_weight(gpu, kind, rows, cols, tokens):
 
 
 @pytest.mark.parametrize("kind", ["swiglu", "lognormal", "outliers", "decades"])
-@pytest.mark.parametrize("rows,cols,tokens", [(300, 1000, 40), (1030, 8200, 70), (4096, 2500, 130)])
+# 1003: rows of activations that are aligned to single numbers
+@pytest.mark.parametrize("rows,cols,tokens", [(300, 1000, 40), (129, 1003, 33), (1030, 8200, 70), (4096, 2500, 130)])
 def test_dense_rows_by_activations_of_wide_range(gpu, kind, rows, cols, tokens):
     rng = np.random.default_rng(rows + cols + tokens)
     _check(gpu, rng.normal(0, 0.02, (rows, cols)).astype(np.float16), _spread(kind, rng, (tokens, cols)))

@@ -58,7 +58,7 @@ def test_tile_edges(gpu, ty, rows, cols, tokens):
 
 @pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
 def test_activations_of_every_magnitude(gpu, ty):
-    """Groups whose activations six digits hold, groups that are kept as f32 numbers, and both in one tile."""
+    """2^-107 to 2^93, every significand bit, one large among small ones, zeros; also in the last token of a partial tile."""
     rng = np.random.default_rng(91 + ty)
     rows, cols, tokens = 96, 2048, 70
     w = K.random_packed(ty, rows, cols, rng)
