@@ -957,7 +957,7 @@ static void pg_fit(const MatView &m, uint32_t tokens, uint32_t tok, uint32_t ks,
     p.job.tok_tiles = (tokens + tok - 1) / tok;
     p.job.ksplit = ks;
     // an odd number of 128-byte lines: a workgroup reads twelve planes of a step at the same slots, and planes a power of two
-    // apart meet on few of the memory's channels (F16 128 tokens 72 -> 68 us, F32 512 tokens 447 -> 437)
+    // apart meet on few of the memory's channels (F16 128 tokens 68 -> 65 us, F32 512 tokens 447 -> 437)
     p.job.mpad = p.job.tok_tiles * tok + 8;
     p.job.n_steps = n_steps;
     p.wgs = p.job.tok_tiles * row_tiles * ks;
@@ -965,9 +965,9 @@ static void pg_fit(const MatView &m, uint32_t tokens, uint32_t tok, uint32_t ks,
     p.part_bytes = ks > 1 ? up256((size_t)ks * tokens * m.rows * sizeof(float)) : 0;
 }
 // Whether a product of F32 / F16 weights that few_takes leaves takes gemm_plain_kernel.  Up to 16 tokens the launch that cuts the activations
-// costs more than the faster matrix instruction gives (F16 4096x14336, 8 tokens: 26.2 us on the f32 instruction, 27.2 here, 16 35.6
-// and 35.5); up to 32 only F16 weights, which need a third of F32's products, are worth it, for matrices too large for few_takes
-// (4096x14336, 20 tokens 53 -> 43 us; F32 56 -> 61).
+// costs more than the faster matrix instruction gives (F16 4096x14336, 8 tokens: 26.8 us on the f32 instruction, 27.1 here, 16 35.4
+// and 35.2); up to 32 only F16 weights, which need a third of F32's products, are worth it, for matrices too large for few_takes
+// (4096x14336, 20 tokens 53 -> 40 us; F32 56 -> 61).
 static bool pg_takes(const MatView &m, uint32_t tokens) {
     if (m.type == T_F16 && m.s0 >= (size_t)1 << 24) return false;  // gemm_f16_kernel finds 256 rows at 32-bit offsets
     return tokens > 32 || (tokens > 16 && m.type == T_F16 && (size_t)m.rows * m.cols >= ((size_t)1 << 23));
@@ -975,11 +975,11 @@ static bool pg_takes(const MatView &m, uint32_t tokens) {
 // Token tile and column shares, priced together: a step of a workgroup that shares its CU with another and of one that
 // has it alone (us, measured on 4096x14336 and 14336x4096; a workgroup of F16's 128-token tile always has its CU alone), two steps
 // for a workgroup's start and end, and what the launch that sums the shares costs (3 TB/s + 3.5 us).
-// Wide tiles win where there is work for the whole chip (4096x14336, 512 tokens on tiles of 32 / 64 / 128: F16 305 / 222 / 196 us, F32
-// 563 / 459 / 438), narrow ones where rows and tokens are few (300x1024, 512 tokens: F16 16.8 / 16.8 / 22.8 us; F32 300x1000, 128 tokens:
+// Wide tiles win where there is work for the whole chip (4096x14336, 512 tokens on tiles of 32 / 64 / 128: F16 276 / 221 / 190 us, F32
+// 563 / 459 / 438), narrow ones where rows and tokens are few (300x1024, 512 tokens: F16 14.8 / 15.8 / 22.7 us; F32 300x1000, 128 tokens:
 // 18.1 / 20.8 / 28.1).  Against the best of all tiles and shares, over seven shapes from 300x1024 to 14336x4096 and 32000x2048 with 24 to
-// 512 tokens, F16 loses 1.0 % on average, most at 24 tokens (14336x4096 51 against 45 us) and 7 % at worst above; F32, over seven
-// shapes with 40 to 512 tokens, 1.1 % and 6 %.
+// 512 tokens, F16 loses 0.3 % on average and 10 % at worst (6144x4096, 512 tokens); F32, over seven shapes with 40 to 512 tokens, 1.1 and
+// 6 %.
 static void pg_plan(const MatView &m, uint32_t tokens, PgPlan &p) {
     static constexpr uint32_t tile[3] = {32, 64, 128};
     static constexpr double price[2][2][3] = {{{0.47, 0.69, 1.25}, {0.55, 0.8, 1.39}}, {{0.36, 0.5, 1.55}, {0.48, 0.6, 1.5}}};  // [F16][alone]
@@ -1008,8 +1008,8 @@ static void pg_plan(const MatView &m, uint32_t tokens, PgPlan &p) {
 
 // The most workspace such a product asks for: cut activations take 6 bytes a value, held as long as the executor lives,
 // where the f32 instruction takes none.  Pieces of this size cost nothing (16384 tokens by 4096x14336, 1.4 GB whole:
-// F16 6.3 -> 5.9 ms in two pieces, F32 14.0 -> 13.4), of a quarter of it 7-25 % (8192 tokens in three pieces: F16 3.02 ->
-// 3.82 ms, F32 6.99 -> 7.45), the last round of workgroups of each piece being partly empty.
+// F16 6.1 -> 5.7 ms in two pieces, F32 14.0 -> 13.4), of a quarter of it 7-24 % (8192 tokens in three pieces: F16 2.93 ->
+// 3.63 ms, F32 6.99 -> 7.45), the last round of workgroups of each piece being partly empty.
 constexpr size_t PG_WS_BYTES = (size_t)1 << 30;
 
 // Tokens per piece of a product that is given less workspace than its plan takes: pieces of whole tiles, as equal as
@@ -1017,7 +1017,7 @@ constexpr size_t PG_WS_BYTES = (size_t)1 << 30;
 // results are those of the whole product bit for bit, and a piece of fewer tokens takes less (a plan of its own would
 // share its columns more finely and could take more).  Narrower tiles where not even one fits.  0: pieces would have
 // fewer than 64 tokens, and reading the weights that often costs more than the f32 instruction does (F16 4096x14336:
-// 45 us per 32 tokens, 48 per 64; the f32 instruction 80 per 64 of 128).
+// 41 us per 32 tokens, 48 per 64; the f32 instruction 80 per 64 of 128).
 static uint32_t pg_piece(PgPlan &p, size_t ws_bytes) {
     const PgJob &j = p.job;
     if (ws_bytes > PG_WS_BYTES) ws_bytes = PG_WS_BYTES;
@@ -1113,9 +1113,9 @@ static hipError_t launch_few_t(hipStream_t stream, const MatView &m, uint32_t to
 // 1024x8192 13.4 / 13.7, 1024x14336 21.5 / 19.0, with 16 tokens 1024x6144 14.0 / 14.4, 1024x8192 16.7 / 14.9; F32
 // 512x2048 5.9 / 10.6, 1024x6144 with 16 tokens 17.2 / 15.3).  17 to 32 tokens take twice the matrix-core time:
 // 512x3072 with 20 11.8 / 13.2 (F32 12.8 / 12.8), F32 512x4096 16.1 / 13.9, F32 4096x4096 with 32 18.7 / 23.3, 3072x8192 33.5 / 32.3.
-// F16 matrices of 2^23 weights and more meet launch_pg there: 4096x4096 with 32 17.1 / 21.1, 2048x4096 15.6 / 17.3, 2048x6144
-// 21.5 / 20.4, 2048x8192 with 20 27.3 / 21.1, 4096x8192 with 32 29.8 / 31.6, 8192x4096 30.6 / 31.1, 14336x4096 with 17 54.6 / 44.1,
-// 4096x14336 with 20 46.9 / 43.0.
+// F16 matrices of 2^23 weights and more meet launch_pg there: 4096x4096 with 32 17.1 / 19.8, 2048x4096 15.7 / 14.8, 2048x6144
+// 21.6 / 17.0, 2048x8192 with 20 27.4 / 20.1, 4096x8192 with 32 29.8 / 29.1, 8192x4096 30.3 / 28.7, 14336x4096 with 17 55.2 / 40.7,
+// 4096x14336 with 20 47.2 / 39.8.
 static bool few_takes(const MatView &m, uint32_t tokens) {
     if ((m.type != T_F32 && m.type != T_F16) || tokens < 2 || tokens > 32 || skinny_pays(m, tokens)) return false;
     const uint32_t tiles = (m.rows + 15) / 16, cus = (uint32_t)g_cu_count;
