@@ -608,12 +608,47 @@ struct MmPlan {
     bool tile16;        // 16-token tiles (gemm_mfma16_kernel) instead
     bool tile16x2;      // Q4_K, 17 to 32 tokens: gemm_mfma16_kernel with two 16-token tiles per workgroup (planned as a 32-token tile)
     uint32_t max_tok;   // most tokens of any job
+    // gemm_whole_kernel: sets of 16 rows and wavefronts of a workgroup; 0: columns are shared between workgroups
+    uint32_t whole_sets, whole_waves;
     uint32_t n_groups;  // groups of 16 columns
     size_t xb_bytes, sx_bytes, part_bytes;
 };
 
 // Most tokens of a job that the 16-token kernel takes (Q6_K fills its rows with 8).
 static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
+
+// Whether whole rows to a workgroup (gemm_whole_kernel) beat columns shared between workgroups, whose launches take shares_us by the
+// estimate below: a launch, and the steps of the CU that gets most, sixteen wavefronts at a time.  16 rows to a workgroup where that leaves
+// no CU a second one, then 32, then 64: fewer rows to a wavefront are spread over more CUs, more are decoded behind each cutting of the
+// activations.  Eight wavefronts where a CU gets two workgroups or sixteen would have less than four steps each, four where both is so.
+// The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens: by this rule they are
+// 1.27 times as fast in the geometric mean as with shared columns alone (Q4_0 at 8 tokens, shared / whole, us: 4096x1024 9.2 / 4.9, 4096x4096
+// 10.5 / 8.1, 8192x8192 18.6 / 16.5, 14336x4096 16.7 / 13.5, 32000x4096 27.6 / 23.7, but 1024x14336 12.5 / 15.5), none slower by more than
+// 5 %.  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6), and where a CU gets two of its workgroups
+// the products of a chain (launch_gemm_act), whose sums another launch reads in either case, lose more than those alone gain ([gate,up] of eight
+// sequences, 28672x4096, with the launch behind it 27.9 / 30.2, 32000x4096 with 4 tokens alone 25.0 / 21.8): the same choice for both, as their sums are the
+// same bits.
+struct WholePlan { uint32_t sets, waves; };
+static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats, uint32_t n, double shares_us) {
+    size_t rows = 0;
+    for (uint32_t j = 0; j < n; j++) rows += mats[j].rows;
+    const size_t cus = (size_t)g_cu_count;
+    const bool eight = max_tok <= 8;
+    WholePlan p;
+    p.sets = rows <= 16 * cus ? 1 : rows <= 32 * cus ? 2 : 4;
+    if (n > (uint32_t)MM_FEW_JOBS || (type == T_Q4_K && !eight && p.sets == 4)) return WholePlan{0, 0};
+    size_t tiles = 0;
+    for (uint32_t j = 0; j < n; j++) tiles += (mats[j].rows + 16 * p.sets - 1) / (16 * p.sets);
+    const uint32_t steps = mats[0].cols / 32;
+    const bool twice = tiles > cus;
+    if (type == T_Q4_K && p.sets == 4 && twice) return WholePlan{0, 0};
+    p.waves = twice && steps <= 32 ? 4 : twice || steps < 64 ? 8 : 16;
+    if (type == T_Q4_K && !eight && p.waves > 8) p.waves = 8;  // LDS
+    static constexpr double step_us[2][3] = {{0.76, 1.02, 1.5}, {0.46, 0.72, 1.22}};  // [eight][sets]
+    const double dtype = type == T_Q6_K ? 1.35 : type == T_Q5_1 ? 1.15 : type != T_Q4_K ? 1.0 : eight ? 1.1 : 1.2;
+    const double us = 4.6 + (double)((tiles + cus - 1) / cus) * steps / 16.0 * step_us[eight][p.sets / 2] * dtype;
+    return us < 0.96 * shares_us ? p : WholePlan{0, 0};
+}
 
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
@@ -670,6 +705,11 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
             ks_launch = ks;
         }
     }
+    WholePlan whole{0, 0};
+    if (p.tile16) whole = whole_plan(mats[0].type, max_tok, mats, n, max_tok <= 8 ? 3.2 + 0.88 * step_us * best : 2.6 + step_us * best);
+    p.whole_sets = whole.sets;
+    p.whole_waves = whole.waves;
+    const uint32_t wg_rows = whole.sets ? 16 * whole.sets : (uint32_t)MM_ROWS;
     for (uint32_t j = 0; j < n; j++) {
         MmJob &job = b.job[j];
         job.m = mats[j];
@@ -683,8 +723,8 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
         job.tok_off = total_tok;
         job.wg_begin = wgs;
         job.tok_tiles = (tokens[j] + tile_tok - 1) / tile_tok;
-        const uint32_t tiles = job.tok_tiles * ((mats[j].rows + MM_ROWS - 1) / MM_ROWS);
-        uint32_t ks = ks_launch;
+        const uint32_t tiles = job.tok_tiles * ((mats[j].rows + wg_rows - 1) / wg_rows);
+        const uint32_t ks = whole.sets ? 1 : ks_launch;
         job.ksplit = ks;
         job.pad = 0;
         wgs += tiles * ks;
@@ -701,9 +741,10 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     p.n_groups = mats[0].cols / 16;
     p.xb_bytes = up256((size_t)p.n_groups * 6 * b.mpad * sizeof(uint4));
     p.sx_bytes = up256((size_t)p.n_groups * b.mpad * sizeof(float));
+    // (asked for as if columns were shared also where they are not: what a caller without room for it is told does not depend on that)
     size_t part = 0;
     for (uint32_t j = 0; j < n; j++)
-        if (b.job[j].ksplit > 1) part += up256((size_t)b.job[j].ksplit * tokens[j] * mats[j].rows * sizeof(float));
+        if (ks_launch > 1) part += up256((size_t)ks_launch * tokens[j] * mats[j].rows * sizeof(float));
     p.part_bytes = part;
 }
 
@@ -799,6 +840,44 @@ static hipError_t launch_mm16_main(hipStream_t stream, const MmBatch &b, uint32_
     return launch_mm16_lo<T, INLINE, false, NORM, NT, 3>(stream, b);
 }
 
+// Up to 16 tokens, whole rows to a workgroup.
+template <uint32_t T, int RS, int LO, int FROM, bool FB = false> static hipError_t launch_whole_lo(hipStream_t stream, const MmPlan &p) {
+    if constexpr (T == T_Q4_K && !FB) {
+        if (p.b.nibble_bf16) return launch_whole_lo<T, RS, LO, FROM, true>(stream, p);
+    }
+    if constexpr (T == T_Q4_0 && !FB) {
+        if (g_nibble_i4) return launch_whole_lo<T, RS, LO, FROM, true>(stream, p);
+    }
+    constexpr uint32_t most = MwTraits<T, LO>::lds_bytes(RS, 16);
+    const uint32_t lds = MwTraits<T, LO>::lds_bytes(RS, p.whole_waves);
+    static_assert(most <= 160 * 1024 || MwTraits<T, LO>::lds_bytes(RS, 8) <= 160 * 1024, "the LDS of a CU");
+    if (lds > 48 * 1024) {
+        static DeviceOnce limit;  // per instantiation
+        const hipError_t e = allow_lds(limit, reinterpret_cast<const void *>(gemm_whole_kernel<T, FB, RS, LO, FROM>), most < 160 * 1024 ? most : 160 * 1024);
+        if (e != hipSuccess) return e;
+    }
+    MmFewBatch few;
+    static_cast<MmHead &>(few) = p.b;
+    std::memcpy(few.job, p.b.job, sizeof(few.job));
+    hipLaunchKernelGGL((gemm_whole_kernel<T, FB, RS, LO, FROM>), dim3(p.b.total_wgs), dim3(64 * p.whole_waves), lds, stream, few);
+    return hipGetLastError();
+}
+template <uint32_t T, int FROM = MW_PLAIN> static hipError_t launch_whole(hipStream_t stream, const MmPlan &p) {
+    auto by_parts = [&](auto sets) {
+        constexpr int RS = decltype(sets)::value;
+        if constexpr (T != T_Q6_K) {
+            if (p.max_tok <= 8) return launch_whole_lo<T, RS, 2, FROM>(stream, p);
+        }
+        if constexpr (T == T_Q4_K && RS == 4) return hipErrorInvalidValue;
+        else return launch_whole_lo<T, RS, 3, FROM>(stream, p);
+    };
+    switch (p.whole_sets) {
+    case 1: return by_parts(std::integral_constant<int, 1>{});
+    case 2: return by_parts(std::integral_constant<int, 2>{});
+    default: return by_parts(std::integral_constant<int, 4>{});
+    }
+}
+
 // Workgroups per job of the share reduction: one float4 per thread (one float for small jobs, as the kernel
 // chooses) where that fills fewer than 512.
 static uint32_t mm_reduce_blocks(const MmBatch &b) {
@@ -832,6 +911,7 @@ static hipError_t launch_mm_t(hipStream_t stream, MmPlan &p, void *ws, size_t ws
             part += up256((size_t)b.job[j].ksplit * b.job[j].tokens * b.job[j].m.rows * sizeof(float));
         }
     hipError_t e;
+    if (p.whole_sets) return launch_whole<T>(stream, p);
     if (p.tile16) {  // the 16-token kernel cuts the activations itself
         e = launch_mm16_main<T, true>(stream, b, p.max_tok);
         if (e != hipSuccess) return e;
@@ -1426,6 +1506,8 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     }
     hipError_t e = mm_by_type(tiled[0].type, [&](auto t) {
         constexpr uint32_t T = decltype(t)::value;
+        if (p.whole_sets)
+            return norm ? launch_whole<T, MW_NORM>(stream, p) : x_plain ? launch_whole<T>(stream, p) : launch_whole<T, MW_CUT>(stream, p);
         if (p.tile16 && norm) return launch_mm16_main<T, true, true>(stream, b, p.max_tok);
         if (p.tile16) return x_plain ? launch_mm16_main<T, true>(stream, b, p.max_tok) : launch_mm16_main<T>(stream, b, p.max_tok);
         if constexpr (T == T_Q4_K) {
