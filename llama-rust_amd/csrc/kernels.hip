@@ -628,25 +628,39 @@ static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
 // the products of a chain (launch_gemm_act), whose sums another launch reads in either case, lose more than those alone gain ([gate,up] of eight
 // sequences, 28672x4096, with the launch behind it 27.9 / 30.2, 32000x4096 with 4 tokens alone 25.0 / 21.8): the same choice for both, as their sums are the
 // same bits.
+// More tokens are tiles of 16 (Q6_K: 8), each a workgroup's, that decode the weights anew: against two or three launches that pays while
+// there is not much to decode (shared / whole, us, Q4_0: 512x2048 at 32 tokens 11.1 / 6.5, at 40 17.1 / 6.6, 1024x4096 at 17 11.1 / 9.1, at 100
+// 22.0 / 11.3, 2048x4096 at 64 21.9 / 12.1, 4096x4096 at 32 15.4 / 12.0, Q4_K 1024x2048 at 64 18.2 / 8.0, 2048x2048 at 100 21.8 / 15.3; 1.7 in the
+// geometric mean over 46 matrices from 256x1024 to 16384x512 at 17 to 160 tokens), and every round of workgroups after the first costs
+// its start (Q4_K 16384x512 at 17 12.9 / 15.5, Q4_0 at 160 23.4 / 25.7).  There the wavefronts depend on the columns alone, so that products
+// of one launch and of several are the same bits.
 struct WholePlan { uint32_t sets, waves; };
-static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats, uint32_t n, double shares_us) {
+static uint32_t whole_slots(uint32_t type, uint32_t max_tok) { return max_tok <= 8 || type == T_Q6_K ? 8 : 16; }
+static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats, const uint32_t *tokens, uint32_t n, double shares_us) {
+    const bool eight = max_tok <= 8 || type == T_Q6_K;
+    const uint32_t slots = whole_slots(type, max_tok);
+    auto tok_tiles = [&](uint32_t j) { return (size_t)((tokens[j] + slots - 1) / slots); };
     size_t rows = 0;
-    for (uint32_t j = 0; j < n; j++) rows += mats[j].rows;
+    for (uint32_t j = 0; j < n; j++) rows += mats[j].rows * tok_tiles(j);
     const size_t cus = (size_t)g_cu_count;
-    const bool eight = max_tok <= 8;
+    const bool several = max_tok > slots;  // token tiles
     WholePlan p;
     p.sets = rows <= 16 * cus ? 1 : rows <= 32 * cus ? 2 : 4;
-    if (n > (uint32_t)MM_FEW_JOBS || (type == T_Q4_K && !eight && p.sets == 4)) return WholePlan{0, 0};
+    if (n > (uint32_t)MM_FEW_JOBS) return WholePlan{0, 0};
+    if (type == T_Q4_K && !eight && p.sets == 4) p.sets = 2;  // registers
     size_t tiles = 0;
-    for (uint32_t j = 0; j < n; j++) tiles += (mats[j].rows + 16 * p.sets - 1) / (16 * p.sets);
+    for (uint32_t j = 0; j < n; j++) tiles += (mats[j].rows + 16 * p.sets - 1) / (16 * p.sets) * tok_tiles(j);
     const uint32_t steps = mats[0].cols / 32;
     const bool twice = tiles > cus;
     if (type == T_Q4_K && p.sets == 4 && twice) return WholePlan{0, 0};
-    p.waves = twice && steps <= 32 ? 4 : twice || steps < 64 ? 8 : 16;
+    if (several) p.waves = steps < 64 ? 8 : 16;
+    else p.waves = twice && steps <= 32 ? 4 : twice || steps < 64 ? 8 : 16;
     if (type == T_Q4_K && !eight && p.waves > 8) p.waves = 8;  // LDS
     static constexpr double step_us[2][3] = {{0.76, 1.02, 1.5}, {0.46, 0.72, 1.22}};  // [eight][sets]
     const double dtype = type == T_Q6_K ? 1.35 : type == T_Q5_1 ? 1.15 : type != T_Q4_K ? 1.0 : eight ? 1.1 : 1.2;
-    const double us = 4.6 + (double)((tiles + cus - 1) / cus) * steps / 16.0 * step_us[eight][p.sets / 2] * dtype;
+    const size_t rounds = (tiles + cus - 1) / cus;
+    double us = 4.6 + (double)rounds * steps / 16.0 * step_us[eight][p.sets / 2] * dtype;
+    if (several) us += (double)(rounds - 1) * (type == T_Q4_K ? 2.0 : 1.0);
     return us < 0.96 * shares_us ? p : WholePlan{0, 0};
 }
 
@@ -706,7 +720,8 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
         }
     }
     WholePlan whole{0, 0};
-    if (p.tile16) whole = whole_plan(mats[0].type, max_tok, mats, n, max_tok <= 8 ? 3.2 + 0.88 * step_us * best : 2.6 + step_us * best);
+    if (p.tile16) whole = whole_plan(mats[0].type, max_tok, mats, tokens, n, max_tok <= 8 ? 3.2 + 0.88 * step_us * best : 2.6 + step_us * best);
+    else whole = whole_plan(mats[0].type, max_tok, mats, tokens, n, (p.tt == 2 ? 2.0 : 3.5) + step_us * best);
     p.whole_sets = whole.sets;
     p.whole_waves = whole.waves;
     const uint32_t wg_rows = whole.sets ? 16 * whole.sets : (uint32_t)MM_ROWS;
@@ -723,6 +738,7 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
         job.tok_off = total_tok;
         job.wg_begin = wgs;
         job.tok_tiles = (tokens[j] + tile_tok - 1) / tile_tok;
+        if (whole.sets) job.tok_tiles = (tokens[j] + whole_slots(mats[0].type, max_tok) - 1) / whole_slots(mats[0].type, max_tok);
         const uint32_t tiles = job.tok_tiles * ((mats[j].rows + wg_rows - 1) / wg_rows);
         const uint32_t ks = whole.sets ? 1 : ks_launch;
         job.ksplit = ks;

@@ -1,4 +1,4 @@
-"""Products of 3 to 16 tokens whose workgroups own whole rows (gemm_whole_kernel, csrc/gemm_kernels.inc), against the oracle's float64
+"""Products whose workgroups own whole rows (gemm_whole_kernel, csrc/gemm_kernels.inc), against the oracle's float64
 product.
 
 Tolerances as in test_gpu_parity.py: the proven bound of any f32 summation order and the reference's observed envelope, both relative
@@ -42,6 +42,23 @@ def test_edges(gpu, ty, rows, cols):
     for tokens in (3, 8, 9, 16):
         x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
         x[0, ::7] *= 3.0e4
+        y = np.full(tokens * rows, np.nan, np.float32)
+        gpu.gemm_resident(m, tokens, x.reshape(-1), y)
+        _check(ty, rows, cols, x, w, y)
+    m.close()
+
+
+@pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (300, 2080), (4097, 288), (8255, 160)])
+def test_token_tiles(gpu, ty, rows, cols):
+    """More tokens than a tile has slots: last tiles of one token, of all but one, and whole ones."""
+    cols = (cols + K.QK[ty] - 1) // K.QK[ty] * K.QK[ty]
+    rng = np.random.default_rng(5 * rows + cols + ty)
+    w = K.random_packed(ty, rows, cols, rng)
+    m = gpu.upload_packed(ty, rows, cols, w)
+    for tokens in (9, 17, 31, 64, 65):
+        x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+        x[-1, ::7] *= 3.0e4
         y = np.full(tokens * rows, np.nan, np.float32)
         gpu.gemm_resident(m, tokens, x.reshape(-1), y)
         _check(ty, rows, cols, x, w, y)
