@@ -856,7 +856,7 @@ static hipError_t launch_mm16_main(hipStream_t stream, const MmBatch &b, uint32_
     return launch_mm16_lo<T, INLINE, false, NORM, NT, 3>(stream, b);
 }
 
-// Up to 16 tokens, whole rows to a workgroup.
+// Whole rows to a workgroup (whole_plan).
 template <uint32_t T, int RS, int LO, int FROM, bool FB = false> static hipError_t launch_whole_lo(hipStream_t stream, const MmPlan &p) {
     if constexpr (T == T_Q4_K && !FB) {
         if (p.b.nibble_bf16) return launch_whole_lo<T, RS, LO, FROM, true>(stream, p);
