@@ -624,7 +624,8 @@ static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
 // The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens: by this rule they are
 // 1.27 times as fast in the geometric mean as with shared columns alone (Q4_0 at 8 tokens, shared / whole, us: 4096x1024 9.2 / 4.9, 4096x4096
 // 10.5 / 8.1, 8192x8192 18.6 / 16.5, 14336x4096 16.7 / 13.5, 32000x4096 27.6 / 23.7, but 1024x14336 12.5 / 15.5), none slower by more than
-// 5 %.  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6), and where a CU gets two of its workgroups
+// 5 %.  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6): 32 rows there (16384x1024 at 12 tokens 11.4 / 8.9,
+// 12288x1024 at 16 11.2 / 9.0); and where a CU gets two of its workgroups
 // the products of a chain (launch_gemm_act), whose sums another launch reads in either case, lose more than those alone gain ([gate,up] of eight
 // sequences, 28672x4096, with the launch behind it 27.9 / 30.2, 32000x4096 with 4 tokens alone 25.0 / 21.8): the same choice for both, as their sums are the
 // same bits.
