@@ -610,6 +610,7 @@ struct MmPlan {
     uint32_t max_tok;   // most tokens of any job
     // gemm_whole_kernel: sets of 16 rows and wavefronts of a workgroup; 0: columns are shared between workgroups
     uint32_t whole_sets, whole_waves;
+    uint32_t shares;    // column shares of a row (planned also where whole rows are taken instead)
     uint32_t n_groups;  // groups of 16 columns
     size_t xb_bytes, sx_bytes, part_bytes;
 };
@@ -725,6 +726,7 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     else whole = whole_plan(mats[0].type, max_tok, mats, tokens, n, (p.tt == 2 ? 2.0 : 3.5) + step_us * best);
     p.whole_sets = whole.sets;
     p.whole_waves = whole.waves;
+    p.shares = ks_launch;
     const uint32_t wg_rows = whole.sets ? 16 * whole.sets : (uint32_t)MM_ROWS;
     for (uint32_t j = 0; j < n; j++) {
         MmJob &job = b.job[j];
@@ -1429,7 +1431,9 @@ hipError_t launch_act_split(hipStream_t stream, void *act, uint32_t type, uint32
 
 // The plan of n products (one dtype, one column count) of the same split activations, `tokens` tokens each.
 // forced_shares: every job writes shares (one when its columns are not shared) into the workspace, for an
-// epilogue launch to sum; otherwise jobs without shared columns write ys directly.
+// epilogue launch to sum; otherwise jobs without shared columns write ys directly.  The workspace has room for the
+// planned shares also where whole rows leave one: what a captured stream is granted (a product no larger than one
+// that has run) does not depend on which way either of them goes.
 static bool act_plan(const MatView *tiled, uint32_t n, uint32_t tokens, float *const *ys, bool forced_shares, MmPlan &p) {
     if (n == 0 || n > (uint32_t)MM_MAX_JOBS || tokens < MM_MIN_TOKENS || !mm_type(tiled[0].type)) return false;
     for (uint32_t j = 1; j < n; j++)
@@ -1444,10 +1448,7 @@ static bool act_plan(const MatView *tiled, uint32_t n, uint32_t tokens, float *c
     mm_plan(tiled, toks, xs, ys, n, p);
     if (forced_shares) {
         size_t part = 0;
-        for (uint32_t j = 0; j < n; j++) {
-            const uint32_t ks = p.b.job[j].ksplit > 1 ? p.b.job[j].ksplit : 1;
-            part += up256((size_t)ks * tokens * tiled[j].rows * sizeof(float));
-        }
+        for (uint32_t j = 0; j < n; j++) part += up256((size_t)p.shares * tokens * tiled[j].rows * sizeof(float));
         p.part_bytes = part;
     }
     return true;

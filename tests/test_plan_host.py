@@ -1,0 +1,42 @@
+"""What the plan of multi-token products decides, on the CPU: it is a function of shapes, token counts and the CU count (256 before a
+device has set it), so no device is needed.  Reached through the library's own C++ symbols."""
+import ctypes as C
+
+import pytest
+
+import cases as K
+import oracle as O
+
+QUANTIZED = [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K, K.Q6_K]
+
+
+class MatView(C.Structure):  # csrc/matview.h
+    _fields_ = [("p", C.c_void_p * 4), ("s", C.c_uint32 * 4), ("type", C.c_uint32), ("rows", C.c_uint32), ("cols", C.c_uint32), ("nb", C.c_uint32)]
+
+
+def views(ty, rows, cols):
+    mats = (MatView * len(rows))()
+    for m, r in zip(mats, rows):
+        m.type, m.rows, m.cols = ty, r, cols
+    return mats
+
+
+@pytest.fixture(scope="module")
+def act_workspace(lib):
+    f = getattr(lib, "_ZN2nh24gemm_act_workspace_bytesEPKNS_7MatViewEjjbb")
+    f.restype, f.argtypes = C.c_size_t, [C.POINTER(MatView), C.c_uint32, C.c_uint32, C.c_bool, C.c_bool]
+
+    def workspace(ty, rows, cols, tokens, epilogue):
+        return f(views(ty, rows, cols), len(rows), tokens, epilogue, False)
+    return workspace
+
+
+@pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
+def test_an_epilogue_asks_for_all_planned_shares(act_workspace, ty):
+    """A chain's product asks for the workspace of its planned column shares whether or not it then takes whole rows, as the same
+    product without an epilogue does; a job whose columns are not shared needs one share for the epilogue to read."""
+    for rows, cols in (([4096], 4096), ([512], 512), ([1024], 14336), ([2048, 2048], 2048), ([14336, 14336], 4096), ([32000], 1024)):
+        for tokens in (3, 8, 9, 16, 17, 32, 33, 160):
+            plain, with_epilogue = act_workspace(ty, rows, cols, tokens, False), act_workspace(ty, rows, cols, tokens, True)
+            one = sum((tokens * r * 4 + 255) // 256 * 256 for r in rows)
+            assert with_epilogue == max(plain, one), (rows, cols, tokens)
