@@ -32,6 +32,12 @@ hipError_t launch_retile(hipStream_t stream, const MatView &tiled, const MatView
 // Products of F32 / F16 weights cut the activations of many tokens into the workspace; given less than that takes they
 // go out in pieces of fewer tokens or on a kernel that cuts nothing.  least: what a call cannot do without.
 size_t gemm_workspace_bytes(const MatView *mats, const uint32_t *tokens, uint32_t n, bool least = false);
+// What the plan of one multi-token launch (one quantized dtype and column count) does: rows and wavefronts of a workgroup that owns whole
+// rows, zeros where columns are shared between workgroups.  xs and ys may be null (they say whether a product writes over its input).
+struct WholeRows {
+    uint32_t rows, waves;
+};
+WholeRows planned_whole_rows(const MatView *mats, const uint32_t *tokens, const float *const *xs, float *const *ys, uint32_t n);
 hipError_t launch_gemm(hipStream_t stream, const MatView &m, const MatView &tiled, uint32_t tokens, const float *x,
                        float *y, void *ws, size_t ws_bytes);
 // n independent products (the experts of one MoE projection, say): consecutive

@@ -666,6 +666,19 @@ static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats
     return us < 0.96 * shares_us ? p : WholePlan{0, 0};
 }
 
+// Whether a product of a launch writes where one of them reads.  Kernels that cut plain activations while other workgroups already
+// store results must not have that; launches whose results leave the workspace only after the last of them has read x may.
+static bool writes_over_inputs(const MatView *mats, const uint32_t *tokens, const float *const *xs, float *const *ys, uint32_t n) {
+    for (uint32_t i = 0; i < n; i++)
+        for (uint32_t j = 0; j < n; j++) {
+            if (!xs[i] || !ys[j]) continue;
+            const uintptr_t x = reinterpret_cast<uintptr_t>(xs[i]), y = reinterpret_cast<uintptr_t>(ys[j]);
+            const size_t x_bytes = (size_t)tokens[i] * mats[i].cols * sizeof(float), y_bytes = (size_t)tokens[j] * mats[j].rows * sizeof(float);
+            if (x < y + y_bytes && y < x + x_bytes) return true;
+        }
+    return false;
+}
+
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Jobs share dtype and column count; every job has at least MM_MIN_TOKENS tokens.
@@ -724,6 +737,7 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     WholePlan whole{0, 0};
     if (p.tile16) whole = whole_plan(mats[0].type, max_tok, mats, tokens, n, max_tok <= 8 ? 3.2 + 0.88 * step_us * best : 2.6 + step_us * best);
     else whole = whole_plan(mats[0].type, max_tok, mats, tokens, n, (p.tt == 2 ? 2.0 : 3.5) + step_us * best);
+    if (whole.sets && xs && ys && writes_over_inputs(mats, tokens, xs, ys, n)) whole = WholePlan{0, 0};
     p.whole_sets = whole.sets;
     p.whole_waves = whole.waves;
     p.shares = ks_launch;
@@ -765,6 +779,13 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     for (uint32_t j = 0; j < n; j++)
         if (ks_launch > 1) part += up256((size_t)ks_launch * tokens[j] * mats[j].rows * sizeof(float));
     p.part_bytes = part;
+}
+
+WholeRows planned_whole_rows(const MatView *mats, const uint32_t *tokens, const float *const *xs, float *const *ys, uint32_t n) {
+    if (n == 0 || n > (uint32_t)MM_MAX_JOBS || !mm_type(mats[0].type)) return WholeRows{0, 0};
+    MmPlan p;
+    mm_plan(mats, tokens, xs, ys, n, p);
+    return WholeRows{16 * p.whole_sets, p.whole_waves};
 }
 
 // Launches f(arguments, their size as a constant) with room for as many jobs as the batch has.
@@ -1434,16 +1455,15 @@ hipError_t launch_act_split(hipStream_t stream, void *act, uint32_t type, uint32
 // epilogue launch to sum; otherwise jobs without shared columns write ys directly.  The workspace has room for the
 // planned shares also where whole rows leave one: what a captured stream is granted (a product no larger than one
 // that has run) does not depend on which way either of them goes.
-static bool act_plan(const MatView *tiled, uint32_t n, uint32_t tokens, float *const *ys, bool forced_shares, MmPlan &p) {
+static bool act_plan(const MatView *tiled, uint32_t n, uint32_t tokens, const float *x_plain, float *const *ys, bool forced_shares, MmPlan &p) {
     if (n == 0 || n > (uint32_t)MM_MAX_JOBS || tokens < MM_MIN_TOKENS || !mm_type(tiled[0].type)) return false;
     for (uint32_t j = 1; j < n; j++)
         if (tiled[j].type != tiled[0].type || tiled[j].cols != tiled[0].cols) return false;
     uint32_t toks[MM_MAX_JOBS];
     const float *xs[MM_MAX_JOBS];
-    static const float same_x = 0.f;  // any one address: the jobs then share their split slots
     for (uint32_t j = 0; j < n; j++) {
         toks[j] = tokens;
-        xs[j] = &same_x;
+        xs[j] = x_plain;  // one address (null: split already): the jobs share their split slots
     }
     mm_plan(tiled, toks, xs, ys, n, p);
     if (forced_shares) {
@@ -1456,7 +1476,7 @@ static bool act_plan(const MatView *tiled, uint32_t n, uint32_t tokens, float *c
 
 size_t gemm_act_workspace_bytes(const MatView *mats, uint32_t n, uint32_t tokens, bool with_epilogue, bool plain_x) {
     MmPlan p;
-    if (!act_plan(mats, n, tokens, nullptr, with_epilogue, p)) return 0;
+    if (!act_plan(mats, n, tokens, nullptr, nullptr, with_epilogue, p)) return 0;
     // plain activations of more than 32 tokens are cut into the workspace first
     return p.part_bytes + (plain_x && p.tt == 2 ? p.xb_bytes + p.sx_bytes : 0);
 }
@@ -1471,7 +1491,7 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     if (fused && (ep.kind == ACT_EPILOGUE_SWIGLU ? n != 2 : n != 1)) return hipErrorInvalidValue;
     if (!fused && !ys) return hipErrorInvalidValue;
     MmPlan p;
-    if (!act_plan(tiled, n, tokens, fused ? nullptr : ys, fused, p)) return hipErrorInvalidValue;
+    if (!act_plan(tiled, n, tokens, x_plain, fused ? nullptr : ys, fused, p)) return hipErrorInvalidValue;
     const bool cut_first = x_plain && p.tt == 2;  // plain activations of more than 32 tokens: mm_xsplit into the workspace
     const size_t split_bytes = cut_first ? p.xb_bytes + p.sx_bytes : 0;
     if (p.part_bytes + split_bytes > ws_bytes) return hipErrorInvalidValue;
@@ -1480,12 +1500,9 @@ hipError_t launch_gemm_act(hipStream_t stream, const MatView *tiled, uint32_t n,
     if (!x_plain) {
         in = act_view(act, tiled[0].type, tiled[0].cols, act_max_tokens, tokens);
         if (in.mpad != b.mpad) return hipErrorInvalidValue;  // the plan's slots and the buffer's must be the same thing
-    } else {
-        for (uint32_t j = 0; j < b.n_jobs; j++) b.job[j].x = x_plain;
-        if (cut_first) {
-            in.xb = static_cast<uint4 *>(ws);
-            in.sx = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + p.xb_bytes);
-        }
+    } else if (cut_first) {
+        in.xb = static_cast<uint4 *>(ws);
+        in.sx = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + p.xb_bytes);
     }
     const uint32_t rows = tiled[0].rows;
     ActView next{};

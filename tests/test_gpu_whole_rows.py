@@ -81,3 +81,25 @@ def test_matrices_of_one_launch(gpu, ty):
         at += r * t
     for m in ms:
         m.close()
+
+
+@pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("shift", [0, 4 * 1024])
+def test_results_over_the_input(pkg, gpu, ty, shift):
+    """y in x's place, and reaching into it: more than 32 tokens of a square matrix, whose activations are cut before anything is stored."""
+    import importlib
+    hip = importlib.import_module("llama-rust_amd.hiprt")
+    n = 1024
+    rng = np.random.default_rng(70 + ty)
+    w = K.random_packed(ty, n, n, rng)
+    m = gpu.upload_packed(ty, n, n, w)
+    for tokens in (33, 64):
+        x = rng.normal(0, 1, (tokens, n)).astype(np.float32)
+        both = np.zeros(tokens * n + shift, np.float32)
+        both[shift:] = x.reshape(-1)
+        buf = hip.DeviceBuffer.from_numpy(both)
+        gpu.gemm_device(m, tokens, buf.ptr + 4 * shift, buf.ptr)
+        gpu.synchronize()
+        _check(ty, n, n, x, w, buf.to_numpy(np.float32)[:tokens * n])
+        buf.free()
+    m.close()

@@ -31,6 +31,40 @@ def act_workspace(lib):
     return workspace
 
 
+@pytest.fixture(scope="module")
+def whole_rows(lib):
+    """(rows, wavefronts) of a workgroup that owns whole rows, (0, 0) where columns are shared."""
+    f = getattr(lib, "_ZN2nh18planned_whole_rowsEPKNS_7MatViewEPKjPKPKfPKPfj")
+
+    class WholeRows(C.Structure):
+        _fields_ = [("rows", C.c_uint32), ("waves", C.c_uint32)]
+
+    f.restype = WholeRows
+
+    def plan(ty, rows, cols, tokens, xs=None, ys=None):
+        n = len(rows)
+        toks = (C.c_uint32 * n)(*(tokens if isinstance(tokens, (list, tuple)) else [tokens] * n))
+        p = f(views(ty, rows, cols), toks, (C.c_void_p * n)(*xs) if xs else None, (C.c_void_p * n)(*ys) if ys else None, C.c_uint32(n))
+        return p.rows, p.waves
+    return plan
+
+
+@pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
+def test_a_product_that_writes_over_its_input_shares_columns(whole_rows, ty):
+    """A workgroup that owns whole rows stores them while others still read x.  With shared columns and more than 32 tokens x is cut by a
+    launch of its own before any result is stored."""
+    n, x = 1024, 1 << 32
+    size = 4 * 64 * n
+    apart = whole_rows(ty, [n], n, 64, [x], [x + size])
+    assert apart[0] in (16, 32, 64) and apart == whole_rows(ty, [n], n, 64)
+    assert apart == whole_rows(ty, [n], n, 64, [x], [x - size])
+    for y in (x, x + 4, x + size - 4, x - size + 4):
+        assert whole_rows(ty, [n], n, 64, [x], [y]) == (0, 0)
+    # another product's input, in one launch
+    assert whole_rows(ty, [n, n], n, 64, [x, x + size], [x + 2 * size, x + 3 * size])[0] != 0
+    assert whole_rows(ty, [n, n], n, 64, [x, x + size], [x + 2 * size, x]) == (0, 0)
+
+
 @pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
 def test_an_epilogue_asks_for_all_planned_shares(act_workspace, ty):
     """A chain's product asks for the workspace of its planned column shares whether or not it then takes whole rows, as the same
