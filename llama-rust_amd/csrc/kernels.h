@@ -87,6 +87,8 @@ uint32_t head_candidates(const MatView &m);
 hipError_t launch_head(hipStream_t stream, const MatView &m, const float *x, const float *norm_w, float eps, float *y, float *cand_v,
                        uint32_t *cand_i);
 size_t act_bytes(uint32_t type, uint32_t cols, uint32_t max_tokens);
+// Token slots from one plane of cut activations of `tokens` tokens to the next.
+uint32_t act_slot_stride(uint32_t type, uint32_t tokens);
 hipError_t launch_act_split(hipStream_t stream, void *act, uint32_t type, uint32_t cols, uint32_t max_tokens, uint32_t tokens,
                             const float *x);
 // x_plain (with act == nullptr): the product's own activations are `tokens` plain f32 rows; up to 32 tokens the

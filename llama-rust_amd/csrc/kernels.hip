@@ -666,6 +666,13 @@ static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats
     return us < 0.96 * shares_us ? p : WholePlan{0, 0};
 }
 
+// Token slots from one plane of cut activations to the next.  A tile may read up to 15, 31 resp. 63 slots past its job's last token.  Up to
+// 32 tokens whole lines of 128 bytes: the eight slots that a quarter of gemm_whole_kernel's lanes reads of a plane are one line then
+// instead of two (down-like products of a chain, us: Q8_0 4096x8192 at 3 tokens 16.6 -> 14.3, Q4_0 15.6 -> 13.1, Q5_0 4096x4096 at
+// 17 14.0 -> 12.9; where columns are shared the same to 0.3).  Products of so few tokens cut their own activations unless they all read one
+// set, whose slots start at 0: up to 16 tokens need no slot more than their tile has.
+static uint32_t slot_stride(uint32_t slots, bool tile16, bool many) { return tile16 ? (slots + 15u) & ~15u : many ? slots + 64u : (slots + 64u) & ~7u; }
+
 // Whether a product of a launch writes where one of them reads.  Kernels that cut plain activations while other workgroups already
 // store results must not have that; launches whose results leave the workspace only after the last of them has read x may.
 static bool writes_over_inputs(const MatView *mats, const uint32_t *tokens, const float *const *xs, float *const *ys, uint32_t n) {
@@ -766,14 +773,16 @@ static void mm_plan(const MatView *mats, const uint32_t *tokens, const float *co
     }
     for (uint32_t j = n; j < (uint32_t)MM_FEW_JOBS; j++) b.job[j] = b.job[0];  // launches copy these too
     b.n_jobs = n;
-    b.mpad = total_tok + (p.tile16 ? 16 : 64);  // a tile may read up to 15 resp. 63 slots past its job's last token
+    b.mpad = slot_stride(total_tok, p.tile16, p.tt == 2);
     b.total_wgs = wgs;
     b.any_split = any_split ? 1u : 0u;
     b.nibble_bf16 = g_nibble_bf16 ? 1u : 0u;
     b.pad0 = b.pad1 = b.pad2 = 0;
     p.n_groups = mats[0].cols / 16;
-    p.xb_bytes = up256((size_t)p.n_groups * 6 * b.mpad * sizeof(uint4));
-    p.sx_bytes = up256((size_t)p.n_groups * b.mpad * sizeof(float));
+    // (room for a tile's slots behind the last token's, whatever the stride: what a call is granted does not depend on that)
+    const size_t room = total_tok + (p.tile16 ? 16u : 64u);
+    p.xb_bytes = up256((size_t)p.n_groups * 6 * room * sizeof(uint4));
+    p.sx_bytes = up256((size_t)p.n_groups * room * sizeof(float));
     // (asked for as if columns were shared also where they are not: what a caller without room for it is told does not depend on that)
     size_t part = 0;
     for (uint32_t j = 0; j < n; j++)
@@ -1398,7 +1407,7 @@ hipError_t launch_gemm_groups(hipStream_t stream, const MatView *mats, const Mat
 
 // ---- activations that stay in the split form between products
 
-static uint32_t act_mpad(uint32_t type, uint32_t tokens) { return tokens + (tokens <= mm_tile16_max(type) ? 16u : 64u); }
+uint32_t act_slot_stride(uint32_t type, uint32_t tokens) { return slot_stride(tokens, tokens <= mm_tile16_max(type), tokens > 32); }
 
 size_t act_bytes(uint32_t type, uint32_t cols, uint32_t max_tokens) {
     if (!mm_type(type) || cols % 32 != 0 || max_tokens == 0) return 0;
@@ -1413,7 +1422,7 @@ static ActView act_view(void *act, uint32_t type, uint32_t cols, uint32_t max_to
     const size_t n_groups = cols / 16;
     v.xb = static_cast<uint4 *>(act);
     v.sx = reinterpret_cast<float *>(static_cast<uint8_t *>(act) + up256(n_groups * 6 * ((size_t)max_tokens + 64) * sizeof(uint4)));
-    v.mpad = act_mpad(type, tokens);
+    v.mpad = act_slot_stride(type, tokens);
     v.n_groups = (uint32_t)n_groups;
     return v;
 }

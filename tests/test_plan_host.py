@@ -74,3 +74,16 @@ def test_an_epilogue_asks_for_all_planned_shares(act_workspace, ty):
             plain, with_epilogue = act_workspace(ty, rows, cols, tokens, False), act_workspace(ty, rows, cols, tokens, True)
             one = sum((tokens * r * 4 + 255) // 256 * 256 for r in rows)
             assert with_epilogue == max(plain, one), (rows, cols, tokens)
+
+
+@pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
+def test_cut_activations_start_on_lines(lib, ty):
+    """The planes of up to 32 tokens' cut activations (16 bytes a slot) are whole 128-byte lines apart; the slots of the last tile, 16, 32
+    or 64, are there, and a buffer made for so many tokens holds them."""
+    stride = getattr(lib, "_ZN2nh15act_slot_strideEjj")
+    stride.restype, stride.argtypes = C.c_uint32, [C.c_uint32, C.c_uint32]
+    for tokens in list(range(3, 130)) + [512, 1000]:
+        s = stride(ty, tokens)
+        tile = 16 if tokens <= (8 if ty == K.Q6_K else 16) else 32 if tokens <= 32 else 64
+        assert s >= (tokens + tile - 1) // tile * tile and s <= tokens + 64
+        assert tokens > 32 or s % 8 == 0, tokens
