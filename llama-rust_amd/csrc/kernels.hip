@@ -622,20 +622,25 @@ static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
 // estimate below: a launch, and the steps of the CU that gets most, sixteen wavefronts at a time.  16 rows to a workgroup where that leaves
 // no CU a second one, then 32, then 64: fewer rows to a wavefront are spread over more CUs, more are decoded behind each cutting of the
 // activations.  Eight wavefronts where a CU gets two workgroups or sixteen would have less than four steps each, four where both is so.
-// The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens: by this rule they are
-// 1.27 times as fast in the geometric mean as with shared columns alone (Q4_0 at 8 tokens, shared / whole, us: 4096x1024 9.2 / 4.9, 4096x4096
-// 10.5 / 8.1, 8192x8192 18.6 / 16.5, 14336x4096 16.7 / 13.5, 32000x4096 27.6 / 23.7, but 1024x14336 12.5 / 15.5), none slower by more than
-// 5 %.  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6): 32 rows there (16384x1024 at 12 tokens 11.4 / 8.9,
-// 12288x1024 at 16 11.2 / 9.0); and where a CU gets two of its workgroups
-// the products of a chain (launch_gemm_act), whose sums another launch reads in either case, lose more than those alone gain ([gate,up] of eight
-// sequences, 28672x4096, with the launch behind it 27.9 / 30.2, 32000x4096 with 4 tokens alone 25.0 / 21.8): the same choice for both, as their sums are the
-// same bits.
+// Without token tiles no more than two rounds of workgroups: each has as much of the weights as of the starts of its wavefronts to wait for
+// (shared / whole, us: Q4_K 20000x256 at 16 tokens 6.0 / 8.0, 32000x512 at 16 8.8 / 10.9, Q8_0 128256x1024 at 16 26.7 / 33.0, 64000x2048 at 8
+// 24.1 / 26.3, Q4_0 128256x256 at 8 9.3 / 11.2, 64000x2048 at 9 26.0 / 25.9; two rounds: Q4_K 14336x512 at 16 8.2 / 6.9).
+// The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens, and checked on 3000
+// more, 64x256 to 128256x1024 with 3 to 1024 tokens: of those that take whole rows by this rule one is slower than with shared columns by
+// more than 7 % (Q8_0 16384x2048 at 32 tokens 19.3 / 21.0), and in the geometric mean they are 1.5 times as fast up to 16 tokens (shared /
+// whole, us, Q4_0 at 8 tokens: 4096x1024 9.2 / 4.9, 4096x4096 10.5 / 8.1, 8192x8192 18.6 / 16.5, 14336x4096 16.7 / 13.5, 32000x4096 27.6 /
+// 23.7, but 1024x14336 12.5 / 15.5).  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6): 32 rows
+// there (16384x1024 at 12 tokens 11.4 / 8.9, 12288x1024 at 16 11.2 / 9.0).  64 rows of Q4_K at more than one workgroup to a CU are left to
+// shared columns, though alone they gain (32000x4096 with 4 tokens 25.0 / 21.8): [gate,up] of eight sequences, 28672x4096, takes 27.9 / 30.2
+// with the launch behind it, and a product makes the same choice as the same one of a chain (launch_gemm_act), as their sums are the same
+// bits.
 // More tokens are tiles of 16 (Q6_K: 8), each a workgroup's, that decode the weights anew: against two or three launches that pays while
 // there is not much to decode (shared / whole, us, Q4_0: 512x2048 at 32 tokens 11.1 / 6.5, at 40 17.1 / 6.6, 1024x4096 at 17 11.1 / 9.1, at 100
 // 22.0 / 11.3, 2048x4096 at 64 21.9 / 12.1, 4096x4096 at 32 15.4 / 12.0, Q4_K 1024x2048 at 64 18.2 / 8.0, 2048x2048 at 100 21.8 / 15.3; 1.7 in the
-// geometric mean over 46 matrices from 256x1024 to 16384x512 at 17 to 160 tokens), and every round of workgroups after the first costs
-// its start (Q4_K 16384x512 at 17 12.9 / 15.5, Q4_0 at 160 23.4 / 25.7).  There the wavefronts depend on the columns alone, so that products
-// of one launch and of several are the same bits.
+// geometric mean over 46 matrices from 256x1024 to 16384x512 at 17 to 160 tokens; 2.3 over 305 products of 161 to 1024 tokens, none slower),
+// less the starts of later rounds (Q4_K 16384x512 at 17 12.9 / 15.5, Q4_0 at 160 23.4 / 25.7).  There the wavefronts depend on the columns
+// alone, so that products of one launch and of several are the same bits where both take whole rows (the choice is the launch's: its rows
+// count together, and more than MM_FEW_JOBS products always share columns).
 struct WholePlan { uint32_t sets, waves; };
 static uint32_t whole_slots(uint32_t type, uint32_t max_tok) { return max_tok <= 8 || type == T_Q6_K ? 8 : 16; }
 static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats, const uint32_t *tokens, uint32_t n, double shares_us) {
@@ -663,6 +668,7 @@ static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats
     const size_t rounds = (tiles + cus - 1) / cus;
     double us = 4.6 + (double)rounds * steps / 16.0 * step_us[eight][p.sets / 2] * dtype;
     if (several) us += (double)(rounds - 1) * (type == T_Q4_K ? 2.0 : 1.0);
+    else if (rounds > 2) return WholePlan{0, 0};
     return us < 0.96 * shares_us ? p : WholePlan{0, 0};
 }
 

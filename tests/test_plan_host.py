@@ -87,3 +87,21 @@ def test_cut_activations_start_on_lines(lib, ty):
         tile = 16 if tokens <= (8 if ty == K.Q6_K else 16) else 32 if tokens <= 32 else 64
         assert s >= (tokens + tile - 1) // tile * tile and s <= tokens + 64
         assert tokens > 32 or s % 8 == 0, tokens
+
+
+# (dtype, rows, cols, tokens): many rounds of workgroups, measured slower with whole rows by 6 to 33 %
+MANY_ROUNDS = [(K.Q4_K, [20000], 256, 9), (K.Q4_K, [20000], 256, 16), (K.Q4_K, [32000], 512, 9), (K.Q4_K, [32000], 512, 16),
+               (K.Q4_K, [4096] * 8, 512, 16), (K.Q8_0, [128256], 1024, 16), (K.Q8_0, [64000], 512, 8), (K.Q8_0, [64000], 1024, 8),
+               (K.Q4_0, [128256], 256, 8), (K.Q4_0, [128256], 512, 8), (K.Q5_0, [128256], 256, 8)]
+
+
+@pytest.mark.parametrize("ty,rows,cols,tokens", MANY_ROUNDS, ids=lambda v: str(v))
+def test_many_rounds_of_workgroups_share_columns(whole_rows, ty, rows, cols, tokens):
+    assert whole_rows(ty, rows, cols, tokens) == (0, 0)
+
+
+@pytest.mark.parametrize("ty,rows,cols,tokens,want", [
+    (K.Q4_0, 14336, 4096, 8, 64), (K.Q4_0, 4096, 4096, 8, 16), (K.Q4_K, 16384, 1024, 12, 32), (K.Q4_K, 12288, 1024, 16, 32),
+    (K.Q8_0, 32000, 1024, 8, 64), (K.Q4_0, 512, 2048, 40, 16)], ids=lambda v: str(v))
+def test_few_rounds_take_whole_rows(whole_rows, ty, rows, cols, tokens, want):
+    assert whole_rows(ty, [rows], cols, tokens)[0] == want
