@@ -625,15 +625,23 @@ static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
 // Without token tiles no more than two rounds of workgroups: each has as much of the weights as of the starts of its wavefronts to wait for
 // (shared / whole, us: Q4_K 20000x256 at 16 tokens 6.0 / 8.0, 32000x512 at 16 8.8 / 10.9, Q8_0 128256x1024 at 16 26.7 / 33.0, 64000x2048 at 8
 // 24.1 / 26.3, Q4_0 128256x256 at 8 9.3 / 11.2, 64000x2048 at 9 26.0 / 25.9; two rounds: Q4_K 14336x512 at 16 8.2 / 6.9).
-// The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens, and checked on 3000
+// The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens, and checked on 5800
 // more, 64x256 to 128256x1024 with 3 to 1024 tokens: of those that take whole rows by this rule one is slower than with shared columns by
-// more than 7 % (Q8_0 16384x2048 at 32 tokens 19.3 / 21.0), and in the geometric mean they are 1.5 times as fast up to 16 tokens (shared /
+// more than 5 % (Q8_0 16384x2048 at 32 tokens 19.3 / 21.0), and in the geometric mean they are 1.5 times as fast up to 16 tokens (shared /
 // whole, us, Q4_0 at 8 tokens: 4096x1024 9.2 / 4.9, 4096x4096 10.5 / 8.1, 8192x8192 18.6 / 16.5, 14336x4096 16.7 / 13.5, 32000x4096 27.6 /
 // 23.7, but 1024x14336 12.5 / 15.5).  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6): 32 rows
 // there (16384x1024 at 12 tokens 11.4 / 8.9, 12288x1024 at 16 11.2 / 9.0).  64 rows of Q4_K at more than one workgroup to a CU are left to
-// shared columns, though alone they gain (32000x4096 with 4 tokens 25.0 / 21.8): [gate,up] of eight sequences, 28672x4096, takes 27.9 / 30.2
-// with the launch behind it, and a product makes the same choice as the same one of a chain (launch_gemm_act), as their sums are the same
-// bits.
+// shared columns, though alone they gain (32000x4096 with 4 tokens 25.0 / 21.8).
+// A product makes the same choice as the same one of a chain (launch_gemm_act), as their sums are the same bits.  In a chain no launch falls
+// away, as an epilogue's follows in either case (with cut activations no cutting launch either), and a product that gains little alone loses
+// there.  So a pair of one shape, which is a chain's [gate,up], takes whole rows only while its steps are short beside the shares they
+// save: over 1500 pairs those left out are 0.98 as fast that way in the geometric mean (Q4_0 2x14336x4096 at 9 tokens 27.5 / 30.0, Q4_K
+// 2x14336x512 at 9 12.6 / 16.4, Q8_0 2x8192x2048 at 33 25.2 / 32.2, Q4_K 2x4096x1024 at 17 12.8 / 15.0), the others 1.36.  Single products: 16 rows
+// of 8192 columns are left out (Q8_0 4096x8192 at 8 tokens 12.2 / 13.1 alone, 12.9 / 14.1 with a residual epilogue), and Q6_K of up to eight
+// tokens from 4096 columns on, whose lanes read cut activations twice (2048x4096 10.5 / 9.5 alone, 10.8 / 11.9 with the epilogue, 10.7 / 12.9
+// on cut activations).  Others keep whole rows for what they gain alone: of 5800 products with the epilogue 97 are slower by more than 5 %
+// (Q8_0 8192x4096 at 16 tokens 13.8 / 15.7, alone 13.2 / 12.8; Q4_K 1536x3072 at 14 9.2 / 10.9; Q6_K 1536x6144 at 14 13.6 / 16.2 on cut ones), all
+// of them 1.4 times as fast in the geometric mean.
 // More tokens are tiles of 16 (Q6_K: 8), each a workgroup's, that decode the weights anew: against two or three launches that pays while
 // there is not much to decode (shared / whole, us, Q4_0: 512x2048 at 32 tokens 11.1 / 6.5, at 40 17.1 / 6.6, 1024x4096 at 17 11.1 / 9.1, at 100
 // 22.0 / 11.3, 2048x4096 at 64 21.9 / 12.1, 4096x4096 at 32 15.4 / 12.0, Q4_K 1024x2048 at 64 18.2 / 8.0, 2048x2048 at 100 21.8 / 15.3; 1.7 in the
@@ -664,11 +672,14 @@ static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats
     else p.waves = twice && steps <= 32 ? 4 : twice || steps < 64 ? 8 : 16;
     if (type == T_Q4_K && !eight && p.waves > 8) p.waves = 8;  // LDS
     static constexpr double step_us[2][3] = {{0.76, 1.02, 1.5}, {0.46, 0.72, 1.22}};  // [eight][sets]
-    const double dtype = type == T_Q6_K ? 1.35 : type == T_Q5_1 ? 1.15 : type != T_Q4_K ? 1.0 : eight ? 1.1 : 1.2;
+    const double dtype = type == T_Q6_K ? (max_tok <= 8 ? 1.5 : 1.35) : type == T_Q5_1 ? 1.15 : type != T_Q4_K ? 1.0 : eight ? 1.1 : 1.2;
     const size_t rounds = (tiles + cus - 1) / cus;
-    double us = 4.6 + (double)rounds * steps / 16.0 * step_us[eight][p.sets / 2] * dtype;
-    if (several) us += (double)(rounds - 1) * (type == T_Q4_K ? 2.0 : 1.0);
-    else if (rounds > 2) return WholePlan{0, 0};
+    double work_us = (double)rounds * steps / 16.0 * step_us[eight][p.sets / 2] * dtype;
+    if (several) work_us += (double)(rounds - 1) * (type == T_Q4_K ? 2.0 : 1.0);
+    else if (rounds > 2 || (p.sets == 1 && steps >= 256)) return WholePlan{0, 0};
+    const bool pair = n == 2 && mats[0].rows == mats[1].rows;  // as [gate,up], with the SiLU launch behind it
+    if (pair && work_us > (max_tok <= 8 ? 8.0 : max_tok <= 16 ? 5.5 : max_tok > 32 ? 15.0 : type == T_Q4_K ? 6.5 : 12.0)) return WholePlan{0, 0};
+    const double us = 4.6 + work_us;
     return us < 0.96 * shares_us ? p : WholePlan{0, 0};
 }
 

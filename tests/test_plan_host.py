@@ -105,3 +105,26 @@ def test_many_rounds_of_workgroups_share_columns(whole_rows, ty, rows, cols, tok
     (K.Q8_0, 32000, 1024, 8, 64), (K.Q4_0, 512, 2048, 40, 16)], ids=lambda v: str(v))
 def test_few_rounds_take_whole_rows(whole_rows, ty, rows, cols, tokens, want):
     assert whole_rows(ty, [rows], cols, tokens)[0] == want
+
+
+# (dtype, rows, cols, tokens): [gate,up] pairs that lost 8 to 28 % with the launch behind them
+LONG_PAIRS = [(K.Q4_0, 14336, 4096, 9), (K.Q4_0, 14336, 8192, 16), (K.Q5_0, 14336, 4096, 16), (K.Q5_0, 14336, 8192, 3), (K.Q4_K, 14336, 512, 9),
+              (K.Q4_K, 11008, 1024, 16), (K.Q8_0, 8192, 2048, 33), (K.Q8_0, 8192, 2048, 32), (K.Q4_K, 4096, 1024, 17), (K.Q5_0, 2048, 2048, 160)]
+
+
+@pytest.mark.parametrize("ty,rows,cols,tokens", LONG_PAIRS, ids=lambda v: str(v))
+def test_long_pairs_share_columns(whole_rows, ty, rows, cols, tokens):
+    """In a chain the launch that would sum the shares runs in either case: a long pair gains nothing by whole rows."""
+    assert whole_rows(ty, [rows, rows], cols, tokens) == (0, 0)
+
+
+@pytest.mark.parametrize("ty,rows,cols,tokens", [(K.Q4_0, 2816, 1024, 8), (K.Q8_0, 4096, 1024, 16), (K.Q4_K, 2048, 512, 24), (K.Q5_0, 1024, 1024, 100)],
+                         ids=lambda v: str(v))
+def test_short_pairs_take_whole_rows(whole_rows, ty, rows, cols, tokens):
+    assert whole_rows(ty, [rows, rows], cols, tokens)[0] != 0
+
+
+@pytest.mark.parametrize("ty,rows,cols,tokens", [(K.Q8_0, 4096, 8192, 8), (K.Q4_K, 4096, 8192, 8), (K.Q6_K, 1024, 4096, 3), (K.Q6_K, 2048, 4096, 8),
+                                                 (K.Q6_K, 8192, 4096, 8)], ids=lambda v: str(v))
+def test_products_a_chain_loses_more_on_than_one_alone_gains(whole_rows, ty, rows, cols, tokens):
+    assert whole_rows(ty, [rows], cols, tokens) == (0, 0)
