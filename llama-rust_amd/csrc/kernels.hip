@@ -624,7 +624,9 @@ static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
 // activations.  Eight wavefronts where a CU gets two workgroups or sixteen would have less than four steps each, four where both is so.
 // Without token tiles no more than two rounds of workgroups: each has as much of the weights as of the starts of its wavefronts to wait for
 // (shared / whole, us: Q4_K 20000x256 at 16 tokens 6.0 / 8.0, 32000x512 at 16 8.8 / 10.9, Q8_0 128256x1024 at 16 26.7 / 33.0, 64000x2048 at 8
-// 24.1 / 26.3, Q4_0 128256x256 at 8 9.3 / 11.2, 64000x2048 at 9 26.0 / 25.9; two rounds: Q4_K 14336x512 at 16 8.2 / 6.9).
+// 24.1 / 26.3, Q4_0 128256x256 at 8 9.3 / 11.2, 64000x2048 at 9 26.0 / 25.9; two rounds: Q4_K 14336x512 at 16 8.2 / 6.9).  And nothing that is
+// long enough for a launch not to matter (Q4_0 12288x11264 at 6 tokens 25.0 / 28.4, 24576x5120 at 5 22.7 / 25.2, 24576x3072 at 72 73.0 / 84.4,
+// Q5_0 17408x3072 at 72 59.9 / 72.4; 8192x8192 at 8 tokens 18.6 / 16.5).
 // The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens, and checked on 5800
 // more, 64x256 to 128256x1024 with 3 to 1024 tokens: of those that take whole rows by this rule one is slower than with shared columns by
 // more than 5 % (Q8_0 16384x2048 at 32 tokens 19.3 / 21.0), and in the geometric mean they are 1.5 times as fast up to 16 tokens (shared /
@@ -679,6 +681,7 @@ static WholePlan whole_plan(uint32_t type, uint32_t max_tok, const MatView *mats
     else if (rounds > 2 || (p.sets == 1 && steps >= 256)) return WholePlan{0, 0};
     const bool pair = n == 2 && mats[0].rows == mats[1].rows;  // as [gate,up], with the SiLU launch behind it
     if (pair && work_us > (max_tok <= 8 ? 8.0 : max_tok <= 16 ? 5.5 : max_tok > 32 ? 15.0 : type == T_Q4_K ? 6.5 : 12.0)) return WholePlan{0, 0};
+    if (work_us > (several ? 38.0 : eight ? 24.0 : 30.0)) return WholePlan{0, 0};
     const double us = 4.6 + work_us;
     return us < 0.96 * shares_us ? p : WholePlan{0, 0};
 }

@@ -128,3 +128,10 @@ def test_short_pairs_take_whole_rows(whole_rows, ty, rows, cols, tokens):
                                                  (K.Q6_K, 8192, 4096, 8)], ids=lambda v: str(v))
 def test_products_a_chain_loses_more_on_than_one_alone_gains(whole_rows, ty, rows, cols, tokens):
     assert whole_rows(ty, [rows], cols, tokens) == (0, 0)
+
+
+@pytest.mark.parametrize("ty,rows,cols,tokens", [(K.Q4_0, 12288, 11264, 6), (K.Q5_0, 24576, 5120, 4), (K.Q5_0, 24576, 3072, 72), (K.Q8_0, 17408, 3072, 72)],
+                         ids=lambda v: str(v))
+def test_long_products_share_columns(whole_rows, ty, rows, cols, tokens):
+    """Measured slower with whole rows by 12 to 27 %: what a launch less gains does not pay for the activations' cutting there."""
+    assert whole_rows(ty, [rows], cols, tokens) == (0, 0)
