@@ -12,8 +12,9 @@ import oracle as O
 pytestmark = pytest.mark.gpu
 
 QUANTIZED = [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K, K.Q6_K]
-# rows: edges of workgroups of 16, 32 (from 4097 rows) and 64 rows (from 8193) and of the layout's 256; columns: fewer steps than
-# wavefronts, shares of different length, an odd count of steps, sixteen, eight and (16385 rows) four wavefronts
+# rows: edges of workgroups of 16, 32 and 64 rows and of the layout's 256; columns: fewer steps than wavefronts, shares of different length, an
+# odd count of steps.  Which of them take whole rows, and how many wavefronts share them, is the plan's: test_gpu_whole_rows_variants.py has
+# every variant, and asks the plan.
 SHAPES = [(1, 32), (15, 96), (17, 480), (255, 1056), (300, 2080), (4096, 96), (4097, 288), (4130, 2304), (8193, 160), (8255, 2048), (16385, 96)]
 
 

@@ -6,47 +6,30 @@ import pytest
 
 import cases as K
 import oracle as O
+import whole_rows as W
 
 QUANTIZED = [K.Q4_0, K.Q5_0, K.Q5_1, K.Q8_0, K.Q4_K, K.Q6_K]
-
-
-class MatView(C.Structure):  # csrc/matview.h
-    _fields_ = [("p", C.c_void_p * 4), ("s", C.c_uint32 * 4), ("type", C.c_uint32), ("rows", C.c_uint32), ("cols", C.c_uint32), ("nb", C.c_uint32)]
-
-
-def views(ty, rows, cols):
-    mats = (MatView * len(rows))()
-    for m, r in zip(mats, rows):
-        m.type, m.rows, m.cols = ty, r, cols
-    return mats
 
 
 @pytest.fixture(scope="module")
 def act_workspace(lib):
     f = getattr(lib, "_ZN2nh24gemm_act_workspace_bytesEPKNS_7MatViewEjjbb")
-    f.restype, f.argtypes = C.c_size_t, [C.POINTER(MatView), C.c_uint32, C.c_uint32, C.c_bool, C.c_bool]
+    f.restype, f.argtypes = C.c_size_t, [C.POINTER(W.MatView), C.c_uint32, C.c_uint32, C.c_bool, C.c_bool]
 
     def workspace(ty, rows, cols, tokens, epilogue):
-        return f(views(ty, rows, cols), len(rows), tokens, epilogue, False)
+        return f(W.views(ty, rows, cols), len(rows), tokens, epilogue, False)
     return workspace
 
 
 @pytest.fixture(scope="module")
 def whole_rows(lib):
-    """(rows, wavefronts) of a workgroup that owns whole rows, (0, 0) where columns are shared."""
-    f = getattr(lib, "_ZN2nh18planned_whole_rowsEPKNS_7MatViewEPKjPKPKfPKPfj")
+    return lambda *product: W.planned(lib, *product)
 
-    class WholeRows(C.Structure):
-        _fields_ = [("rows", C.c_uint32), ("waves", C.c_uint32)]
 
-    f.restype = WholeRows
-
-    def plan(ty, rows, cols, tokens, xs=None, ys=None):
-        n = len(rows)
-        toks = (C.c_uint32 * n)(*(tokens if isinstance(tokens, (list, tuple)) else [tokens] * n))
-        p = f(views(ty, rows, cols), toks, (C.c_void_p * n)(*xs) if xs else None, (C.c_void_p * n)(*ys) if ys else None, C.c_uint32(n))
-        return p.rows, p.waves
-    return plan
+@pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
+def test_variants_are_what_the_gpu_tests_take_them_for(whole_rows, ty):
+    for rows, cols, tokens, wg_rows, waves in W.VARIANTS[ty] + W.CHAINED[ty]:
+        assert whole_rows(ty, [rows], cols, tokens) == (wg_rows, waves), (rows, cols, tokens)
 
 
 @pytest.mark.parametrize("ty", QUANTIZED, ids=lambda t: O.TYPE_NAMES[t])
