@@ -626,12 +626,12 @@ static uint32_t mm_tile16_max(uint32_t type) { return type == T_Q6_K ? 8 : 16; }
 // (shared / whole, us: Q4_K 20000x256 at 16 tokens 6.0 / 8.0, 32000x512 at 16 8.8 / 10.9, Q8_0 128256x1024 at 16 26.7 / 33.0, 64000x2048 at 8
 // 24.1 / 26.3, Q4_0 128256x256 at 8 9.3 / 11.2, 64000x2048 at 9 26.0 / 25.9; two rounds: Q4_K 14336x512 at 16 8.2 / 6.9).  And nothing that is
 // long enough for a launch not to matter (Q4_0 12288x11264 at 6 tokens 25.0 / 28.4, 24576x5120 at 5 22.7 / 25.2, 24576x3072 at 72 73.0 / 84.4,
-// Q5_0 17408x3072 at 72 59.9 / 72.4; 8192x8192 at 8 tokens 18.6 / 16.5).
+// Q5_0 17408x3072 at 72 59.9 / 72.4; 8192x8192 at 8 tokens 17.0 / 14.2).
 // The prices are fitted to 900 products of six dtypes, 64x1024 to 32000x4096 and 8192x14336, with 4, 8 and 16 tokens, and checked on 5800
 // more, 64x256 to 128256x1024 with 3 to 1024 tokens: of those that take whole rows by this rule one is slower than with shared columns by
 // more than 5 % (Q8_0 16384x2048 at 32 tokens 19.3 / 21.0), and in the geometric mean they are 1.5 times as fast up to 16 tokens (shared /
-// whole, us, Q4_0 at 8 tokens: 4096x1024 9.2 / 4.9, 4096x4096 10.5 / 8.1, 8192x8192 18.6 / 16.5, 14336x4096 16.7 / 13.5, 32000x4096 27.6 /
-// 23.7, but 1024x14336 12.5 / 15.5).  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6): 32 rows
+// whole, us, Q4_0 at 8 tokens: 4096x1024 8.4 / 4.5, 4096x4096 10.2 / 7.6, 8192x8192 17.0 / 14.2, 14336x4096 15.6 / 13.0, 32000x4096 24.0 /
+// 21.5, but 1024x14336 12.5 / 15.5).  Q4_K's 64 rows at more than eight tokens do not fit the registers (14336x4096 19.4 / 28.6): 32 rows
 // there (16384x1024 at 12 tokens 11.4 / 8.9, 12288x1024 at 16 11.2 / 9.0).  64 rows of Q4_K at more than one workgroup to a CU are left to
 // shared columns, though alone they gain (32000x4096 with 4 tokens 25.0 / 21.8).
 // A product makes the same choice as the same one of a chain (launch_gemm_act), as their sums are the same bits.  In a chain no launch falls
